@@ -1,0 +1,487 @@
+"""Measured workloads of the batched rigid step, through the gs.Scene / RigidEntity surface, the fused batch and the
+serving loop.
+
+A case is one scene family at one env count with the number of steps of one pass:
+
+* "arm":       the 9-DoF Panda over a plane under PD position targets (mesh collision, self-collision off).
+* "quadruped": the 18-DoF go2 over a plane, standing pose plus noise as PD targets, observations read every step.
+               "randomized" gives every env its own masses, friction, gains and armature (domain randomisation).
+* "pile":      free boxes of random sizes resting in a heap, no control.
+* "mixed":     arm, quadruped and 20-box pile stepped by one captured fused launch per step.
+* "serve":     rollout requests of the three scene types served to completion.
+* "pose":      link poses of given joint positions, without a step.
+
+Rollouts ("loop": "rollout") start every pass from the same state, as sampling-based planning and evaluation do; control
+loops ("loop": "control") go on from where the last pass ended, as reinforcement learning and teleoperation do.
+"""
+import base64
+import json
+import math
+import os
+
+import numpy as np
+import torch
+
+import genesis_amd as gs
+from genesis_amd.batch import FusedBatch, Group
+from genesis_amd.serving import Pool, Request, Server
+
+DEV = "cuda"
+ARM_HOME = (0.0, 0.25, 0.0, -2.35, 0.0, 2.6, 0.8, 0.03, 0.03)
+ARM_LO = (-2.8973, -1.7628, -2.8973, -3.0718, -2.8973, -0.0175, -2.8973, 0.0, 0.0)
+ARM_HI = (2.8973, 1.7628, 2.8973, -0.0698, 2.8973, 3.7525, 2.8973, 0.04, 0.04)
+STANDING = (0.0, 0.0, 0.0, 0.0, 0.8, 0.8, 1.0, 1.0, -1.5, -1.5, -1.5, -1.5)
+MIX = (0.3352, 0.3326, 0.3322)  # arm, quadruped, pile shares of a mixed batch
+# degrees of freedom, generalized positions, controlled dofs and floats of persistent state beside them, per scene type
+SIZES = {"arm": (9, 9, 9), "quadruped": (18, 19, 12)}
+
+
+def listed():
+    return [
+        # one robot under a controller at its own rate: the smallest call, all launches and latency
+        {"name": "arm_1", "family": "arm", "envs": 1, "steps": 1, "loop": "control", "dt": 0.01},
+        # the CPU-runnable configuration: 64 arms following random targets
+        {"name": "arm_64", "family": "arm", "envs": 64, "steps": 10, "loop": "rollout", "dt": 0.01},
+        # a large batch of arms working close to the floor, an odd count
+        {"name": "arm_5001", "family": "arm", "envs": 5001, "steps": 4, "loop": "rollout", "dt": 0.01},
+        # locomotion training at its usual size with randomised dynamics, not a multiple of the wavefront
+        {"name": "quadruped_4000r", "family": "quadruped", "envs": 4000, "steps": 2, "loop": "control", "dt": 0.01,
+         "randomized": True},
+        # locomotion at scale
+        {"name": "quadruped_32768", "family": "quadruped", "envs": 32768, "steps": 1, "loop": "control", "dt": 0.005},
+        # a few cluttered tables
+        {"name": "pile7_100", "family": "pile", "boxes": 7, "envs": 100, "steps": 4, "loop": "rollout", "dt": 0.01},
+        # clutter at the size of a planner's sample set
+        {"name": "pile20_1500", "family": "pile", "boxes": 20, "envs": 1500, "steps": 3, "loop": "rollout", "dt": 0.01},
+        # the contact-heavy configuration at a few envs and at its full size
+        {"name": "pile64_96", "family": "pile", "boxes": 64, "envs": 96, "steps": 2, "loop": "rollout", "dt": 0.01},
+        {"name": "pile64_4096", "family": "pile", "boxes": 64, "envs": 4096, "steps": 2, "loop": "rollout", "dt": 0.01},
+        # the heterogeneous batch in one captured launch sequence per step
+        {"name": "mixed_16384", "family": "mixed", "envs": 16384, "steps": 3, "loop": "rollout", "dt": 0.01},
+        # a burst of rollout requests of all scene types
+        {"name": "serve_12", "family": "serve", "envs": 96, "steps": 14, "requests": 12, "loop": "rollout", "dt": 0.01},
+        # workspace sampling: joint positions in, link poses out
+        {"name": "pose_20000", "family": "pose", "envs": 20000, "steps": 1, "loop": "rollout", "dt": 0.01},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    family = rng.choice(("arm", "arm", "quadruped", "quadruped", "pile", "pile", "pile", "mixed", "serve", "pose"))
+    if family == "arm":
+        return {"family": "arm", "envs": _log_int(rng, 1, 6000), "steps": rng.randint(2, 10), "loop": "rollout", "dt": 0.01}
+    if family == "quadruped":
+        return {"family": "quadruped", "envs": _log_int(rng, 16, 32768), "steps": rng.randint(1, 2), "loop": "control",
+                "dt": rng.choice((0.005, 0.01)), "randomized": rng.random() < 0.4}
+    if family == "pile":
+        boxes = _log_int(rng, 4, 64)
+        return {"family": "pile", "boxes": boxes, "envs": _log_int(rng, 16, min(4096, 4096 * 64 // (boxes * 2))),
+                "steps": rng.randint(1, 2), "loop": "rollout", "dt": 0.01}
+    if family == "mixed":
+        return {"family": "mixed", "envs": _log_int(rng, 300, 16384), "steps": rng.randint(1, 3), "loop": "rollout", "dt": 0.01}
+    if family == "serve":
+        return {"family": "serve", "envs": _log_int(rng, 8, 128), "steps": rng.randint(6, 14),
+                "requests": rng.randint(4, 14), "loop": "rollout", "dt": 0.01}
+    return {"family": "pose", "envs": _log_int(rng, 64, 32768), "steps": 1, "loop": "rollout", "dt": 0.01}
+
+
+# ---- scenes and their states ------------------------------------------------------------------------------------
+def _gen(seed):
+    return torch.Generator(device=DEV).manual_seed(int(seed))
+
+
+def _uniform(g, shape, lo, hi):
+    lo, hi = (torch.as_tensor(x, dtype=torch.float32, device=DEV) for x in (lo, hi))
+    return lo + (hi - lo) * torch.rand(shape, generator=g, device=DEV)
+
+
+def _quat_mul(a, b):
+    aw, ax, ay, az = a.unbind(-1)
+    bw, bx, by, bz = b.unbind(-1)
+    return torch.stack([aw * bw - ax * bx - ay * by - az * bz, aw * bx + ax * bw + ay * bz - az * by,
+                        aw * by - ax * bz + ay * bw + az * bx, aw * bz + ax * by - ay * bx + az * bw], -1)
+
+
+def _quat_mat(q):
+    w, x, y, z = q.unbind(-1)
+    return torch.stack([torch.stack([1 - 2 * (y * y + z * z), 2 * (x * y - w * z), 2 * (x * z + w * y)], -1),
+                        torch.stack([2 * (x * y + w * z), 1 - 2 * (x * x + z * z), 2 * (y * z - w * x)], -1),
+                        torch.stack([2 * (x * z - w * y), 2 * (y * z + w * x), 1 - 2 * (x * x + y * y)], -1)], -2)
+
+
+def _box_sizes():
+    return np.random.default_rng(1).uniform(0.05, 0.2, (64, 3))
+
+
+def _heaps(boxes, seed):
+    """Settled heaps of `boxes` boxes: poses (n_heaps, boxes, 7) and the boxes' sizes. 20 and 64 boxes have several
+    heaps; another count is what is left of one of them when its uppermost boxes are taken away."""
+    whole = 20 if boxes <= 20 else 64
+    q = np.stack([np.frombuffer(base64.b85decode(h), "<i2").reshape(whole, 7) for h in HEAPS[whole]]).astype(np.float64)
+    q /= np.array([25000.0] * 3 + [32000.0] * 4)
+    if boxes == whole:
+        return q, _box_sizes()[:whole]
+    q = q[seed % len(q)]
+    low = np.sort(np.argsort(q[:, 2], kind="stable")[:boxes])
+    return q[None, low], _box_sizes()[low]
+
+
+# Settled heaps of the boxes _box_sizes() gives (the first 20 of them, and all 64), dropped from random poses and stepped
+# by the CPU oracle until they rested: per box x, y, z in 1/25000 m and a quaternion (w, x, y, z) in 1/32000, as 16-bit
+# integers. Fractions of a millimetre of overlap at each contact, 76 to 80 contacts a 20-box heap and 248 to 267 a 64-box one.
+HEAPS = {
+    20: [
+        'OYBzNE(VnWU|4JZU|2Ey_8_+eA6Fk&74a4EAQWjLbp`+c;f(<^007Ye!ONlo{Yj<I{YhIe2M)jA*#u0iWE@Paoa2h)!Uk#s8BQ5aWhrGTV&)>w>;'
+        'n`hxUdu_NKX>b0~x~!mtPsSU<`^K%o()sy$5u%j7@7QmDQ?1LgkzT{5||V13v>l033tJNCOU6@~BG>weTGw!v^dIKi5Ckk+G4n$nrneO$HSE6#Kx'
+        'Zz^82b8|32x5BCwM@dy#9LeU@d#s-1gflz_lf3Hv4!6PgNkyUQ0+vzD5^U7rAZwIKP00000tg2SOh$PhmJgGOSE$=k%R0I3-'
+        ')dRarYtluuYtpgxeK+F;005tly*2;<',
+        'Zrm~vE(UM4b}w(WiqH|(X7-2$001{)Q%wK>Y!pz>ZUq8Z{--'
+        'kt&G$I<>?3#vjsJ^#(h}4HRp=ov#tJ`$vlYMx@%k#|usy&92gkNUAjf*VyC^*M>;uOHzNf|nLRdpF;Xr%@qRCLYqRFsDgaIt>Wd{6a00000C%M1l'
+        'AHQ`3gf*wRe9EV}Q!8)jHU>5K4XDcq4X8dQa~&TDk@J42Zw!8@ulgVfxdNw9*4w90DkQzmXXD`l)g>md9NHbQoE26Rl?VU;*}d_V007$gL_6{a1G'
+        'NAE0091*TGu=YZwN9^GEYAzKPR{8p&`@*PBBL@Vo6&`Xd?qY2Lsm#DfjYM4yaK9@F-&mD-sFeO8Z=h',
+        'w(FA9eFO8000000b1vunRvd^0007$IPk8_Umky=Abp`+c5I9GW001%}9rB<8RLx*WuQGN>*Y`x^*#wKPXxodgm?Y=VfyrtERVAz1;;$Z188G$vS_'
+        'IwjBM<AS6;}b|11fw3D9n~eD9mcOYwG0)y$2>GCM7gbG*IQ+cph~GyR{V1yS3~u@fh&VNCT%+S*(g2cH>JQvKfd8lN==m&ZnPK6xdrqxdMJv^cjM'
+        'y^ck4j0rKMlG*lktG*sdm1S$C8Rs{D*_edVj9?r=7b}K9f{7wY1tS401ofNt2)&|7j3_G$BDQHX$VKOoZzYKR*zYK|}+7vk^1OscRS*VW-'
+        'y$hln#RS?2TT)w686X)T',
+        'v=b)&eFFdh?|kk1003tVq3O2-'
+        'Rzy}r@yGGUEHeKBbp`+c`+T+i003R#+}5H3sJJdPsJPP0S^sYI*#vg`Mp$<Hx~IU|9x7@BH0?C)qN$>(^7B;o>;n$Gc*hRBh&ZCkF9Uo8JhXe##7'
+        'le9211tcWd@3d00000h#dy`^xK>R%my_1;HMy18ZhqU0S63Hy$&Z=-'
+        'yj(jm>wnx`)B|F001StI{W$=xdI8>N>B;gwy#1m;?*Gs<@VzC7N`}d)!K{b#s+;peZhmleZl&@BjzdwR1Ke~tn#0zS|7CMgabar;J!Y@AVDAHZ~`'
+        '(2M6KrFyi(@iclnYB)dQneff1utf9`29niARwOu4j13pMr1',
+        'Rr<^Yd;{S?{r~^}*lP6v3h}iBLAb_8X3U&3%-'
+        '^{NZ3SRKWI=&Db34cuG|{30lv6$9lvBeT9>os<*#v^HTiJe3TiMJp)$?it_#Fu1CsWz1_2&^AS_DqWvNxhcUc34CaO@cjo4EW=^xUk-'
+        ';yRB%y$4e5Qth0noT&vVFBf$LmZ%dAmZ<IW5FdsjNCN=&0QN4ZE~uIcalq^b!%V|W(ks#{r~j(o3<Mr4pi#oer$6%RISO?Qw7wJAld7^Y4%0Tt#s'
+        '-t`*;Z~4*;WAR)8JYOGS1?^yjOGEiXYqpgagvJXEZKHXEbyZsUlAZ{;vQ4000YMLiWPN)dRe!^YKJi^YO3-jU?I#@%9f1>{k@1',
+        '&*!}~E(SK-FRwM+(NKLjB>1-'
+        'k&9u$5bS`u*uhLV~bp}GB00000P_5(T_Ya@~Q8X||Q#7`?DHcP^*#wd;M6_<wM6?3oe9U4600023cU=Gg>=Hd2>;rpK^x}oA^x_l9*5P~vbhUmjb'
+        'hU!eDf80zu?)t|qdET9aax?}59*o&a?*Lyz)QhPND6}wHU@I)xK(oMNUD|LH~=3AN;mdIN;e9-'
+        'h6XD4wE}!lP}@{cx+L4=;o|lNJoG<E9L=9sX!&yqRs`r(7OKh=IqReGwHjUuY`SP$pd|Vr(B5$(gabEFASE|Y;M!>a4(X%@NzX*rzQHJ{gU3h=)d'
+        'MKYCb`%&Cb=yH7A)EbHb*u`q|2ns',
+    ],
+    64: [
+        '*X6PMXb+wM6-KbWOHg|Y3L%aMXjL9qTnA(61R~23_!whNk-YXi4JGRRuH%slWANKuts=R$^crsFr3C8#s5uvr003O=76uUtj7(QdIV^-'
+        'M82{q9S_Iv!BU1z({NXs>UIJVYa6=DSjLRnM<0HQDy$5cwkxqUng4h2(uJ3jPNvRAGMXBNLQx&noL<29;;V$Y*1GTR$sRj@ZTkmzyO5hceR`*cZ!'
+        'UoX)s1y&Xou}agzUAKn_w#<J^b2071=<Mm#RhBHrcb5Wey}y;Y$PlO8dB!1L*Kn1+r%U5ZwSP?JVo+04$02TrXkh?1jYo$O1(<Gmkb8<(*yZTozw'
+        ')gg48kSfHl1clopGsZ0U=tTkyO0v<+SPin&(?*JdC;N8gPI%)>N1NWZv16~@Uq0tBhHRWVmdRWX)4VEgk00RVV>d-'
+        'VSQe=WeShXszsayqfSPePd=*dY1~0?zIznBV(lq!P*%P!anh1xf!{D&Nr-0^0cl%|ZtN|NmK*Ec$5lmIhF(+|8ZX!@XAZ^9?HnMpjT({p`f-'
+        'zu$n_RRsV5*kjAI002B4O)Odjsnb_1c1(%0irg{8H3N`Ehc<A!hc*KeYs`cSt=kB**QMbPM!x6%$p{kHsj(8*S5CS?(b3)mGg$xt005F#2rrcs{0'
+        'ow&v!@sW0|Ma!Jk?tZ^C$q<v9VK5vjMLZE(Oex?*Hrm>Bi#`+x0sU<+b@N$~}caXX;k#Aq?N-'
+        'X$*$5yP>TGcLGWl?Zsxj%*BpEc+kcHJOhO^=(vS67)RvN_7TtrOEKjaWHIYx`6vb~#ue03Tpy8A_25<MKvB*H99ZP10SEv14EXgJp$B^8LZ92j)h'
+        'vwdYuNn*L{z-1uNqP1_AEy%9R|rx=qC=b>nCRe=F@@$`TyaTUA+GP5e~%U;|xCW+g)3*_z&Og&H_{e6EXG9dP#1!^BQ?O&I7~2!#+Je!#;Wgkp-'
+        '3rJL;@ewiT^a?Hm99J_hmsA$6!L{QryEj0+zMXm8f{v;XJEo-'
+        'I)o;{!<psi#u|P*@u2kP{IFH_TtS$unQLWh!XdjsgGx)09*|006ZBrSU=%`Jb5&T-'
+        'd%t&(H|l_XFX*00000?3Fd_sl|>0aVd}15>D>1viXA}mkw3_@#iGl1&fIO_%YoExC%_DMD;wV',
+        'is-'
+        'a2WC<?e+8!dU&Qd++9tMX60RRzcxI+a1i5St}ehAGBi>Nd6i>SW^TQT4UH~DdO=p#=SAopY=SQNSU3s{v01y~sgv`J1AxaUb239AED3OIBG>;rHE'
+        'uBUMWQdkc}8Blx#Gs_;iGt1&e;tDnJc?nxe$}d|=Hqavjo8z1VKB~V}Y!#I1giZ9_HU_%Nhek#<herQ3|128_ZT2Imp9vwTgbl<XxdOCT1NF35{R'
+        ')EVJ?@nU<S3rZArx_F`yhcNz6c`D1f_%DQo=6@+eh&SmBIr6`~M-6K-'
+        'eKBgad6+o!xCwV<Ob{Nk8%kV_3V*tw{3$A01~vvIqbG(|lX`000{h12+x|d?IYv=kqj=BNqGla0GEXp1y{}mA*Uqd<A|4`~U1|UqS%@(d79?00g@'
+        'iCsj@8B~_C$mh!U-xwlZ_5AGPCTOTp-#}JsTL>-{4sp4_=T*I6K&b*YyGDDQcj9g>?eF)b_g3Q-Pels#E^f?a*=j`X~O;$}-'
+        '=17ri;{x+Y4Y%Ym6V9OE<usuKvLNuSwje7~<>kOUObyY=i>Dbm4k&jae@KJ{000{JK!X4Psrw%lH3ebTFaQMr-gRL+UG@hFXFjgmpUfy&(mrMw$q'
+        'OP|<`&Ny46++9C?DMe>Sh1{3;^>+$t2rWPy_$~y>zlH000c&y!nX^$Vo$5iQll`lRA8B@CGnf)UGw%3GqxiXFSCPf_4A^002MO*7)owzXxKW^#A<'
+        '-uu;(sO99jh53QA_G2*uQydX$7>jN18833K9ou{%SZ<M(NfzN@@<w@m9`80Vda~Kc+;o4kx4FJ3w%4W_6URa{17yju1YAqT@{{p@400000&3nona'
+        'V=p31B2iH1pt!)iRiZ&E(q+h?6SVpzSJV#nq!6o006s>3dsNf4p*>1m;?X-j2jb%001Nc1`>7-'
+        '&^H~&#8orYbff!JAp`&b6^Vo<000;ukqW8|h8H5J@=-b&b0E|m1rgB?+Q%uD5a7GVh6Az$->*<5-><ORZz6T`<O7+(mp)-'
+        'Wp+4RB`tijG#v;_O{jG*0AqGzXi~>CXr{o8QEdWaH+fV8VE&fC9Y~db=QvM4)bQ5S0*y@9h_0oL%0Rf8(l)GO<0XPZBYuak{Sp>MPNm91oMIgfxr'
+        'xH~NhQN70gFSx2',
+        '1;k+BE(R^BkPy>WkPv^yqaCFRAUrh1Kr6pdv&Id~bq3e+00000PJGMx82<AIFBLBp&{fb?#JbG*rvv~1L}zbC003gPAnj@cB~aV1MkTu1))UzMSp'
+        ';GGl?1$}Mp$*mb1-@YVa&`&a?C-vhr=BQWCnOR1pxj3g>O!y-y56*;-})L=mzKpcKn&tMFT!k-'
+        '>r)veBV+Om>G5t@L@ABYsT0U{=5P_AP9xiH^IB?WS^j-#{uI4>GuIx<M;WeJqoGvD+xsgcuc6B+V{`Z&^A2^-'
+        '%?z*)d?8K>&Ywr6c7$bbJcH18aib0)JWC?4oMD4Kh8hS)9wBvj|MC-'
+        'VzO~a?9z1A;||FTv&U}@^|XOeq#biWd;$YD12*?X_eJ*>FVlYn007(DSBL-rZt_qwAq~_=I=wKp!0T-'
+        '+ul0Qi)49Dh)44;+OzV6Sz6!c*H}rKJk;)<_M=Y8GszqfsvqhuHT+?vidk9=uLIPY^%>5lAdG9*}4Y08#4X{tzqA159n+G-'
+        'Wa``GX7;xF~r`!(*=$;WM;1`p?y$!`Xe+RC^WxuY&n?U64J1v3*Cjh#eUA650FS$P^I0XOzT@!+Y003kTp2au^`l<S<Q4~=W1-'
+        'iXMhYjp;`YC4;T^C^1J0I@^F{;1nIjTYxDFa<9RtPTw19`3X)g2om`xDIur7WsR;;vCBzYqW@S_8|cC0N(_90t^}^aP;_d%s*#^t_A>$MebUzy}N'
+        'fW?ay#5CEH-'
+        'V(%aYP@Mn(006j5qvFjW4h6iEj{1H*X7)rNLFBsx6CUHN6CNE?t>vNLZxA)eP3^x&KdgP_h5P*nk+W$mbWBw&+Og|1{{jF2jGJXj001uE&lX?<Bm'
+        'g{}o=h$P?f+Limju730s#O2hFGiRnKyz12mt?l;r{*q(D%s*$O%fgv!`_ZKg<9JmNL!<)Bykh008}bVwfV*&I17<|55+m|52+jn+Qq;zo@^c9S$8'
+        '1#NI0_4i1?x-dY&C?Fz}!()CmYsQg+3R9LO2+4%|_{09U8h&lOg`u~%(CQ}Xt66G#b>KZdtf!fsYIt5huBUn`V-'
+        'KSRldBV*H5qkX>S_1wHbO%)o@&h8=1pxd1zjxOOWCDc>k(8;>681pW{ma^{S_E3prZCG%HMX8-AQ;{TG6@%`G70Hd',
+        'uN2$=d;<gk_j~{Y|Nj9Agz<<4`~L}M%eMvq5jEEPYy}gk^Hvn__zx=11>B(mrM+xAO+srrI_VGY*92r#l;ufOdK$y*J1Fc4-'
+        'y>E=jZQ$vdG`kSvkwNcn(7s!N)>z15&?V!H>j@l$ycuRy-`Eqy$7SGqo>{d-'
+        'TgfN=+lV_000u>WrhF%yc_lATM?cqfk+?_hFcUG0v*x|aZ)xXIxO|J4Dk6J01w#c{aPagY*H0M%D>|RK)n#gz(Nql3Da)uRs?JbYzZEy9;idEDDN'
+        'r;-ucs~A_mi^Zy@#Y4GH(<7U#mN2vx`Fa|bdAkh=lMU_=badK6?1m<|u$;<$fc?()esVHMg4j;V51ZxWI1G6yCK`W5j)WI`0i*~Q2C-'
+        '6OOILF!nlL+Y_ry4WSQ0t5}XS2OcRS2Hs6`}*_+;!Fbo3jlDPq$lO@xDIPNY*&y%JM`WA2JD#v3-'
+        '8HR;1Ic1O)yg8L<ju;n;RB}{{OohJ>wn*sSCZZ@?IqJz~a07z7KXRxE|&d!)~kmq53Ta;6W(955@L6aP<(qw*!_jTh1~`<+jT)GAwxlUC?w&qc3z'
+        'yJpmUiI0XOzE%6?F002fJLkN8h?EhbUhYSG#s}Ow2u?s?9+Ot>lsposzoZK@9`yNK+Yl<-'
+        'oF!`ekx(P=`<u*q}8_BfjKQ#3MGtga1MbMwMVck{CFa-brv|I92007$O_!)u){<vz(>$sFOAqe8!?Gk!BMrDNf;MJ8CIPS9rcEXB1hCiXerRmhhJ'
+        'Ok6G-T5t8-'
+        'TAR1H_5pKfwPy>r?Y4*`7v;;ItbZ=00000d+~wLX2|{rC_FyD*uy@*oeu`@bP)<YmN%$B`9!?o1L$W1m2Ut5005}RCIPbIeFz#CllY`1OpDLyeC<'
+        'UJ!YC{ZeFKAvm=+7!DGH#+qrAhsH9Cl{yC}{F004a#I)wlLtl0w&Aq0!W00000^ldN|C@&QXGqg4TVpxjOG3=w)0|%B%(k+%tF49~f$Jks6s{apJ'
+        'w^yD2kO{#R5ehg_8`Md&;3E4lkW&!_jRqxHjRxDN;oM#%jsgGxW`hg%008pE;t+-'
+        'e{eu7i006BI4kDxr@&o&K4FLZC@7$@>Tll2}1OPP(YlA%i`2>ptzX`%d2FpOX2+J?`PrQ5%3jj}q3=%B>',
+        'we_wG;}j4#>ILBoZf^nkRPnV06SL$@ZPbh_eBNjL4GPvFrAL}8N>-*5r^*-'
+        'yHCJOSYfOL+Hn_+P*#x*hzQVXaLOla3YV~OYx*<&7yirrGmEOP}S_G2IZZs)J*SP2iBJSD{@K3l*MdLg&rYB}8QVGQA>sC`#aO(FRLladBPNzk#V'
+        'di)1i5CziMgwf~Tl0IUji^-)p1bV|MKjx31U}9n{RH0en+PgbEJWAjXfsLA#R|v_;nF^0Fw^ZT?yE<-'
+        'Rs^}Pxv%^r{3N~J_UJ4I(AX^}K2ON7Vi_6+egnX_^)ft2<}zaoULsEjW2688000YB5Cwg_0|Q15`|+%(ELXVl>K`);F!aSAE^2GXQ1~YTB?teT(E'
+        'rH)0kyOkm-a9T+iV6U=nBs-ZUBV>0}@N;daV!TdsZsjg2=E2FXW89Jzi}mbpKY@zXkvR;MGuy^#5z@^#08aq|*M9*x0P|D9qR-eF#tM5vs8i5vr^'
+        'Jax^;x-W|`Z-W@Sh-{Qy0;tpv|u16-|0>zgV)77B^NKgaY#INt#UgCuZx&u{Maad*lPX7?{!RL7b#8B-'
+        'c!cZ67OC+}05eJyJXh=@YvNDVLjSsyC^-WOL8L~#!SjolRz7N(5-'
+        '3wW$d8quycNX3Q|C0a!000xg<>?R2H3ZPhx67!wzPRchXTbIX{!MSz{7s=L77SnIE(H&W761VN%-'
+        'jtZ(cx7Pve#rNsZL<A90eZ&xdvFxb4aH$YDnNxZvG$zJB$DT007(2bpc=|=L1_9Q5Y4g`KnUxKi<0pzfor1Kdxfl5>zMOj0py|UoZx?q0jCU^$Hs'
+        'k`{qi!$E+L1;uOUe{sOW@_x}I@l9y&f&>m+4bQ=Hw000e!stL==w-'
+        'SauY&(Bi67@?o80Uinv{>u^1OV=*Zp$eCmjv8*{Qvs@hTPgbh%8tGB?{a1&Q~(1tlIYwOa<~t?Y7i0FwWpAm&%w3>$3yX>$CkV=kK{iKn4H+WT(}'
+        'q004R{^A1!6n^tD2tr1x6%>>XF`v>*^)#8nL0|1e?DftlvAFwFeAF$XZWiN~!=MB-'
+        ')%y4Y=rR4G)EaZX&1OUEp1<C>d*7Od&tp%(2RR<MV>!*wH=mT8|F1r`V8o;SMMa`brR|Mh~)D~z}TUB;0w(1`b6Zv_IkSvq~',
+    ],
+}
+
+
+def _arm_scene(envs, dt):
+    scene = gs.Scene(sim_options=gs.options.SimOptions(dt=dt),
+                     rigid_options=gs.options.RigidOptions(enable_self_collision=False))
+    scene.add_entity(gs.morphs.Plane())
+    arm = scene.add_entity(gs.morphs.MJCF(file="xml/franka_emika_panda/panda.xml"))
+    scene.build(n_envs=envs)
+    return scene, arm
+
+
+def _arm_state(g, scene, arm):
+    n = scene.n_envs
+    spread = torch.tensor([0.5, 0.12, 0.5, 0.12, 0.3, 0.2, 0.6, 0.01, 0.01], device=DEV)
+    home = torch.tensor(ARM_HOME, device=DEV)
+    arm.set_qpos(home + spread * _uniform(g, (n, 9), -1.0, 1.0))
+    arm.set_dofs_velocity(_uniform(g, (n, 9), -0.3, 0.3) * (spread > 0.05))
+
+
+def _quadruped_scene(envs, dt, randomized=False):
+    ro = gs.options.RigidOptions(batch_dofs_info=True, batch_links_info=True) if randomized else None
+    scene = gs.Scene(sim_options=gs.options.SimOptions(dt=dt), rigid_options=ro)
+    scene.add_entity(gs.morphs.Plane())
+    dog = scene.add_entity(gs.morphs.URDF(file="urdf/go2/urdf/go2.urdf"))
+    scene.build(n_envs=envs)
+    return scene, dog
+
+
+def _quadruped_state(g, scene, dog):
+    n = scene.n_envs
+    yaw = _uniform(g, (n,), -math.pi, math.pi) / 2
+    tilt = _uniform(g, (n, 2), -0.02, 0.02)
+    zero = torch.zeros_like(yaw)
+    q = _quat_mul(torch.stack([torch.cos(yaw), zero, zero, torch.sin(yaw)], -1),
+                  torch.stack([zero + 1, tilt[:, 0], tilt[:, 1], zero], -1))
+    q = torch.nn.functional.normalize(q, dim=-1)
+    joints = torch.tensor(STANDING, device=DEV) + _uniform(g, (n, 12), -0.08, 0.08)
+    base = torch.cat([_uniform(g, (n, 2), -1.0, 1.0), _uniform(g, (n, 1), 0.325, 0.345)], -1)
+    dog.set_qpos(torch.cat([base, q, joints], -1))
+    dog.set_dofs_velocity(_uniform(g, (n, 18), -0.2, 0.2))
+
+
+def _randomize(g, scene, dog):
+    n = scene.n_envs
+    legs = list(range(6, 18))
+    kp, kv = _uniform(g, (n, 1), 80.0, 120.0), _uniform(g, (n, 1), 8.0, 12.0)
+    dog.set_dofs_kp(kp.expand(n, 12), legs)
+    dog.set_dofs_kv(kv.expand(n, 12), legs)
+    dog.set_dofs_damping(_uniform(g, (n, 12), 0.0, 0.1), legs)
+    dog.set_mass_shift(_uniform(g, (n, 1), -0.5, 1.0), [0])
+    dog.set_COM_shift(_uniform(g, (n, 1, 3), -0.02, 0.02), [0])
+    dog.set_friction_ratio(_uniform(g, (n, dog.n_links), 0.6, 1.4))
+
+
+def _pile_scene(boxes, envs, dt, seed):
+    scene = gs.Scene(sim_options=gs.options.SimOptions(dt=dt),
+                     rigid_options=gs.options.RigidOptions(max_collision_pairs=1000))
+    scene.add_entity(gs.morphs.Plane())
+    heaps, sizes = _heaps(boxes, seed)
+    for i in range(boxes):
+        scene.add_entity(gs.morphs.Box(size=tuple(sizes[i]), pos=(0.0, 0.0, 0.5 + i)),
+                         material=gs.materials.Rigid(rho=1000.0, friction=1.0))
+    scene.build(n_envs=envs)
+    return scene, torch.as_tensor(heaps, dtype=torch.float32, device=DEV)
+
+
+def _pile_state(g, scene, heaps):
+    """Every env holds one of the heaps, turned about the vertical and moved, each box displaced by a few hundredths of
+    a millimetre, with the slow motion of a heap that has nearly come to rest."""
+    n, b = scene.n_envs, heaps.shape[1]
+    heap = heaps[torch.arange(n, device=DEV) % len(heaps)]
+    half = _uniform(g, (n, 1), -math.pi, math.pi) / 2
+    zero = torch.zeros_like(half)
+    turn = torch.stack([torch.cos(half), zero, zero, torch.sin(half)], -1)  # (n, 1, 4)
+    p, q = heap[..., :3], heap[..., 3:]
+    c, s = torch.cos(2 * half), torch.sin(2 * half)
+    p = torch.stack([c * p[..., 0] - s * p[..., 1], s * p[..., 0] + c * p[..., 1], p[..., 2]], -1)
+    p = p + 2e-5 * torch.randn((n, b, 3), generator=g, device=DEV)
+    p[..., :2] += _uniform(g, (n, 1, 2), -0.2, 0.2)
+    q = torch.nn.functional.normalize(_quat_mul(turn.expand(n, b, 4), q), dim=-1)
+    solver = scene.rigid_solver
+    solver.set_qpos(torch.cat([p, q], -1).reshape(n, 7 * b))
+    solver.set_dofs_velocity(0.02 * torch.randn((n, 6 * b), generator=g, device=DEV))
+
+
+def _arm_targets(g, envs):
+    return _uniform(g, (envs, 9), ARM_LO, ARM_HI)
+
+
+def _leg_targets(g, envs, steps):
+    return [torch.tensor(STANDING, device=DEV) + _uniform(g, (envs, 12), -0.3, 0.3) for _ in range(steps)]
+
+
+# ---- prepare / run ----------------------------------------------------------------------------------------------
+def prepare(case, seed):
+    family, n, dt, steps = case["family"], case["envs"], case["dt"], case["steps"]
+    g = _gen(seed)
+    if family == "arm":
+        scene, arm = _arm_scene(n, dt)
+        _arm_state(g, scene, arm)
+        if case["loop"] == "control":  # the controller moves between two poses close to the present one
+            home = arm.get_qpos()
+            targets = [home + _uniform(g, (n, 9), -0.05, 0.05), home]
+        else:
+            targets = [_arm_targets(g, n)]
+        return {"family": family, "scene": scene, "robot": arm, "targets": targets, "steps": steps, "turn": 0,
+                "start": scene.get_state() if case["loop"] == "rollout" else None}
+    if family == "quadruped":
+        scene, dog = _quadruped_scene(n, dt, case.get("randomized", False))
+        if case.get("randomized", False):
+            _randomize(g, scene, dog)
+        _quadruped_state(g, scene, dog)
+        return {"family": family, "scene": scene, "robot": dog, "targets": _leg_targets(g, n, 4), "steps": steps,
+                "legs": list(range(6, 18)), "turn": 0}
+    if family == "pile":
+        scene, heaps = _pile_scene(case["boxes"], n, dt, seed)
+        _pile_state(g, scene, heaps)
+        return {"family": family, "scene": scene, "steps": steps, "start": scene.get_state()}
+    if family == "mixed":
+        counts = [max(1, int(n * x)) for x in MIX]
+        (arms, arm), (dogs, dog) = _arm_scene(counts[0], dt), _quadruped_scene(counts[1], dt)
+        piles, heaps = _pile_scene(20, counts[2], dt, seed)
+        _arm_state(g, arms, arm)
+        _quadruped_state(g, dogs, dog)
+        _pile_state(g, piles, heaps)
+        scenes = [arms, dogs, piles]
+        # the plan autotune() settles on for this mix: heavy tiles first, one launch per stage
+        batch = FusedBatch([Group(dogs.rigid_solver, envs_per_tile=64, solver_variant=1, collide_variant=0,
+                                  wave_envs_per_tile=1),
+                            Group(arms.rigid_solver, envs_per_tile=8, solver_variant=1, collide_variant=1),
+                            Group(piles.rigid_solver, envs_per_tile=1, solver_variant=1, collide_variant=1)],
+                           phased=True)
+        batch.capture(1)
+        return {"family": family, "scenes": scenes, "start": [s.get_state() for s in scenes], "batch": batch, "arm": arm,
+                "dog": dog, "targets": _arm_targets(g, counts[0]), "steps": steps, "leg_targets": _leg_targets(g, counts[1], steps),
+                "legs": list(range(6, 18))}
+    if family == "serve":
+        scenes = ("arm", "quadruped", "pile20")
+        r, seeds = np.random.default_rng(n), np.random.default_rng(seed)  # the burst's sizes belong to the case
+        wanted = [Request(i, scenes[i % 3], 1 + int(r.integers(n)), max(2, steps - int(r.integers(5))), 0.0,
+                          seed=int(seeds.integers(1 << 31))) for i in range(case["requests"])]
+        # three quarters of what the burst asks for is resident, so the last requests wait for tiles
+        pools = {}
+        for s in scenes:
+            asked = [q.n_envs for q in wanted if q.scene == s]
+            pools[s] = Pool(s, max(asked + [1, 3 * sum(asked) // 4]), dt=dt)
+        return {"family": family, "server": Server(pools, 12 << 30), "wanted": wanted}
+    scene, dog = _quadruped_scene(n, dt)
+    quat = torch.nn.functional.normalize(torch.randn((n, 4), generator=g, device=DEV), dim=-1)
+    joints = torch.tensor(STANDING, device=DEV) + _uniform(g, (n, 12), -0.5, 0.5)
+    return {"family": family, "scene": scene, "robot": dog,
+            "qpos": torch.cat([_uniform(g, (n, 3), -1.0, 1.0), quat, joints], -1)}
+
+
+def run(state):
+    family = state["family"]
+    if family == "arm":
+        scene, arm = state["scene"], state["robot"]
+        if state["start"] is not None:
+            scene.reset(state["start"])
+        arm.control_dofs_position(state["targets"][state["turn"]])
+        state["turn"] = (state["turn"] + 1) % len(state["targets"])
+        for _ in range(state["steps"]):
+            scene.step()
+        return [arm.get_dofs_position(), arm.get_dofs_velocity(), arm.get_links_pos(), arm.get_links_quat()]
+    if family == "quadruped":
+        scene, dog, out = state["scene"], state["robot"], None
+        for _ in range(state["steps"]):
+            dog.control_dofs_position(state["targets"][state["turn"]], state["legs"])
+            state["turn"] = (state["turn"] + 1) % len(state["targets"])
+            scene.step()
+            out = [dog.get_qpos(), dog.get_dofs_velocity(), dog.get_links_net_contact_force()]
+        return out
+    if family == "pile":
+        scene = state["scene"]
+        scene.reset(state["start"])
+        for _ in range(state["steps"]):
+            scene.step()
+        return [scene.rigid_solver.get_qpos(), scene.rigid_solver.get_dofs_velocity()]
+    if family == "mixed":
+        for scene, start in zip(state["scenes"], state["start"]):
+            scene.reset(start)
+        state["arm"].control_dofs_position(state["targets"])
+        for k in range(state["steps"]):
+            state["dog"].control_dofs_position(state["leg_targets"][k], state["legs"])
+            state["batch"].replay()
+        return [x for s in state["scenes"] for x in (s.rigid_solver.get_qpos(), s.rigid_solver.get_dofs_velocity())]
+    if family == "serve":
+        requests = [Request(r.rid, r.scene, r.n_envs, r.horizon, 0.0, r.seed) for r in state["wanted"]]
+        state["server"].run(requests, record=True)
+        return [x for r in requests for x in (r.result["qpos"], r.result["vel"])]
+    dog = state["robot"]
+    dog.set_qpos(state["qpos"], zero_velocity=False)
+    return [dog.get_links_pos(), dog.get_links_quat()]
+
+
+# ---- what a pass cannot do without ------------------------------------------------------------------------------
+def _step_work(family, boxes, envs):
+    """Bytes: positions, velocities, warm start in and out and targets in; operations: the mass matrix, its
+    factorisation, bias forces and two Newton solves of the block-sparse system, per env."""
+    if family == "pile":
+        d, q, c, links, blocks = 6 * boxes, 7 * boxes, 0, boxes, boxes * 6 ** 3
+    else:
+        (d, q, c), links = SIZES[family], 13
+        blocks = d ** 3
+    rows = {"arm": 4, "quadruped": 20}.get(family, 15 * boxes)
+    flops = 700 * links + 14 * d * d + blocks + 2 * (blocks + rows * 12 * 16)
+    return 4 * envs * (2 * q + 4 * d + c), flops * envs
+
+
+def work(case):
+    family, n, steps = case["family"], case["envs"], case["steps"]
+    if family in ("arm", "quadruped", "pile"):
+        b, f = _step_work(family, case.get("boxes", 0), n)
+        return {"bytes": b * steps, "flops": f * steps}
+    if family == "mixed":
+        parts = [_step_work(k, 20, max(1, int(n * x))) for k, x in zip(("arm", "quadruped", "pile"), MIX)]
+        return {"bytes": sum(p[0] for p in parts) * steps, "flops": sum(p[1] for p in parts) * steps}
+    if family == "serve":
+        parts = [_step_work(k, 20, n / 2 * case["requests"] / 3) for k in ("arm", "quadruped", "pile")]
+        return {"bytes": sum(p[0] for p in parts) * (steps - 2), "flops": sum(p[1] for p in parts) * (steps - 2)}
+    return {"bytes": 4 * n * (19 + 13 * 7), "flops": n * 13 * 150}
+
+
+def exact(case, seed):
+    """Link poses in 64 bits from the robot's description; None for whole steps, whose contact sets and iteration
+    counts are decisions in 32 bits, with no value of their own in 64."""
+    if case["family"] != "pose":
+        return None
+    n, g = case["envs"], _gen(seed)
+    quat = torch.nn.functional.normalize(torch.randn((n, 4), generator=g, device=DEV), dim=-1)
+    joints = torch.tensor(STANDING, device=DEV) + _uniform(g, (n, 12), -0.5, 0.5)
+    base = torch.cat([_uniform(g, (n, 3), -1.0, 1.0), quat], -1).double()
+    joints = joints.double()
+    with open(os.path.join(os.path.dirname(gs.__file__), "assets", "go2.json")) as f:
+        links = json.load(f)["links"]
+
+    def turned(v, q):
+        return (_quat_mat(q) * v[:, None, :]).sum(-1)
+
+    pos, rot, at = [], [], 0
+    for link in links:
+        def const(x):
+            return torch.tensor(np.float32(x), dtype=torch.float64, device=DEV).expand(n, -1)
+        if link["parent"] < 0:
+            p, q = base[:, :3], base[:, 3:] / base[:, 3:].norm(dim=-1, keepdim=True)
+        else:
+            par = link["parent"]
+            p, q = pos[par] + turned(const(link["pos"]), rot[par]), _quat_mul(rot[par], const(link["quat"]))
+            for j in link["joints"]:
+                if j["type"] == 1:
+                    half = joints[:, at:at + 1] / 2
+                    at += 1
+                    q = _quat_mul(q, torch.cat([torch.cos(half), torch.sin(half) * const(j["axis"])], -1))
+        pos.append(p)
+        rot.append(q)
+    return [torch.stack(pos, 1), torch.stack(rot, 1)]
