@@ -354,10 +354,12 @@ def prepare(case, seed):
         _quadruped_state(g, dogs, dog)
         _pile_state(g, piles, heaps)
         scenes = [arms, dogs, piles]
-        # the plan autotune() settles on for this mix: heavy tiles first, one launch per stage
-        batch = FusedBatch([Group(dogs.rigid_solver, envs_per_tile=64, solver_variant=1, collide_variant=0,
-                                  wave_envs_per_tile=1),
-                            Group(arms.rigid_solver, envs_per_tile=8, solver_variant=1, collide_variant=1),
+        # the plans autotune() settles on for this mix: heavy tiles first, one launch per stage; with few envs a tile is
+        # one env, and the quadrupeds collide one wavefront per env too
+        many = counts[1] > 2048
+        batch = FusedBatch([Group(dogs.rigid_solver, envs_per_tile=64 if many else 1, solver_variant=1,
+                                  collide_variant=0 if many else 1, wave_envs_per_tile=1),
+                            Group(arms.rigid_solver, envs_per_tile=8 if many else 1, solver_variant=1, collide_variant=1),
                             Group(piles.rigid_solver, envs_per_tile=1, solver_variant=1, collide_variant=1)],
                            phased=True)
         batch.capture(1)
