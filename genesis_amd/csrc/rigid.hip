@@ -189,7 +189,7 @@ int check(const gsr_model* m, const gsr_state* s) {
   if (m->n_geoms >= (1 << 15)) return GSR_E_SHAPE;
   if (m->solver_variant == 1) {
     if (m->n_entities > kMaxPatternEntities) return GSR_E_SHAPE;
-    if (m->wave_h_floats < 0 || wave_lds_bytes(*m) > 160 * 1024)
+    if (m->wave_h_floats < 0 || solve_lds_bytes(*m) > 160 * 1024)
       return GSR_E_SHAPE;
   }
   if (m->collide_variant == 1) {
@@ -469,7 +469,7 @@ static int phase_lds(const gsr_batch_info& b, int phase) {
     const gsr_model& m = b.models[k];
     if (phase == 1 && m.collide_variant == 1) lds = std::max(lds, (size_t)wave_collide_lds_bytes(m.n_geoms));
     if (phase == 3 && m.solver_variant == 1)
-      lds = std::max(lds, (size_t)wave_lds_bytes(m));
+      lds = std::max(lds, (size_t)solve_lds_bytes(m));
   }
   return (int)lds;
 }
@@ -506,7 +506,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
       out.states[type] = G.state;
     }
     if (G.model.solver_variant == 1)
-      lds = std::max(lds, wave_lds_bytes(G.model));
+      lds = std::max(lds, solve_lds_bytes(G.model));
     if (G.model.collide_variant == 1) lds = std::max(lds, wave_collide_lds_bytes(G.model.n_geoms));
     const int n_t = (G.n_envs + G.envs_per_tile - 1) / G.envs_per_tile, n_w = (G.n_envs + Tw - 1) / Tw;
     ranges[g] = BatchRange{type, G.env_begin, G.n_envs, G.envs_per_tile, tiles, tiles + n_t, Tw, wtiles, wtiles + n_w,
@@ -625,7 +625,7 @@ int gsr_launch_fused_kernel(const void* dev_table, const gsr_batch_info* info, i
   } else {
     const gsr_model& m = info->models[k - 1];
     const gsr_state& st = info->states[k - 1];
-    const size_t lds = m.solver_variant == 1 ? wave_lds_bytes(m) : 0;
+    const size_t lds = m.solver_variant == 1 ? solve_lds_bytes(m) : 0;
     launch_gjk_resume(m, st, (unsigned)lds, stream);
   }
   return launch_status();
@@ -730,7 +730,7 @@ int gsr_serve_init(const gsr_serve_pool* pools, int32_t n_pools, double mem_budg
     out.models[p] = P.model;
     out.states[p] = P.state;
     if (P.model.solver_variant == 1)
-      lds = std::max(lds, wave_lds_bytes(P.model));
+      lds = std::max(lds, solve_lds_bytes(P.model));
     if (P.model.collide_variant == 1) lds = std::max(lds, wave_collide_lds_bytes(P.model.n_geoms));
     tiles += P.n_tiles;
   }

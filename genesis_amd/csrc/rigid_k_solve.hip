@@ -17,14 +17,25 @@ __global__ void __launch_bounds__(kWave) k_solve_wave(gsr_model m, gsr_state s) 
   if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
   const int b = xcd_env(blockIdx.x, s.n_envs);
   Env e(m, s, b);
-  wave_solve(e, lds);
+  wave_solve_blocks(e, lds);
+}
+
+// the single-entity solver alone: it takes about half the registers of the entity-block solver, so a SIMD holds more envs
+__global__ void __launch_bounds__(kWave) k_solve_dense(gsr_model m, gsr_state s) {
+  extern __shared__ char lds[];
+  if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
+  const int b = xcd_env(blockIdx.x, s.n_envs);
+  Env e(m, s, b);
+  wave_solve_dense(e, lds);
 }
 
 }  // namespace
 
 void launch_solve(const gsr_model& m, const gsr_state& s, hipStream_t st) {
-  if (m.solver_variant == 1)
-    hipLaunchKernelGGL(k_solve_wave, dim3(s.n_envs), dim3(kWave), wave_lds_bytes(m), st, m, s);
+  if (m.solver_variant == 1 && dense_solver(m))
+    hipLaunchKernelGGL(k_solve_dense, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
+  else if (m.solver_variant == 1)
+    hipLaunchKernelGGL(k_solve_wave, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
   else
     hipLaunchKernelGGL(k_solve, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);
 }

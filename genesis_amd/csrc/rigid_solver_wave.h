@@ -13,10 +13,9 @@
 // Vectors over dofs live in LDS; constraint rows live in global memory, env-major.
 #pragma once
 #include "rigid_env.h"
+#include "rigid_wave.h"
 
 namespace gsr {
-
-constexpr int kWave = 64;
 
 // LDS pointers carry their address space so every access compiles to ds_* instructions (not flat), and the compiler
 // knows they never alias global memory.
@@ -26,22 +25,6 @@ typedef GSR_LDS int lds_i;
 typedef GSR_LDS unsigned long long lds_u64;
 typedef GSR_LDS char lds_c;
 constexpr int kMaxPatternEntities = 128;  // two 64-bit words per entity row of the pattern
-
-__device__ __forceinline__ float wave_sum(float v) {
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-// Sums over rows or dofs whose rounding steers discrete decisions (the line search's bracketing, the Newton stop
-// test) are accumulated in double: the reference adds them one by one in FP32, an order a wavefront cannot follow,
-// and a tree of FP32 partial sums has a different rounding error; the double sum is closer to both.
-__device__ __forceinline__ double wave_sum_d(double v) {
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-__device__ __forceinline__ int wave_or(int v) {
-  for (int o = kWave / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
-  return v;
-}
 
 // A constraint row of up to kStage entries (every row of the arm, quadruped and box scenes) is loaded into
 // registers with independent loads before it is used, so a lane does not wait for one global load per entry; wider
@@ -172,12 +155,6 @@ struct WaveCtx {
   const Env& e;
   const WaveLds& L;
   int lane, D, E, n_con, ne, nef;
-  // Models whose dofs all belong to one entity (an arm or a legged robot over a plane), at most 64 of them, with H
-  // in LDS: H is one dense packed triangle (dense_h), and the rows staged per pass of the dense sums below (0: the
-  // per-entity row walk) with their LDS staging area
-  bool dense_h;
-  int dense_rows;
-  lds_f* dense_buf;
   // entity-block mass matrix entry (i, j) of entity ie (model numbering: entity and dofs), geometry read from LDS
   __device__ __forceinline__ float mm(int ie, int i, int j) const {
     int st = L.nes[ie], n = L.nee[ie] - st;
@@ -208,13 +185,11 @@ __device__ inline void wave_min_degree(const WaveCtx& w, unsigned long long (&ad
     // (degree, entity) minimum over the alive entities
     int k0 = has0 && ((al0 >> lane) & 1ull) ? ((__popcll(adj0[0] & al0) + __popcll(adj0[1] & al1)) << 8) | e0 : 0x7fffffff;
     int k1 = has1 && ((al1 >> lane) & 1ull) ? ((__popcll(adj1[0] & al0) + __popcll(adj1[1] & al1)) << 8) | e1 : 0x7fffffff;
-    int k = min(k0, k1);
-    for (int o = kWave / 2; o > 0; o >>= 1) k = min(k, __shfl_xor(k, o, kWave));
-    const int v = k & 0xff;
+    const int v = __builtin_amdgcn_readfirstlane(wave_min_i(min(k0, k1))) & 0xff;
     // v's live neighbours become a clique
     const int src = v & 63;
-    unsigned long long n0 = __shfl(v < 64 ? adj0[0] : adj1[0], src, kWave);
-    unsigned long long n1 = __shfl(v < 64 ? adj0[1] : adj1[1], src, kWave);
+    unsigned long long n0 = lane_value(v < 64 ? adj0[0] : adj1[0], src);
+    unsigned long long n1 = lane_value(v < 64 ? adj0[1] : adj1[1], src);
     if (v < 64) al0 &= ~(1ull << v); else al1 &= ~(1ull << (v - 64));
     n0 &= al0;
     n1 &= al1;
@@ -244,7 +219,7 @@ __device__ inline void wave_min_degree(const WaveCtx& w, unsigned long long (&ad
 // set: measured on 20-box piles (120 dofs) the solve takes 15 % less time, on 64-box piles (384 dofs, six passes)
 // 15 % more, hence the bound.
 __device__ __forceinline__ bool wave_dof_lanes(const WaveCtx& w) {
-  return w.dense_rows == 0 && w.e.m.row_width <= kStage && w.D <= 2 * kWave;
+  return w.e.m.row_width <= kStage && w.D <= 2 * kWave;
 }
 
 // The entries of entity ea (eb) in row c as one run: first dof | position << 16 | count << 24 when they are
@@ -382,7 +357,7 @@ __device__ inline void wave_build_structure(const WaveCtx& w) {
     if (runs && valid) row_runs(w, c, ea, eb, run_a, run_b);
     int rank_a = 0, rank_b = 0, cnt_a = 0, cnt_b = 0;
     for (int j = 0; j < kWave; j++) {
-      int ra = __shfl(ea, j, kWave), rb = __shfl(eb, j, kWave);
+      const int ra = lane_value(ea, j), rb = lane_value(eb, j);
       bool ta = valid && (ra == ea || rb == ea);
       bool tb = valid && (ra == eb || rb == eb);
       if (j < w.lane) { rank_a += ta; rank_b += tb; }
@@ -528,106 +503,6 @@ struct HLds {
   __device__ __forceinline__ lds_f* blk(int i, int ei, int ek) const { return row(i, ei) + off(ei, ek) + L.es[ek]; }
 };
 
-// ---- single-entity models: rows staged densely --------------------------------------------------------------------
-// When every dof belongs to one entity, every row touches only that entity and its row list is every row in
-// ascending order. J^T f and the J^T D J part of the Hessian are then summed with one lane per dof (per entry) over
-// rows staged densely in LDS, dense_rows at a time, instead of one lane walking every row through global memory.
-// Each sum adds the general path's terms in the same row order from +0 (an absent dof contributes +-0, which changes
-// no bit of a sum that starts at +0), so both paths give the same bits.
-
-// lane-local: row c into staging slot `lane` (values over the model's dofs, zero elsewhere) with its scale, or a
-// zero row when `use` is false
-__device__ __forceinline__ void dense_stage_row(const WaveCtx& w, int c, bool use, float scale) {
-  const Env& e = w.e;
-  lds_f* row = w.dense_buf + w.lane * w.D;
-  for (int d = 0; d < w.D; d++) row[d] = 0.f;
-  if (use) {
-    const int nnz = e.EI(e.s.jac_nnz, c);
-    if (nnz <= kStage) {
-      RowStage r;
-      stage_row(e, c, nnz, r);
-#pragma unroll
-      for (int k = 0; k < kStage; k++)
-        if (k < nnz) row[r.d[k]] = r.v[k];
-    } else {
-      for (int k = 0; k < nnz; k++) row[e.JI(c, k)] = e.JV(c, k);
-    }
-  }
-  w.dense_buf[w.dense_rows * w.D + w.lane] = use ? scale : 0.f;
-}
-
-// J^T f into L.qfrc (lane d owns dof d)
-__device__ inline void wave_jtf_dense(const WaveCtx& w) {
-  const Env& e = w.e;
-  const int D = w.D, R = w.dense_rows;
-  const lds_f* sc = w.dense_buf + R * D;
-  float acc = 0.f;
-  for (int c0 = 0; c0 < w.n_con; c0 += R) {
-    const int nr = min(R, w.n_con - c0);
-    if (w.lane < nr) {
-      const float f = e.EF(e.s.efc_force, c0 + w.lane);
-      dense_stage_row(w, c0 + w.lane, f != 0.f, f);
-    }
-    __syncthreads();
-    if (w.lane < D) {
-      const lds_f* col = w.dense_buf + w.lane;
-      for (int r = 0; r < nr; r++) acc = acc + col[r * D] * sc[r];
-    }
-    __syncthreads();
-  }
-  if (w.lane < D) w.L.qfrc[w.lane] = acc;
-}
-
-// H = M + J^T D J over the active rows, lanes over the entries of the lower triangle (entry t = i (i + 1) / 2 + j,
-// j <= i, for t = lane, lane + 64, ...); each entry's partial sum waits in the entry itself between passes
-__device__ __forceinline__ void dense_entry(int t, int& i, int& j) {
-  i = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
-  while (i * (i + 1) / 2 > t) i--;
-  while ((i + 1) * (i + 2) / 2 <= t) i++;
-  j = t - i * (i + 1) / 2;
-}
-
-template <class HS>
-__device__ inline void wave_hessian_dense(const WaveCtx& w, const HS& h) {
-  const Env& e = w.e;
-  const gsr_state& s = e.s;
-  const WaveLds& L = w.L;
-  const int D = w.D, R = w.dense_rows, ntri = D * (D + 1) / 2;
-  const float eps = e.m.eps;
-  const lds_f* sc = w.dense_buf + R * D;
-  const int v = L.ent_of_dof[0], ne = L.ord[v], n0 = L.nes[ne], f0 = L.es[v];
-  for (int c0 = 0; c0 < w.n_con; c0 += R) {
-    const int nr = min(R, w.n_con - c0);
-    if (w.lane < nr) {
-      const int c = c0 + w.lane;
-      dense_stage_row(w, c, (e.EI(s.efc_active, c) & 1) != 0, e.EF(s.efc_D, c));
-    }
-    __syncthreads();
-    for (int t = w.lane; t < ntri; t += kWave) {
-      int i, j;
-      dense_entry(t, i, j);
-      // pair (row's later dof i, earlier dof j), skipped when |J[c, i]| <= eps, as the row walk skips it
-      const lds_f* pi = w.dense_buf + i;
-      const lds_f* pj = w.dense_buf + j;
-      auto q = h.blk(f0 + i, v, v) + j;
-      float a = c0 == 0 ? 0.f : *q;
-      for (int r = 0; r < nr; r++) {
-        const float vi = pi[r * D];
-        const float vm = fabsf(vi) > eps ? vi : 0.f;
-        a = a + pj[r * D] * vm * sc[r];
-      }
-      *q = a;
-    }
-    __syncthreads();
-  }
-  for (int t = w.lane; t < ntri; t += kWave) {
-    int i, j;
-    dense_entry(t, i, j);
-    auto q = h.blk(f0 + i, v, v) + j;
-    *q = (w.n_con > 0 ? *q : 0.f) + w.mm(ne, n0 + i, n0 + j);
-  }
-}
-
 // M x (entity blocks), one dof per lane, serial inner sum in the reference order
 __device__ inline void wave_mass_mul(const WaveCtx& w, const lds_f* x, lds_f* out) {
   const Env& e = w.e;
@@ -673,9 +548,7 @@ __device__ inline void wave_update_constraint(const WaveCtx& w, double& cost, fl
   const int* ptr = s.ent_row_ptr + (size_t)e.b * (w.E + 1);
   const int* lst = s.ent_row_list + (size_t)e.b * 2 * e.m.max_rows;
   const bool split = wave_dof_lanes(w);
-  if (w.dense_rows > 0) {
-    wave_jtf_dense(w);
-  } else if (split) {
+  if (split) {
     // one lane per dof walks the rows of its dof's entity, two rows per iteration (both rows' loads issued before
     // either is used, the next pair's indices loaded meanwhile), and sums entry(row, d) * force in row order from
     // +0 in a register: the per-entity walk's terms in its order, so the same bits
@@ -724,7 +597,7 @@ __device__ inline void wave_update_constraint(const WaveCtx& w, double& cost, fl
     for (int d = w.lane; d < w.D; d += kWave) L.qfrc[d] = 0.f;
     __syncthreads();
   }
-  for (int ie = w.lane; ie < w.E && w.dense_rows == 0 && !split; ie += kWave) {
+  for (int ie = w.lane; ie < w.E && !split; ie += kWave) {
     const int s0 = L.nes[ie], s1 = L.nee[ie];
     if (s1 <= s0) continue;
     // two rows per iteration: both rows' loads are issued before either is accumulated (in row order); the next
@@ -827,108 +700,6 @@ __device__ __forceinline__ LaneGroup lane_group(int n, int lane) {
   while (G > 1 && G * n > kWave) G >>= 1;
   return LaneGroup{G, lane / G, lane & (G - 1), kWave / G};
 }
-__device__ __forceinline__ float group_sum(float v, int G) {
-  for (int o = G >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-
-// ---- single-entity models: the factor as one dense packed triangle ------------------------------------------------
-// With every dof in one entity and H in LDS, H is the packed lower triangle at the start of the LDS store, H(i, j) at
-// hl[i (i + 1) / 2 + j] (factor and model numbering agree). The factorisation, the substitutions and the rank-1
-// updates then run with one lane per row and every sum serial over its index, the operation order of
-// func_nt_chol_factor / func_nt_chol_solve / func_nt_hessian_incremental (constraint_solver_decomp.py), instead of
-// the chunked per-entity forms below with their pattern lookups.
-__device__ __forceinline__ lds_f* dense_row(const WaveLds& L, int i) { return L.hl + i * (i + 1) / 2; }
-
-__device__ inline void wave_chol_factor_dense(const WaveCtx& w) {
-  const float EPS = w.e.m.eps;
-  const int D = w.D;
-  for (int i = 0; i < D; i++) {
-    lds_f* ri = dense_row(w.L, i);
-    float tmp = ri[i];
-#pragma unroll 8
-    for (int j = 0; j < i; j++) {
-      const float h = ri[j];
-      tmp -= h * h;
-    }
-    const float hii = sqrtf(fmaxf(tmp, EPS));
-    const float inv = 1.f / hii;
-    // rows j > i, one per lane
-    for (int j = i + 1 + w.lane; j < D; j += kWave) {
-      lds_f* rj = dense_row(w.L, j);
-      float dt = 0.f;
-#pragma unroll 8
-      for (int k = 0; k < i; k++) dt += rj[k] * ri[k];
-      rj[i] = (rj[i] - dt) * inv;
-    }
-    if (w.lane == 0) ri[i] = hii;
-    __syncthreads();
-  }
-}
-
-// x = H^-1 x in place, lane d holding x[d] in a register: forward substitution (row i subtracts L(i, j) y(j) for j
-// ascending as y(j) becomes final: the serial order of func_nt_chol_solve), then backward substitution column by
-// column (row i subtracts L(j, i) x(j) for j descending as x(j) becomes final)
-__device__ inline void wave_chol_solve_dense(const WaveCtx& w, lds_f* x) {
-  const int D = w.D, lane = w.lane;
-  __syncthreads();
-  float a = lane < D ? x[lane] : 0.f;
-  const lds_f* rl = dense_row(w.L, lane < D ? lane : 0);
-  for (int j = 0; j < D; j++) {
-    const float yj = __shfl(a, j, kWave) / dense_row(w.L, j)[j];
-    if (lane == j) a = yj;
-    else if (lane > j && lane < D) a = a - rl[j] * yj;
-  }
-  for (int i = D - 1; i >= 0; i--) {
-    const lds_f* ri = dense_row(w.L, i);
-    const float xi = __shfl(a, i, kWave) / ri[i];
-    if (lane == i) a = xi;
-    else if (lane < i) a = a - ri[lane] * xi;
-  }
-  if (lane < D) x[lane] = a;
-  __syncthreads();
-}
-
-// rank-1 update / downdate of the factor with row c; returns false on rank loss (the update is then incomplete and
-// the caller rebuilds the factor)
-__device__ inline bool wave_rank1_dense(const WaveCtx& w, int c, float sgn) {
-  const Env& e = w.e;
-  const gsr_state& s = e.s;
-  const float eps = e.m.eps;
-  const int D = w.D, lane = w.lane;
-  const float sq = sqrtf(e.EF(s.efc_D, c));
-  lds_f* x = w.L.vec;
-  for (int d = lane; d < D; d += kWave) x[d] = 0.f;
-  __syncthreads();
-  const int nnz = e.EI(s.jac_nnz, c);
-  for (int k = lane; k < nnz; k += kWave) x[e.JI(c, k)] = e.JV(c, k) * sq;
-  __syncthreads();
-  float xi = lane < D ? x[lane] : 0.f;
-  lds_f* rl = dense_row(w.L, lane < D ? lane : 0);
-  bool ok = true;
-  for (int k = 0; k < D; k++) {
-    const float vk = __shfl(xi, k, kWave);
-    if (!(fabsf(vk) > eps)) continue;
-    lds_f* dk = dense_row(w.L, k) + k;
-    const float Lkk = *dk;
-    float tmp = Lkk * Lkk + vk * vk * sgn;
-    if (tmp < eps) {
-      tmp = eps;
-      ok = false;
-    }
-    const float r = sqrtf(tmp), cc = r / Lkk, cinv = 1.f / cc, sv = vk / Lkk;
-    if (lane > k && lane < D) {
-      const float hv = (rl[k] + sv * xi * sgn) * cinv;
-      rl[k] = hv;
-      xi = xi * cc - sv * hv;
-    }
-    __syncthreads();
-    if (lane == 0) *dk = r;
-    __syncthreads();
-  }
-  return ok;
-}
-
 // Left-looking Cholesky over the pattern (func_nt_chol_factor's entries), level by level, lane groups per entity,
 // kChunk dofs of an entity at a time:
 //   1. the chunk's diagonal block less the products of its rows over the earlier columns (terms dealt round-robin
@@ -1155,18 +926,10 @@ __device__ __forceinline__ void wave_hessian_direct(const WaveCtx& w, const HS& 
   const WaveLds& L = w.L;
   const int* ptr = s.ent_row_ptr + (size_t)e.b * (w.E + 1);
   const int* lst = s.ent_row_list + (size_t)e.b * 2 * m.max_rows;
-  if (w.dense_rows > 0) {
-    wave_hessian_dense(w, h);
-    __syncthreads();
-    if (!HS::kFence && w.dense_h) wave_chol_factor_dense(w);
-    else wave_chol_factor(w, h);
-    return;
-  }
   if (wave_dof_lanes(w)) {
     wave_hessian_by_dof(w, h, ptr, lst);
     __syncthreads();
-    if (!HS::kFence && w.dense_h) wave_chol_factor_dense(w);
-    else wave_chol_factor(w, h);
+    wave_chol_factor(w, h);
     return;
   }
   for (int ei = w.lane; ei < w.E; ei += kWave) {
@@ -1269,8 +1032,7 @@ __device__ __forceinline__ void wave_hessian_direct(const WaveCtx& w, const HS& 
     }
   }
   __syncthreads();
-  if (!HS::kFence && w.dense_h) wave_chol_factor_dense(w);
-  else wave_chol_factor(w, h);
+  wave_chol_factor(w, h);
 }
 
 // rank-1 update / downdate of the factor with row c (func_nt_hessian_incremental); returns false on rank loss
@@ -1503,27 +1265,104 @@ __device__ __forceinline__ void wave_chol_solve(const WaveCtx& w, const HS& h, l
   }
 }
 
-// grad = M qacc - force - J^T f into vec (factor space), then vec = H^-1 grad in place; returns this lane's share
-// of |grad|^2 (dofs lane, lane + 64, ... in that order). The Newton direction is -vec read back through pdof.
-template <class HS>
-__device__ __forceinline__ double wave_update_gradient(const WaveCtx& w, const HS& h) {
+// grad = M qacc - force - J^T f, into vec (factor space) when `keep`; returns this lane's share of |grad|^2 (dofs
+// lane, lane + 64, ... in that order)
+template <bool keep>
+__device__ __forceinline__ double wave_gradient(const WaveCtx& w) {
   const WaveLds& L = w.L;
   const Env& e = w.e;
   double g2 = 0.0;
   for (int d = w.lane; d < w.D; d += kWave) {
     float g = L.Ma[d] - e.F(e.s.force, d) - L.qfrc[d];
     g2 += (double)(g * g);
-    L.vec[L.pdof[d]] = g;
+    if (keep) L.vec[L.pdof[d]] = g;
   }
-  if (!HS::kFence && w.dense_h) wave_chol_solve_dense(w, L.vec);
-  else wave_chol_solve(w, h, L.vec);
-  __syncthreads();
   return g2;
 }
 
 struct WLS {
   float alpha, cost, d0, d1;
 };
+
+// the line search's point at alpha from the quadratic coefficients of the smooth terms (qg) and the rows' sums (t)
+__device__ __forceinline__ WLS ls_point_from(const Env& e, float qg0, float qg1, float qg2, double t0, double t1, double t2,
+                                             float alpha, int& ls_it) {
+  const float T0 = (float)((double)qg0 + t0);
+  const float T1 = (float)((double)qg1 + t1);
+  const float T2 = (float)((double)qg2 + t2);
+  WLS p;
+  p.alpha = alpha;
+  p.cost = alpha * alpha * T2 + alpha * T1 + T0;
+  p.d0 = 2.f * alpha * T2 + T1;
+  p.d1 = 2.f * T2;
+  if (p.d1 <= 0.f) p.d1 = e.m.eps;
+  ls_it++;
+  return p;
+}
+
+// The points of the exact line search (func_linesearch, constraint_solver_decomp.py:1440-1792): point(alpha, ls_it)
+// evaluates one and counts it; returns the step
+template <class Point>
+__device__ __forceinline__ float linesearch_points(const gsr_model& m, float gtol, Point point) {
+  int ls_it = 0;
+  WLS p0 = point(0.f, ls_it);
+  WLS p1 = point(p0.alpha - p0.d0 / p0.d1, ls_it);
+  if (p0.cost < p1.cost) p1 = p0;
+  if (fabsf(p1.d0) < gtol) return p1.alpha;
+  float direction = (p1.d0 < 0.f) ? 1.f : -1.f;
+  int p2update = 0;
+  WLS p2 = p1;
+  while (p1.d0 * direction <= -gtol && ls_it < m.ls_iterations) {
+    p2 = p1;
+    p2update = 1;
+    p1 = point(p1.alpha - p1.d0 / p1.d1, ls_it);
+    if (fabsf(p1.d0) < gtol) return p1.alpha;
+  }
+  if (ls_it >= m.ls_iterations) return p1.alpha;
+  if (!p2update) return p1.alpha;
+  WLS p2n = p1;
+  WLS p1n = point(p1.alpha - p1.d0 / p1.d1, ls_it);
+  while (ls_it < m.ls_iterations) {
+    WLS pm = point((p1.alpha + p2.alpha) * 0.5f, ls_it);
+    // candidates p1n, p2n, pm in this order (named values, not an indexed array, so they stay in registers)
+    const WLS c0 = p1n, c1 = p2n, c2 = pm;
+    int best = -1;
+    float bcost = 0.f, balpha = 0.f;
+    auto consider = [&](const WLS& c, int idx) {
+      if (fabsf(c.d0) < gtol && (best < 0 || c.cost < bcost)) {
+        bcost = c.cost;
+        best = idx;
+        balpha = c.alpha;
+      }
+    };
+    consider(c0, 0);
+    consider(c1, 1);
+    consider(c2, 2);
+    if (best >= 0) return balpha;
+    // p1, then p2, moves to the candidates whose slope has its sign and is closer to zero
+    auto narrow = [&](WLS& p) {
+      int flag = 0;
+      auto step = [&](const WLS& c) {
+        if (p.d0 < 0.f && c.d0 < 0.f && p.d0 < c.d0) { p = c; flag = 1; }
+        else if (p.d0 > 0.f && c.d0 > 0.f && p.d0 > c.d0) { p = c; flag = 2; }
+      };
+      step(c0);
+      step(c1);
+      step(c2);
+      return flag;
+    };
+    const int f1 = narrow(p1);
+    p1n = p1;
+    if (f1 > 0) p1n = point(p1.alpha - p1.d0 / p1.d1, ls_it);
+    const int f2 = narrow(p2);
+    p2n = p2;
+    if (f2 > 0) p2n = point(p2.alpha - p2.d0 / p2.d1, ls_it);
+    if (f1 == 0 && f2 == 0) return pm.alpha;
+  }
+  if (p1.cost <= p2.cost && p1.cost < p0.cost) return p1.alpha;
+  if (p2.cost <= p1.cost && p2.cost < p1.cost) return p2.alpha;
+  return 0.f;
+}
 
 // The line search's per-row terms of rows lane, lane + 64, ..., up to kLsRows of them per lane, stay in registers
 // across its points; rows beyond are read back from the env's row arrays. Each point sums the same terms in the same
@@ -1567,17 +1406,7 @@ __device__ __forceinline__ WLS wave_ls_point(const WaveCtx& w, const LsCache& rc
   }
   for (int c = w.lane + kWave * kLsRows; c < w.n_con; c += kWave)
     ls_row_terms(w, c, e.EF(s.efc_Jaref, c), e.EF(s.efc_jv, c), e.QD(c, 0), e.QD(c, 1), e.QD(c, 2), alpha, t0, t1, t2);
-  const float T0 = (float)((double)qg0 + wave_sum_d(t0));
-  const float T1 = (float)((double)qg1 + wave_sum_d(t1));
-  const float T2 = (float)((double)qg2 + wave_sum_d(t2));
-  WLS p;
-  p.alpha = alpha;
-  p.cost = alpha * alpha * T2 + alpha * T1 + T0;
-  p.d0 = 2.f * alpha * T2 + T1;
-  p.d1 = 2.f * T2;
-  if (p.d1 <= 0.f) p.d1 = e.m.eps;
-  ls_it++;
-  return p;
+  return ls_point_from(e, qg0, qg1, qg2, wave_sum_d(t0), wave_sum_d(t1), wave_sum_d(t2), alpha, ls_it);
 }
 
 __device__ inline float wave_linesearch(const WaveCtx& w, float gauss) {
@@ -1628,70 +1457,14 @@ __device__ inline float wave_linesearch(const WaveCtx& w, float gauss) {
   }
   float qg0 = gauss, qg1 = (float)wave_sum_d(a1), qg2 = (float)wave_sum_d(a2);
   __syncthreads();
-  int ls_it = 0;
-  WLS p0 = wave_ls_point(w, rc, qg0, qg1, qg2, 0.f, ls_it);
-  WLS p1 = wave_ls_point(w, rc, qg0, qg1, qg2, p0.alpha - p0.d0 / p0.d1, ls_it);
-  if (p0.cost < p1.cost) p1 = p0;
-  if (fabsf(p1.d0) < gtol) return p1.alpha;
-  float direction = (p1.d0 < 0.f) ? 1.f : -1.f;
-  int p2update = 0;
-  WLS p2 = p1;
-  while (p1.d0 * direction <= -gtol && ls_it < m.ls_iterations) {
-    p2 = p1;
-    p2update = 1;
-    p1 = wave_ls_point(w, rc, qg0, qg1, qg2, p1.alpha - p1.d0 / p1.d1, ls_it);
-    if (fabsf(p1.d0) < gtol) return p1.alpha;
-  }
-  if (ls_it >= m.ls_iterations) return p1.alpha;
-  if (!p2update) return p1.alpha;
-  WLS p2n = p1;
-  WLS p1n = wave_ls_point(w, rc, qg0, qg1, qg2, p1.alpha - p1.d0 / p1.d1, ls_it);
-  while (ls_it < m.ls_iterations) {
-    WLS pm = wave_ls_point(w, rc, qg0, qg1, qg2, (p1.alpha + p2.alpha) * 0.5f, ls_it);
-    // candidates p1n, p2n, pm in this order (named values, not an indexed array, so they stay in registers)
-    const WLS c0 = p1n, c1 = p2n, c2 = pm;
-    int best = -1;
-    float bcost = 0.f, balpha = 0.f;
-    auto consider = [&](const WLS& c, int idx) {
-      if (fabsf(c.d0) < gtol && (best < 0 || c.cost < bcost)) {
-        bcost = c.cost;
-        best = idx;
-        balpha = c.alpha;
-      }
-    };
-    consider(c0, 0);
-    consider(c1, 1);
-    consider(c2, 2);
-    if (best >= 0) return balpha;
-    // p1, then p2, moves to the candidates whose slope has its sign and is closer to zero
-    auto narrow = [&](WLS& p) {
-      int flag = 0;
-      auto step = [&](const WLS& c) {
-        if (p.d0 < 0.f && c.d0 < 0.f && p.d0 < c.d0) { p = c; flag = 1; }
-        else if (p.d0 > 0.f && c.d0 > 0.f && p.d0 > c.d0) { p = c; flag = 2; }
-      };
-      step(c0);
-      step(c1);
-      step(c2);
-      return flag;
-    };
-    const int f1 = narrow(p1);
-    p1n = p1;
-    if (f1 > 0) p1n = wave_ls_point(w, rc, qg0, qg1, qg2, p1.alpha - p1.d0 / p1.d1, ls_it);
-    const int f2 = narrow(p2);
-    p2n = p2;
-    if (f2 > 0) p2n = wave_ls_point(w, rc, qg0, qg1, qg2, p2.alpha - p2.d0 / p2.d1, ls_it);
-    if (f1 == 0 && f2 == 0) return pm.alpha;
-  }
-  if (p1.cost <= p2.cost && p1.cost < p0.cost) return p1.alpha;
-  if (p2.cost <= p1.cost && p2.cost < p1.cost) return p2.alpha;
-  return 0.f;
+  return linesearch_points(m, gtol, [&](float alpha, int& ls_it) { return wave_ls_point(w, rc, qg0, qg1, qg2, alpha, ls_it); });
 }
 
 // Above this many activity changes in one Newton iteration the factor is rebuilt instead of updated row by row.
 constexpr int kMaxRank1PerIter = 8;
 
-// Newton iterations (func_solve / func_solve_body) from the initial factorisation on; returns the iteration count
+// Newton iterations (func_solve / func_solve_body) from the first factorisation on; returns the iteration count. The
+// stop test needs the gradient only, so the last iteration neither updates the factor nor solves with it.
 template <class HS>
 __device__ __forceinline__ int wave_newton(const WaveCtx& w, const HS& h, double cost, float gauss) {
   const Env& e = w.e;
@@ -1699,114 +1472,103 @@ __device__ __forceinline__ int wave_newton(const WaveCtx& w, const HS& h, double
   const gsr_state& s = e.s;
   const WaveLds& L = w.L;
   const int lane = w.lane, D = w.D, n_con = w.n_con;
-  wave_hessian_direct(w, h);
-  wave_update_gradient(w, h);
-  for (int d = lane; d < D; d += kWave) L.search[d] = -L.vec[L.pdof[d]];
-  __syncthreads();
+  const float tol_scaled = (e.meaninertia() * (float)(D > 1 ? D : 1)) * m.tolerance;
   int iters = 0;
-  if (n_con <= 0) return 0;
-  for (int it = 0; it < m.iterations; it++) {
+  bool build = true;
+  while (iters < m.iterations) {
+    if (build) wave_hessian_direct(w, h);
+    wave_gradient<true>(w);
+    wave_chol_solve(w, h, L.vec);
+    for (int d = lane; d < D; d += kWave) L.search[d] = -L.vec[L.pdof[d]];
+    __syncthreads();
     iters++;
-    float alpha = wave_linesearch(w, gauss);
-    bool improved;
-    if (fabsf(alpha) < m.eps) {
-      improved = false;
-    } else {
-      for (int d = lane; d < D; d += kWave) {
-        L.qacc[d] = L.qacc[d] + L.search[d] * alpha;
-        L.Ma[d] = L.Ma[d] + L.mv[d] * alpha;
-      }
-      for (int c = lane; c < n_con; c += kWave) e.EF(s.efc_Jaref, c) = e.EF(s.efc_Jaref, c) + e.EF(s.efc_jv, c) * alpha;
-      __syncthreads();
-      double prev_cost = cost;
-      wave_update_constraint(w, cost, gauss);
-      // activity changes in row order; rank-1 updates or a rebuild of the factor
-      int n_changed = 0;
-      for (int c = lane; c < n_con; c += kWave) {
-        int a = e.EI(s.efc_active, c);
-        n_changed += ((a & 1) != ((a >> 1) & 1));
-      }
-      for (int o = kWave / 2; o > 0; o >>= 1) n_changed += __shfl_xor(n_changed, o, kWave);
-      if (n_changed > kMaxRank1PerIter) {
-        wave_hessian_direct(w, h);
-      } else if (n_changed > 0) {
-        bool rebuilt = false;
-        for (int c0 = 0; c0 < n_con && !rebuilt; c0 += kWave) {
-          int c = c0 + lane;
-          int a = c < n_con ? e.EI(s.efc_active, c) : 0;
-          unsigned long long chg = __ballot((a & 1) != ((a >> 1) & 1));
-          while (chg && !rebuilt) {
-            int j = __ffsll((long long)chg) - 1;
-            chg &= chg - 1;
-            int aj = __shfl(a, j, kWave);
-            const float sgn = (aj & 1) ? 1.f : -1.f;
-            if (!((!HS::kFence && w.dense_h) ? wave_rank1_dense(w, c0 + j, sgn) : wave_rank1(w, h, c0 + j, sgn))) {
-              wave_hessian_direct(w, h);
-              rebuilt = true;
-            }
-          }
-        }
-      }
-      double g2 = wave_update_gradient(w, h);
-      float tol_scaled = (w.e.meaninertia() * (float)(D > 1 ? D : 1)) * m.tolerance;
-      double improvement = prev_cost - cost;
-      float gn = sqrtf((float)wave_sum_d(g2));
-      if (gn < tol_scaled || improvement < tol_scaled) {
-        improved = false;
-      } else {
-        improved = true;
-        for (int d = lane; d < D; d += kWave) L.search[d] = -L.vec[L.pdof[d]];
-      }
-      __syncthreads();
+    const float alpha = wave_linesearch(w, gauss);
+    if (fabsf(alpha) < m.eps) break;
+    for (int d = lane; d < D; d += kWave) {
+      L.qacc[d] = L.qacc[d] + L.search[d] * alpha;
+      L.Ma[d] = L.Ma[d] + L.mv[d] * alpha;
     }
-    if (!improved) break;
+    for (int c = lane; c < n_con; c += kWave) e.EF(s.efc_Jaref, c) = e.EF(s.efc_Jaref, c) + e.EF(s.efc_jv, c) * alpha;
+    __syncthreads();
+    const double prev_cost = cost;
+    wave_update_constraint(w, cost, gauss);
+    const double improvement = prev_cost - cost;
+    const float gn = sqrtf((float)wave_sum_d(wave_gradient<false>(w)));
+    if (gn < tol_scaled || improvement < tol_scaled) break;
+    __syncthreads();
+    // activity changes in row order; rank-1 updates or a rebuild of the factor
+    int n_changed = 0;
+    for (int c = lane; c < n_con; c += kWave) {
+      int a = e.EI(s.efc_active, c);
+      n_changed += ((a & 1) != ((a >> 1) & 1));
+    }
+    n_changed = wave_sum_i(n_changed);
+    build = n_changed > kMaxRank1PerIter;
+    for (int c0 = 0; c0 < n_con && n_changed > 0 && !build; c0 += kWave) {
+      int c = c0 + lane;
+      int a = c < n_con ? e.EI(s.efc_active, c) : 0;
+      unsigned long long chg = __ballot((a & 1) != ((a >> 1) & 1));
+      while (chg && !build) {
+        int j = __ffsll((long long)chg) - 1;
+        chg &= chg - 1;
+        build = !wave_rank1(w, h, c0 + j, (lane_value(a, j) & 1) ? 1.f : -1.f);
+      }
+    }
   }
   return iters;
 }
 
-__device__ __forceinline__ void wave_solve(const Env& e, char* lds) {
+// contact forces from the pyramid rows' forces (func_update_contact_force), contacts first, first + stride, ...
+__device__ __forceinline__ void contact_forces(const Env& e, int first, int stride) {
+  const gsr_model& m = e.m;
+  const gsr_state& s = e.s;
+  const int cs = e.I(s.n_con, 1) + e.I(s.n_con, 2);
+  const int nc = m.enable_collision ? e.I(s.n_contacts, 0) : 0;
+  for (int ic = first; ic < nc; ic += stride) {
+    f3 cn = e.L3(s.contact_normal, ic);
+    float fr = e.F(s.contact_friction, ic);
+    f3 d1, d2;
+    orthogonals(cn, d1, d2);
+    f3 f = zero3();
+    for (int i = 0; i < 4; i++) {
+      f3 dd = (float)(2 * (i % 2) - 1) * (i < 2 ? d1 : d2);
+      f3 n = dd * fr - cn;
+      f = f + n * e.EF(s.efc_force, ic * 4 + i + cs);
+    }
+    e.S3(s.contact_force, ic, f);
+  }
+}
+
+__device__ __forceinline__ void wave_solve_blocks(const Env& e, char* lds) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
   const int lane = threadIdx.x;
   const int D = m.n_dofs, E = m.n_entities;
   WaveLds L = wave_lds_carve((lds_c*)lds, D, E, m.wave_h_floats);
   int n_con = e.I(s.n_con, 0), ne = e.I(s.n_con, 1), nef = ne + e.I(s.n_con, 2);
-  // the dense row sums when one entity holds every dof (at most 64, with H in LDS and room after it for 8 or more
-  // staged rows)
-  bool dense_h = false;
-  int dense_rows = 0;
-  lds_f* dense_buf = nullptr;
-  {
-    int n_ent = 0;
-    for (int i = 0; i < E; i++) n_ent += m.ent_dof_end[i] > m.ent_dof_start[i] ? 1 : 0;
-    const int tri = D * (D + 1) / 2, tri4 = (tri + 3) & ~3;
-    dense_h = n_ent == 1 && D <= kWave && tri <= m.wave_h_floats;
-    if (dense_h && tri4 < m.wave_h_floats) {
-      const int R = min(kWave, (m.wave_h_floats - tri4) / (D + 1));
-      if (R >= 8) {
-        dense_rows = R;
-        dense_buf = L.hl + tri4;
-      }
-    }
-  }
-  WaveCtx w{e, L, lane, D, E, n_con, ne, nef, dense_h, dense_rows, dense_buf};
+  WaveCtx w{e, L, lane, D, E, n_con, ne, nef};
   int ws = e.I(s.is_warmstart, 0);
   // force (the smooth force until the epilogue) and acc_smooth are read from the state: nothing writes them here
   for (int d = lane; d < D; d += kWave) L.qacc[d] = (n_con > 0 && ws) ? e.F(s.qacc_ws, d) : e.F(s.acc_smooth, d);
   __syncthreads();
-  wave_build_structure(w);
-  wave_mass_mul(w, L.qacc, L.Ma);
-  for (int c = lane; c < n_con; c += kWave) {
-    float ja = -e.EF(s.efc_aref, c);
-    int nnz = e.EI(s.jac_nnz, c);
-    ja = row_dot_vec(e, c, nnz, ja, L.qacc);
-    e.EF(s.efc_Jaref, c) = ja;
+  int iters = 0;
+  if (n_con > 0) {
+    wave_build_structure(w);
+    wave_mass_mul(w, L.qacc, L.Ma);
+    for (int c = lane; c < n_con; c += kWave) {
+      float ja = -e.EF(s.efc_aref, c);
+      int nnz = e.EI(s.jac_nnz, c);
+      ja = row_dot_vec(e, c, nnz, ja, L.qacc);
+      e.EF(s.efc_Jaref, c) = ja;
+    }
+    __syncthreads();
+    double cost;
+    float gauss;
+    wave_update_constraint(w, cost, gauss);
+    iters = L.hmode[0] ? wave_newton(w, HLds{L}, cost, gauss) : wave_newton(w, HGlobal{e, L.es}, cost, gauss);
+  } else {
+    for (int d = lane; d < D; d += kWave) L.qfrc[d] = 0.f;
   }
-  __syncthreads();
-  double cost;
-  float gauss;
-  wave_update_constraint(w, cost, gauss);
-  int iters = L.hmode[0] ? wave_newton(w, HLds{L}, cost, gauss) : wave_newton(w, HGlobal{e, L.es}, cost, gauss);
   // epilogue (func_update_qacc, func_update_contact_force)
   int bad = 0;
   for (int d = lane; d < D; d += kWave) {
@@ -1822,21 +1584,7 @@ __device__ __forceinline__ void wave_solve(const Env& e, char* lds) {
     e.I(s.is_warmstart, 0) = 1;
     if (bad) e.I((int32_t*)s.errno_env, 0) |= (int)GSR_ERR_NAN_QACC;
   }
-  int cs = ne + e.I(s.n_con, 2);
-  int nc = m.enable_collision ? e.I(s.n_contacts, 0) : 0;
-  for (int ic = lane; ic < nc; ic += kWave) {
-    f3 cn = e.L3(s.contact_normal, ic);
-    float fr = e.F(s.contact_friction, ic);
-    f3 d1, d2;
-    orthogonals(cn, d1, d2);
-    f3 f = zero3();
-    for (int i = 0; i < 4; i++) {
-      f3 dd = (float)(2 * (i % 2) - 1) * (i < 2 ? d1 : d2);
-      f3 n = dd * fr - cn;
-      f = f + n * e.EF(s.efc_force, ic * 4 + i + cs);
-    }
-    e.S3(s.contact_force, ic, f);
-  }
+  contact_forces(e, lane, kWave);
 }
 
 }  // namespace gsr

@@ -10,6 +10,7 @@
 #include "rigid_collide.h"
 #include "rigid_solver.h"
 #include "rigid_solver_wave.h"
+#include "rigid_solver_dense.h"
 #include "rigid_collide_wave.h"
 
 namespace gsr {

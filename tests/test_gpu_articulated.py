@@ -1,0 +1,73 @@
+"""Articulated models at the sizes where the wavefront kernels change form: the single-entity Newton solver (one lane
+per dof up to 64 dofs, rows staged 64 at a time) against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from genesis_amd import workloads as W
+from genesis_amd.model import (CompileOptions, EntitySpec, JOINT_FREE, JOINT_PRISMATIC, JOINT_REVOLUTE, JointSpec,
+                               LinkSpec, compile_model)
+from tests.sync import gpu_to_oracle
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-4
+
+
+def chain_entity(n, free_base=False):
+    """Chains of up to 12 one-dof links on a fixed or a floating base, n links in all (every fifth prismatic), with
+    frictionloss on every joint and limits of +-0.05 on each fourth."""
+    rng = np.random.default_rng(n)
+    base_joint = JointSpec("base", JOINT_FREE, kp=0.0, kv=0.0, init_qpos=np.array([0, 0, 1.0, 1, 0, 0, 0])) if free_base \
+        else JointSpec("base", 0)
+    links = [LinkSpec("base", -1, np.array([0, 0, 1.0]), np.array([1.0, 0, 0, 0]), [base_joint], [], np.zeros(3),
+                      np.array([1.0, 0, 0, 0]), np.eye(3) * 0.05, 4.0)]
+    for i in range(n):
+        axis = np.eye(3)[i % 3]
+        limit = np.array([[-0.05, 0.05]]) if i % 4 == 0 else np.array([[-np.inf, np.inf]])
+        j = JointSpec(f"j{i}", JOINT_PRISMATIC if i % 5 == 4 else JOINT_REVOLUTE, axis=axis, limit=limit, damping=0.1,
+                      armature=0.1, stiffness=0.2, frictionloss=0.05, kp=5.0, kv=0.5)
+        parent = 0 if i % 12 == 0 else i
+        links.append(LinkSpec(f"l{i}", parent, rng.uniform(-0.05, 0.05, 3), np.array([1.0, 0, 0, 0]), [j], [],
+                              rng.uniform(-0.02, 0.02, 3), np.array([1.0, 0, 0, 0]), np.diag(rng.uniform(0.5, 1, 3) * 1e-2),
+                              rng.uniform(0.3, 1.0)))
+    return EntitySpec(links, name="chain")
+
+
+def start(S, M, B, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = torch.as_tensor(np.tile(M.qpos0, (B, 1)), dtype=torch.float32)
+    first = 7 if M.n_qs > M.n_dofs else 0  # the floating base stays where it is
+    q[:, first:] += 0.3 * (torch.rand((B, M.n_qs - first), generator=g) - 0.5)
+    S.set_qpos(q)
+    S.set_dofs_velocity(torch.rand((B, M.n_dofs), generator=g) - 0.5)
+    S.control_dofs_position(0.2 * (torch.rand((B, M.n_dofs), generator=g) - 0.5))
+
+
+@pytest.mark.parametrize("n,free_base", [(7, False), (17, True), (33, False), (64, False), (65, False)])
+def test_single_entity_solver_matches_oracle(n, free_base):
+    """64 dofs is the last size with a lane per dof; its frictionloss and limit rows exceed the 64 staged at once. Each step starts the oracles from the HIP state; bound as in the other wavefront parity tests: 1e-4, or 4x
+    the largest FP32-vs-FP64 spread of the oracle in that env."""
+    from genesis_amd.rigid_solver import RigidSolver
+    from oracle.oracle import Oracle
+    M = compile_model([chain_entity(n, free_base)], CompileOptions(dt=0.005, enable_collision=False))
+    B = 6
+    S = RigidSolver(M, B, "cuda", solver_variant=1, wave_h_floats=4096)
+    start(S, M, B, n)
+    O, O64 = Oracle(M, B, 32), Oracle(M, B, 64)
+    most = 0
+    for step in range(4):
+        torch.cuda.synchronize()
+        gpu_to_oracle(S, O)
+        gpu_to_oracle(S, O64)
+        S.substep()
+        O.run(1)
+        O64.run(1)
+        torch.cuda.synchronize()
+        most = max(most, int(S.st.t["n_con"][0].max()))
+        for name in ("qpos", "vel"):
+            got, o, o64 = S.st.t[name].T.cpu().numpy(), O.get(name), O64.get(name)
+            for b in range(B):
+                bound = np.maximum(TOL + TOL * np.abs(o[b]), 4 * np.abs(o[b] - o64[b]).max() + TOL)
+                assert (np.abs(got[b] - o[b]) <= bound).all(), f"step {step} env {b} {name}"
+    assert most > (64 if n == 64 else 0), most
