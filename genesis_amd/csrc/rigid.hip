@@ -43,20 +43,60 @@ __global__ void __launch_bounds__(kBlock) k_step1(gsr_model m, gsr_state s, int 
 }
 
 
+// G lanes per env: the lanes share an articulated env's tree ...
+template <int G>
+__global__ void __launch_bounds__(kWave) k_step1_tree(gsr_model m, gsr_state s) {
+  extern __shared__ char lds[];
+  const TreeTables t = tree_tables<true>(m, lds);
+  int b;
+  lds_f* p;
+  if (!tree_env<G>(m, blockIdx.x, s.n_envs, lds, b, p)) return;
+  tree_step1<G>(Env(m, s, b), t, p);
+}
+
+template <int G>
+__global__ void __launch_bounds__(kWave) k_step2_tree(gsr_model m, gsr_state s) {
+  extern __shared__ char lds[];
+  const TreeTables t = tree_tables<false>(m, lds);
+  int b;
+  lds_f* p;
+  if (!tree_env<G>(m, blockIdx.x, s.n_envs, lds, b, p)) return;
+  tree_step2<G>(Env(m, s, b), t, p);
+}
+
+template <int G>
+__global__ void __launch_bounds__(kWave) k_kinematics_tree(gsr_model m, gsr_state s, const int32_t* envs_idx, int n_idx) {
+  extern __shared__ char lds[];
+  const TreeTables t = tree_tables<false>(m, lds);
+  int k;
+  lds_f* p;
+  if (!tree_env<G>(m, blockIdx.x, n_idx, lds, k, p)) return;
+  const int b = envs_idx ? envs_idx[k] : k;
+  if (b < 0 || b >= s.n_envs) return;
+  Env e(m, s, b);
+  tree_refresh<G>(e, t, p);
+  __syncthreads();
+  if (m.enable_collision) wave_update_aabbs<G>(e, threadIdx.x & (G - 1));
+}
+
+template <class K16, class K64, class... Args>
+void launch_tree(K16 k16, K64 k64, const gsr_model& m, int n, hipStream_t st, Args... args) {
+  const int G = tree_lanes(m, n), per = kWave / G;
+  const dim3 grid((n + per - 1) / per);
+  if (G == 16) hipLaunchKernelGGL(k16, grid, dim3(kWave), tree_lds_bytes(m, 16), st, args...);
+  else hipLaunchKernelGGL(k64, grid, dim3(kWave), tree_lds_bytes(m, kWave), st, args...);
+}
+
+// ... and take the entities of an env of free bodies
 __global__ void __launch_bounds__(kWave) k_step1_wave(gsr_model m, gsr_state s) {
   if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
-  const int b = xcd_env(blockIdx.x, s.n_envs);
-  Env e(m, s, b);
-  wave_step1(e);
+  dev_smooth_dynamics(Env(m, s, xcd_env(blockIdx.x, s.n_envs)), threadIdx.x, kWave);
 }
 
 __global__ void __launch_bounds__(kWave) k_step2_wave(gsr_model m, gsr_state s) {
   if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
-  const int b = xcd_env(blockIdx.x, s.n_envs);
-  Env e(m, s, b);
-  wave_step2(e);
+  wave_step2_entities(Env(m, s, xcd_env(blockIdx.x, s.n_envs)));
 }
-
 
 __global__ void __launch_bounds__(kBlock) k_step2(gsr_model m, gsr_state s) {
   int b = env_id();
@@ -208,13 +248,22 @@ int launch_status() {
 
 inline dim3 grid_for(int n) { return dim3((n + kBlock - 1) / kBlock); }
 
+// kinematics of n listed envs (all when idx is null); an articulated env takes a wavefront whatever the step's variant
+void launch_kinematics(const gsr_model& m, const gsr_state& s, const int32_t* idx, int n, hipStream_t st) {
+  if (tree_dynamics(m))
+    launch_tree(k_kinematics_tree<16>, k_kinematics_tree<kWave>, m, n, st, m, s, idx, n);
+  else
+    hipLaunchKernelGGL(k_kinematics, grid_for(n), dim3(kBlock), 0, st, m, s, idx, n);
+}
+
 void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
   dim3 g = grid_for(s->n_envs);
   switch (k) {
     // kinematics of the current pose are refreshed at the end of every step (and by gsr_forward_kinematics after a
     // pose write), so kernel_step_1 never needs to recompute them (enable_mujoco_compatibility = False)
     case 0:
-      if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step1_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
+      if (dyn_lds_bytes(*m)) launch_tree(k_step1_tree<16>, k_step1_tree<kWave>, *m, s->n_envs, st, *m, *s);
+      else if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step1_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
       else hipLaunchKernelGGL(k_step1, g, dim3(kBlock), 0, st, *m, *s, 0);
       break;
     case 1:
@@ -224,7 +273,8 @@ void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
       launch_solve(*m, *s, st);
       break;
     default:
-      if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step2_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
+      if (dyn_lds_bytes(*m)) launch_tree(k_step2_tree<16>, k_step2_tree<kWave>, *m, s->n_envs, st, *m, *s);
+      else if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step2_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
       else hipLaunchKernelGGL(k_step2, g, dim3(kBlock), 0, st, *m, *s);
       break;
   }
@@ -381,7 +431,7 @@ int gsr_forward_kinematics(const gsr_model* model, const gsr_state* state, const
   if (rc) return rc;
   int n = envs_idx ? n_idx : state->n_envs;
   if (n <= 0) return GSR_OK;
-  hipLaunchKernelGGL(k_kinematics, grid_for(n), dim3(kBlock), 0, stream, *model, *state, envs_idx, n);
+  launch_kinematics(*model, *state, envs_idx, n, stream);
   return launch_status();
 }
 
@@ -449,9 +499,8 @@ int gsr_launch_kernel(const gsr_model* model, const gsr_state* state, int32_t ke
 int gsr_run_stage(const gsr_model* model, const gsr_state* state, int32_t stage, hipStream_t stream) {
   int rc = check(model, state);
   if (rc) return rc;
-  dim3 g = grid_for(state->n_envs);
   if (stage == 0) return run_substep(model, state, stream);
-  hipLaunchKernelGGL(k_kinematics, g, dim3(kBlock), 0, stream, *model, *state, (const int32_t*)nullptr, state->n_envs);
+  launch_kinematics(*model, *state, nullptr, state->n_envs, stream);
   if (stage >= 2) launch_one(model, state, 0, stream);
   if (stage >= 3) launch_one(model, state, 1, stream);
   return launch_status();
@@ -462,19 +511,22 @@ int64_t gsr_batch_table_bytes(int32_t n_groups) {
   return (int64_t)(kRangesOffset + sizeof(BatchRange) * (size_t)n_groups);
 }
 
-// dynamic LDS of phase 1 (wavefront collision) or 3 (wavefront solver): the largest over the batch's scene types
+// dynamic LDS of phase 0 or 4 (dynamics), 1 (wavefront collision) or 3 (wavefront solver): the largest over the batch's
+// scene types
 static int phase_lds(const gsr_batch_info& b, int phase) {
   size_t lds = 0;
   for (int k = 0; k < b.n_types; k++) {
     const gsr_model& m = b.models[k];
     if (phase == 1 && m.collide_variant == 1) lds = std::max(lds, (size_t)wave_collide_lds_bytes(m.n_geoms));
+    // room for tiles of several envs: a group's tile size is not known here
+    if (phase == 0 || phase == 4) lds = std::max(lds, dyn_lds_bytes(m, kWave));
     if (phase == 3 && m.solver_variant == 1)
       lds = std::max(lds, (size_t)solve_lds_bytes(m));
   }
   return (int)lds;
 }
 
-static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, size_t lds,
+static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int dyn_tiles, size_t lds,
                               gsr_batch_info* info);
 
 int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table, int64_t table_bytes,
@@ -484,7 +536,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
   std::vector<BatchRange> ranges(n_groups);
   gsr_batch_info out;
   std::memset(&out, 0, sizeof(out));
-  int tiles = 0, wtiles = 0;
+  int tiles = 0, wtiles = 0, dtiles = 0;
   size_t lds = 0;
   for (int g = 0; g < n_groups; g++) {
     const gsr_group& G = groups[g];
@@ -508,9 +560,13 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
     if (G.model.solver_variant == 1)
       lds = std::max(lds, solve_lds_bytes(G.model));
     if (G.model.collide_variant == 1) lds = std::max(lds, wave_collide_lds_bytes(G.model.n_geoms));
+    lds = std::max(lds, dyn_lds_bytes(G.model, G.envs_per_tile));
+    const int Td = dyn_tile_envs(G.model, G.n_envs, G.envs_per_tile);
     const int n_t = (G.n_envs + G.envs_per_tile - 1) / G.envs_per_tile, n_w = (G.n_envs + Tw - 1) / Tw;
+    const int n_d = (G.n_envs + Td - 1) / Td;
     ranges[g] = BatchRange{type, G.env_begin, G.n_envs, G.envs_per_tile, tiles, tiles + n_t, Tw, wtiles, wtiles + n_w,
-                           0, 0, 0};
+                           Td, dtiles, dtiles + n_d};
+    dtiles += n_d;
     tiles += n_t;
     wtiles += n_w;
   }
@@ -533,7 +589,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
       if (B.env_begin < A.env_begin + A.n_envs) return GSR_E_ARG;
     }
   }
-  BatchHeader h{n_groups, tiles, 0u, 0u, wtiles, 0, 0, 0};
+  BatchHeader h{n_groups, tiles, 0u, 0u, wtiles, dtiles, 0, 0};
   FusedTypes ty;
   std::memset(&ty, 0, sizeof(ty));
   for (int k = 0; k < out.n_types; k++) {
@@ -547,21 +603,24 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
   if (hipMemcpy(static_cast<char*>(dev_table) + kTypesOffset, &ty, sizeof(ty), hipMemcpyHostToDevice) != hipSuccess)
     return GSR_E_LAUNCH;
   if (hipMemcpy(dev_table, &h, 2 * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(static_cast<char*>(dev_table) + offsetof(BatchHeader, n_wave_tiles), &h.n_wave_tiles, sizeof(int32_t),
-                hipMemcpyHostToDevice) != hipSuccess)
+      hipMemcpy(static_cast<char*>(dev_table) + offsetof(BatchHeader, n_wave_tiles), &h.n_wave_tiles,
+                2 * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess)
     return GSR_E_LAUNCH;
-  return finish_launch_info(out, n_groups, tiles, wtiles, lds, info);
+  return finish_launch_info(out, n_groups, tiles, wtiles, dtiles, lds, info);
 }
 
 // Launch form of a batch whose types are in `out`: kernel attributes (dynamic LDS), grid and the form's flags, read
 // from `info` and written back to it.
-static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, size_t lds,
+static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int dyn_tiles, size_t lds,
                               gsr_batch_info* info) {
   int dev = 0, n_cu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return GSR_E_LAUNCH;
   if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return GSR_E_LAUNCH;
   if (info->phased) {
-    const int lc = phase_lds(out, 1), ls = phase_lds(out, 3);
+    const int lc = phase_lds(out, 1), ls = phase_lds(out, 3), ld = phase_lds(out, 0);
+    for (int k = 0; k <= 4; k += 4)
+      if (ld > 0 && hipFuncSetAttribute(phase_kernel(k), hipFuncAttributeMaxDynamicSharedMemorySize, ld) != hipSuccess)
+        return GSR_E_LAUNCH;
     if (lc > 0 && hipFuncSetAttribute(phase_kernel(1), hipFuncAttributeMaxDynamicSharedMemorySize, lc) !=
                       hipSuccess)
       return GSR_E_LAUNCH;
@@ -575,7 +634,7 @@ static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int 
     out.waves_per_simd = 0;
     out.gjk_inline = 0;
     out.phased = 1;
-    out.grid = tiles;
+    out.grid = dyn_tiles;
     out.lds_bytes = (int32_t)lds;
     *info = out;
     return GSR_OK;
@@ -616,8 +675,9 @@ int gsr_launch_fused_kernel(const void* dev_table, const gsr_batch_info* info, i
   if (k < 0 || k >= n) return GSR_E_ARG;
   const char* t = static_cast<const char*>(dev_table);
   if (info->phased) {
-    const int lds = k == 1 ? phase_lds(*info, 1) : k == 3 ? phase_lds(*info, 3) : 0;
-    launch_phase(k, dim3(k == 2 || k == 3 ? info->n_wave_tiles : info->n_tiles), lds, stream, t);
+    const int lds = k == 2 ? 0 : phase_lds(*info, k);
+    const int tiles = k == 2 || k == 3 ? info->n_wave_tiles : k == 1 ? info->n_tiles : info->grid;
+    launch_phase(k, dim3(tiles), lds, stream, t);
   } else if (k == 0) {
     uint32_t* queue = reinterpret_cast<uint32_t*>(const_cast<char*>(t) + 2 * sizeof(int32_t));
     launch_fused(info->waves_per_simd == 4 ? 4 : 2, info->gjk_inline ? 1 : 0, dim3(info->grid), info->lds_bytes,
@@ -625,7 +685,7 @@ int gsr_launch_fused_kernel(const void* dev_table, const gsr_batch_info* info, i
   } else {
     const gsr_model& m = info->models[k - 1];
     const gsr_state& st = info->states[k - 1];
-    const size_t lds = m.solver_variant == 1 ? solve_lds_bytes(m) : 0;
+    const size_t lds = std::max(m.solver_variant == 1 ? solve_lds_bytes(m) : 0, dyn_lds_bytes(m));
     launch_gjk_resume(m, st, (unsigned)lds, stream);
   }
   return launch_status();
@@ -732,6 +792,7 @@ int gsr_serve_init(const gsr_serve_pool* pools, int32_t n_pools, double mem_budg
     if (P.model.solver_variant == 1)
       lds = std::max(lds, solve_lds_bytes(P.model));
     if (P.model.collide_variant == 1) lds = std::max(lds, wave_collide_lds_bytes(P.model.n_geoms));
+    lds = std::max(lds, dyn_lds_bytes(P.model, P.envs_per_tile));
     tiles += P.n_tiles;
   }
   out.n_types = n_pools;
@@ -741,7 +802,7 @@ int gsr_serve_init(const gsr_serve_pool* pools, int32_t n_pools, double mem_budg
                             stream);
   if (rc) return rc;
   // every tile may be active: the launches cover all of them (idle ones return at once)
-  return finish_launch_info(out, tiles, tiles, tiles, lds, info);
+  return finish_launch_info(out, tiles, tiles, tiles, tiles, lds, info);
 }
 
 int gsr_serve_tick(void* dev_state, void* dev_table, const gsr_batch_info* info, gsr_serve_host* host,

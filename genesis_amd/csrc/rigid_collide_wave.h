@@ -34,10 +34,11 @@ __host__ __device__ inline size_t wave_collide_lds_bytes(int G) {
   return sizeof(float) * 4 * (size_t)G + sizeof(int) * 6 * (size_t)G + 64;
 }
 
+template <int G = 64>
 __device__ inline void wave_update_aabbs(const Env& e, int lane) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  for (int g = lane; g < m.n_geoms; g += 64) {
+  for (int g = lane; g < m.n_geoms; g += G) {
     f3 gp = e.L3(s.geoms_pos, g);
     q4 gq = e.L4(s.geoms_quat, g);
     f3 lo{INFINITY, INFINITY, INFINITY}, hi{-INFINITY, -INFINITY, -INFINITY};

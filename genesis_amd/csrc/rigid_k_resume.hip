@@ -19,7 +19,7 @@ k_gjk_resume(gsr_model m, gsr_state s) {
   else if (threadIdx.x == 0) dev_solve(e);
   __syncthreads();
   if (m.dyn_variant == 1) {
-    wave_step2(e);
+    wave_step2<false>(m, s, b, 1, lds);
   } else if (threadIdx.x == 0) {
     dev_integrate(e);
     dev_kinematics(e);

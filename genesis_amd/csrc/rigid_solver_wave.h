@@ -17,13 +17,6 @@
 
 namespace gsr {
 
-// LDS pointers carry their address space so every access compiles to ds_* instructions (not flat), and the compiler
-// knows they never alias global memory.
-#define GSR_LDS __attribute__((address_space(3)))
-typedef GSR_LDS float lds_f;
-typedef GSR_LDS int lds_i;
-typedef GSR_LDS unsigned long long lds_u64;
-typedef GSR_LDS char lds_c;
 constexpr int kMaxPatternEntities = 128;  // two 64-bit words per entity row of the pattern
 
 // A constraint row of up to kStage entries (every row of the arm, quadruped and box scenes) is loaded into

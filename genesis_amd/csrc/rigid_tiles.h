@@ -7,6 +7,7 @@
 
 #include "genesis_rigid.h"
 #include "rigid_kin.h"
+#include "rigid_kin_wave.h"
 #include "rigid_collide.h"
 #include "rigid_solver.h"
 #include "rigid_solver_wave.h"
@@ -19,25 +20,31 @@ constexpr int kBlock = 64;
 
 __device__ __forceinline__ int env_id() { return blockIdx.x * blockDim.x + threadIdx.x; }
 
-// Workgroup -> env for the one-env-per-workgroup kernels. The dispatcher deals workgroups to the 8 XCDs round-robin
-// (workgroup i to XCD i % 8) and every XCD has its own L2, while the env-minor state arrays put 32 neighbouring envs
-// in one 128-byte line. Within each chunk of 256 workgroups, XCD x therefore gets a run of 32 consecutive envs, so
-// the waves it holds at once share their lines in its L2 instead of each XCD fetching every line. A bijection on
-// [0, n): a partial last chunk is split the same way over its m workgroups.
-__device__ __forceinline__ int xcd_env(int blk, int n) {
-  constexpr int kRun = 32, kChunk = 8 * kRun;
-  const int base = blk - blk % kChunk;
-  const int m = min(kChunk, n - base);
-  const int j = blk - base;
-  const int q = m >> 3, r = m & 7, x = j & 7, k = j >> 3;
-  return base + x * q + min(x, r) + k;
+// step_1 / step_2 of envs [b0, b0 + n) on one wavefront: articulated models spread their tree over the lanes
+// (rigid_kin_wave.h), four envs at a time where there are several; of free bodies each lane takes whole entities (no
+// entity reads another's state) env after env, and only the geom poses, split by geom index, need the link poses of
+// every lane, hence the barrier.
+__device__ __forceinline__ bool tree_packed(const gsr_model& m, int n) {
+  return n > 1 && tree_lds_bytes(m, 16) <= kTreeMaxLds;
+}
+__device__ __forceinline__ void wave_step1(const gsr_model& m, const gsr_state& s, int b0, int n, char* lds) {
+  if (!tree_dynamics(m)) {
+    for (int j = 0; j < n; j++) dev_smooth_dynamics(Env(m, s, b0 + j), threadIdx.x, kWave);
+    return;
+  }
+  const TreeTables t = tree_tables<true>(m, lds);
+  const int sub = threadIdx.x / 16;
+  if (tree_packed(m, n)) {
+    for (int j = 0; j < n; j += 4) {
+      if (j + sub < n) tree_step1<16>(Env(m, s, b0 + j + sub), t, tree_words(m, lds, sub));
+      __syncthreads();
+    }
+  } else {
+    for (int j = 0; j < n; j++) tree_step1<kWave>(Env(m, s, b0 + j), t, tree_words(m, lds, 0));
+  }
 }
 
-// step_1 / step_2 of one env on one wavefront: the env's entities are spread over the lanes (no entity reads another's
-// state); only the geom poses, split by geom index, need the link poses of every lane, hence the barrier.
-__device__ __forceinline__ void wave_step1(const Env& e) { dev_smooth_dynamics(e, threadIdx.x, kWave); }
-
-__device__ __forceinline__ void wave_step2(const Env& e) {
+__device__ __forceinline__ void wave_step2_entities(const Env& e) {
   const int lane = threadIdx.x;
   bool valid = dev_integrate_next(e, lane, kWave);
   valid = __all(valid);
@@ -48,6 +55,38 @@ __device__ __forceinline__ void wave_step2(const Env& e) {
   dev_update_geoms(e, lane, kWave);
   dev_forward_velocity(e, lane, kWave);
   __syncthreads();
+}
+// `pending`: skip envs that wait for the GJK/EPA pass
+template <bool pending>
+__device__ __forceinline__ void wave_step2(const gsr_model& m, const gsr_state& s, int b0, int n, char* lds) {
+  auto skip = [&](int b) { return pending && Env(m, s, b).I(s.gjk_defer_n, 0) > 0; };
+  if (!tree_dynamics(m)) {
+    for (int j = 0; j < n; j++)
+      if (!skip(b0 + j)) wave_step2_entities(Env(m, s, b0 + j));
+    return;
+  }
+  const TreeTables t = tree_tables<false>(m, lds);
+  const int sub = threadIdx.x / 16;
+  if (tree_packed(m, n)) {
+    for (int j = 0; j < n; j += 4) {
+      if (j + sub < n && !skip(b0 + j + sub)) tree_step2<16>(Env(m, s, b0 + j + sub), t, tree_words(m, lds, sub));
+      __syncthreads();
+    }
+  } else {
+    for (int j = 0; j < n; j++)
+      if (!skip(b0 + j)) tree_step2<kWave>(Env(m, s, b0 + j), t, tree_words(m, lds, 0));
+  }
+}
+// dynamic LDS of wave_step1 and wave_step2 over tiles of n envs
+__host__ __device__ inline size_t dyn_lds_bytes(const gsr_model& m, int n = 1) {
+  if (m.dyn_variant != 1 || !tree_dynamics(m)) return 0;
+  return tree_lds_bytes(m, n > 1 && tree_lds_bytes(m, 16) <= kTreeMaxLds ? 16 : kWave);
+}
+// envs per tile of the phased dynamics of a group of n envs: what a wavefront serves at once, or the group's own tiles
+// where a lane serves an env
+__host__ __device__ inline int dyn_tile_envs(const gsr_model& m, int n, int envs_per_tile) {
+  if (m.dyn_variant != 1) return envs_per_tile;
+  return tree_dynamics(m) ? kWave / tree_lanes(m, n) : 1;
 }
 
 // an env whose narrowphase deferred pairs to the GJK/EPA pass: its contact list and rows are completed there
@@ -61,14 +100,16 @@ struct BatchHeader {
   int32_t n_groups, n_tiles;
   uint32_t counter, done;  // work queue: next tile, finished workgroups (the last one resets both)
   int32_t n_wave_tiles;    // tiles of the phased launch's wavefront-per-env stages (GJK/EPA pass, solve)
-  int32_t pad0, pad1, pad2;
+  int32_t n_dyn_tiles;     // tiles of the phased launch's dynamics stages (step_1, step_2)
+  int32_t pad0, pad1;
 };
-// A group's envs cut into tiles twice: envs_per_tile for the single fused kernel and the phased per-env stages, and
+// A group's envs cut into tiles three times: envs_per_tile for the single fused kernel and the phased collision;
 // wave_envs_per_tile for the phased GJK/EPA pass and solve, whose wavefront variants take a tile's envs one after
-// the other (a lane-per-env collision wants 64 envs a tile, a wavefront solve few)
+// the other (a lane-per-env collision wants 64 envs a tile, a wavefront solve few); and dyn_envs_per_tile for the phased
+// dynamics, as many envs as their wavefront serves at once (dyn_tile_envs)
 struct BatchRange {
   int32_t type, env_begin, n_envs, envs_per_tile, tile_begin, tile_end;
-  int32_t wave_envs_per_tile, wave_tile_begin, wave_tile_end, pad0, pad1, pad2;
+  int32_t wave_envs_per_tile, wave_tile_begin, wave_tile_end, dyn_envs_per_tile, dyn_tile_begin, dyn_tile_end;
 };
 struct FusedTypes {
   gsr_model m[GSR_MAX_TYPES];
@@ -115,9 +156,10 @@ __device__ __forceinline__ void run_tile(const gsr_model& m, const gsr_state& s,
     }
   }
   __syncthreads();
+  if (dv) wave_step1(m, s, env0, n_here, lds);
+  __syncthreads();
   for (int j = 0; j < n_here; j++) {
     Env e(m, s, env0 + j);
-    if (dv) wave_step1(e);
     if (cw) wave_collide<kGjk>(e, lds);
     __syncthreads();
     if (sw && !gjk_pending(e)) wave_solve(e, lds);
@@ -135,10 +177,7 @@ __device__ __forceinline__ void run_tile(const gsr_model& m, const gsr_state& s,
   }
   if (dv) {
     __syncthreads();
-    for (int j = 0; j < n_here; j++) {
-      Env e(m, s, env0 + j);
-      if (!gjk_pending(e)) wave_step2(e);
-    }
+    wave_step2<true>(m, s, env0, n_here, lds);
   }
 }
 
@@ -192,13 +231,19 @@ __device__ __forceinline__ void phase_tile(const gsr_model& m, const gsr_state& 
     }
     return;
   }
+  if (P == 0) {
+    wave_step1(m, s, env0, n_here, lds);
+    return;
+  }
+  if (P == 4) {
+    wave_step2<false>(m, s, env0, n_here, lds);
+    return;
+  }
   for (int j = 0; j < n_here; j++) {
     Env e(m, s, env0 + j);
-    if (P == 0) wave_step1(e);
     if (P == 1) wave_collide(e, lds);
     if (P == 2 && wave_gjk_fixup(e)) wave_rows(e);
     if (P == 3) wave_solve(e, lds);
-    if (P == 4) wave_step2(e);
     __syncthreads();
   }
 }
@@ -210,19 +255,19 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 8
   const BatchHeader* __restrict__ H = reinterpret_cast<const BatchHeader*>(table);
   ConstTypes* types = (ConstTypes*)(table + kTypesOffset);
   const BatchRange* __restrict__ R = reinterpret_cast<const BatchRange*>(table + kRangesOffset);
-  constexpr bool kWaveTiles = P == 2 || P == 3;
-  const int n_tiles = kWaveTiles ? H->n_wave_tiles : H->n_tiles, n_groups = H->n_groups;
+  constexpr bool kWaveTiles = P == 2 || P == 3, kDynTiles = P == 0 || P == 4;
+  const int n_tiles = kWaveTiles ? H->n_wave_tiles : kDynTiles ? H->n_dyn_tiles : H->n_tiles, n_groups = H->n_groups;
   if ((int)blockIdx.x >= n_tiles) return;
   const int tile = xcd_env(blockIdx.x, n_tiles);
   int lo = 0, hi = n_groups - 1;
   while (lo < hi) {
     int mid = (lo + hi) >> 1;
-    if (tile < (kWaveTiles ? R[mid].wave_tile_end : R[mid].tile_end)) hi = mid;
+    if (tile < (kWaveTiles ? R[mid].wave_tile_end : kDynTiles ? R[mid].dyn_tile_end : R[mid].tile_end)) hi = mid;
     else lo = mid + 1;
   }
   const BatchRange g = R[lo];
-  const int T = kWaveTiles ? g.wave_envs_per_tile : g.envs_per_tile;
-  const int first = (tile - (kWaveTiles ? g.wave_tile_begin : g.tile_begin)) * T;
+  const int T = kWaveTiles ? g.wave_envs_per_tile : kDynTiles ? g.dyn_envs_per_tile : g.envs_per_tile;
+  const int first = (tile - (kWaveTiles ? g.wave_tile_begin : kDynTiles ? g.dyn_tile_begin : g.tile_begin)) * T;
   const int n_here = min(T, g.n_envs - first);
   const int k = __builtin_amdgcn_readfirstlane(g.type);
   const FusedTypes* ty = (const FusedTypes*)types;

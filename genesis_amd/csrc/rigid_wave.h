@@ -9,6 +9,28 @@ namespace gsr {
 
 constexpr int kWave = 64;
 
+// LDS pointers carry their address space so every access compiles to ds_* instructions (not flat), and the compiler
+// knows they never alias global memory.
+#define GSR_LDS __attribute__((address_space(3)))
+typedef GSR_LDS float lds_f;
+typedef GSR_LDS int lds_i;
+typedef GSR_LDS unsigned long long lds_u64;
+typedef GSR_LDS char lds_c;
+
+// Workgroup -> env for the one-env-per-workgroup kernels. The dispatcher deals workgroups to the 8 XCDs round-robin
+// (workgroup i to XCD i % 8) and every XCD has its own L2, while the env-minor state arrays put 32 neighbouring envs
+// in one 128-byte line. Within each chunk of 256 workgroups, XCD x therefore gets a run of 32 consecutive envs, so
+// the waves it holds at once share their lines in its L2 instead of each XCD fetching every line. A bijection on
+// [0, n): a partial last chunk is split the same way over its m workgroups.
+__device__ __forceinline__ int xcd_env(int blk, int n) {
+  constexpr int kRun = 32, kChunk = 8 * kRun;
+  const int base = blk - blk % kChunk;
+  const int m = min(kChunk, n - base);
+  const int j = blk - base;
+  const int q = m >> 3, r = m & 7, x = j & 7, k = j >> 3;
+  return base + x * q + min(x, r) + k;
+}
+
 // DPP control words: lane i of a row of 16 reads lane i + n (shl), i - n (shr), (i + n) mod 16 (ror by 16 - n)
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppShl4 = 0x104, kDppShr4 = 0x114, kDppRor4 = 0x124, kDppRor8 = 0x128;
 

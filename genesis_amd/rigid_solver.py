@@ -77,6 +77,14 @@ def default_stage_variant(M: RigidModel, n_envs: int = None) -> int:
     return 1 if (M.n_dofs >= 48 or (n_envs is not None and n_envs <= WAVE_MAX_SMALL_ENVS)) else 0
 
 
+def default_dyn_variant(M: RigidModel, n_envs: int = None) -> int:
+    """Variant of the dynamics stages: articulated models take a wavefront per env at every env count (the lanes share
+    the tree, four envs a wavefront where there are many; 32,768 quadrupeds: step_1 571 -> 232 us, step_2
+    190 -> 145 us, 64 arms: 172 -> 23 us and 92 -> 36 us), models of free bodies alone follow
+    default_stage_variant."""
+    return 1 if M.max_entity_dofs > 6 else default_stage_variant(M, n_envs)
+
+
 def default_collide_variant(M: RigidModel, n_envs: int = None) -> int:
     """As default_stage_variant, except that mesh geoms take the wavefront collision (support-field lookups diverge
     across a lane-per-env wavefront: the Panda's meshes collide 10x slower one lane per env at 5,492 envs)."""
@@ -186,7 +194,7 @@ class DeviceModel:
         if collide_variant is None:
             collide_variant = d.solver_variant if explicit else default_collide_variant(M, n_envs)
         if dyn_variant is None:
-            dyn_variant = d.solver_variant if explicit else default_stage_variant(M, n_envs)
+            dyn_variant = d.solver_variant if explicit else default_dyn_variant(M, n_envs)
         d.collide_variant, d.dyn_variant = int(collide_variant), int(dyn_variant)
         d.batch_dofs, d.batch_links, d.batch_joints = int(self.batch_dofs), int(self.batch_links), int(self.batch_joints)
         d.batch_eqs = 1

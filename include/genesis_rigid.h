@@ -235,7 +235,7 @@ typedef struct gsr_group {
 
 typedef struct gsr_batch_info {
   int32_t n_groups, n_tiles; /* groups and tiles in the batch */
-  int32_t grid;              /* workgroups per launch */
+  int32_t grid;              /* workgroups per launch (phased: of the dynamics stages) */
   int32_t lds_bytes;         /* dynamic LDS per workgroup (largest wavefront-variant group) */
   int32_t n_types;           /* distinct (model, state) pairs, in first-appearance order */
   int32_t persistent;        /* input: 1 = CUs x resident workgroups pull tiles from a queue, 0 = one per tile */

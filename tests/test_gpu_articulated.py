@@ -71,3 +71,39 @@ def test_single_entity_solver_matches_oracle(n, free_base):
                 bound = np.maximum(TOL + TOL * np.abs(o[b]), 4 * np.abs(o[b] - o64[b]).max() + TOL)
                 assert (np.abs(got[b] - o[b]) <= bound).all(), f"step {step} env {b} {name}"
     assert most > (64 if n == 64 else 0), most
+
+
+COMPARED = ["qpos", "vel", "acc", "acc_smooth", "dofs_pos", "links_pos", "links_quat", "geoms_pos", "geoms_quat",
+            "aabb_min", "aabb_max", "cdof_ang", "cdof_vel", "cdofd_ang", "cdofd_vel", "root_com", "cd_vel", "cd_ang",
+            "cinr_inertial", "cinr_pos", "cinr_mass", "links_iquat", "mass_blk", "mass_L_blk", "mass_D_inv",
+            "qf_applied", "qf_passive", "qf_bias", "qf_smooth", "force", "xanchor", "xaxis", "errno_env"]
+
+
+def _entities(name):
+    if name == "quadruped":
+        return [W.plane_entity(), W.go2_entity()]
+    if name == "arm_boxes":  # an articulated entity beside free bodies: several blocks of the mass matrix
+        return [W.plane_entity(), W.panda_entity()] + [W.box_entity((0.1, 0.1, 0.1), (0.6 + 0.3 * i, 0.5, 0.3)) for i in range(2)]
+    n, free = name
+    return [chain_entity(n, free)]
+
+
+@pytest.mark.parametrize("name", ["quadruped", "arm_boxes", (7, False), (16, False), (17, False), (33, False), (11, True)],
+                         ids=str)
+@pytest.mark.parametrize("B", [1, 5, 1027])  # 64 lanes per env up to 1,024 envs, 16 above (1,027: a partial wavefront)
+def test_tree_dynamics_equal_the_lane_per_env_ones(name, B):
+    """step_1, step_2 and the kinematics refresh of articulated models spread over lanes give the bits of the one-lane
+    walk: 16 dofs fill one register of the 16-lane substitutions, 17 two, 33 take the loop over LDS."""
+    from genesis_amd.rigid_solver import RigidSolver
+    M = compile_model(_entities(name), CompileOptions(dt=0.005, enable_self_collision=False,
+                                                      enable_collision=isinstance(name, str)))
+    out = []
+    for dyn in (0, 1):
+        S = RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=1, dyn_variant=dyn)
+        start(S, M, B, 3)
+        for _ in range(3):
+            S.substep()
+        torch.cuda.synchronize()
+        out.append({k: S.st.t[k].clone() for k in COMPARED})
+    for k in COMPARED:
+        assert torch.equal(out[0][k], out[1][k]), k
