@@ -29,12 +29,32 @@ __global__ void __launch_bounds__(kWave) k_solve_dense(gsr_model m, gsr_state s)
   wave_solve_dense(e, lds);
 }
 
+// Free bodies, kWaves wavefronts per env. Left to itself the compiler takes 250 VGPRs (two waves a SIMD); held to three
+// waves (168) for two wavefronts an env and to four (128) for four it spills to scratch but hides more latency: 1,500
+// 20-box piles 3,758 -> 3,318 us a pass, 4,096 64-box piles 32,383 -> 25,206 us (two, three, four: 32.9, 27.7, 25.2 ms).
+template <int kWaves>
+__global__ void __launch_bounds__(kWave * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves == 2 ? 3 : 4))) k_solve_bodies(gsr_model m, gsr_state s) {
+  extern __shared__ char lds[];
+  if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
+  const int b = xcd_env(blockIdx.x, s.n_envs);
+  Env e(m, s, b);
+  solve_bodies<kWaves>(e, lds);
+}
+
+template <int kWaves>
+void launch_bodies(const gsr_model& m, const gsr_state& s, hipStream_t st) {
+  hipLaunchKernelGGL(k_solve_bodies<kWaves>, dim3(s.n_envs), dim3(kWave * kWaves), solve_lds_bytes(m), st, m, s);
+}
+
 }  // namespace
 
 void launch_solve(const gsr_model& m, const gsr_state& s, hipStream_t st) {
   if (m.solver_variant == 1 && dense_solver(m))
     hipLaunchKernelGGL(k_solve_dense, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
-  else if (m.solver_variant == 1)
+  else if (m.solver_variant == 1 && bodies_solver(m)) {
+    if (bodies_waves(m.n_dofs) == 2) launch_bodies<2>(m, s, st);
+    else launch_bodies<4>(m, s, st);
+  } else if (m.solver_variant == 1)
     hipLaunchKernelGGL(k_solve_wave, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
   else
     hipLaunchKernelGGL(k_solve, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);

@@ -18,6 +18,7 @@
 // 377 -> 164 us, 32,768 quadrupeds 1,805 -> 543 us.
 #pragma once
 #include "rigid_env.h"
+#include "rigid_solver_bodies.h"
 #include "rigid_solver_wave.h"
 
 namespace gsr {
@@ -455,11 +456,14 @@ __device__ __forceinline__ void wave_solve_dense(const Env& e, char* lds) {
 // the Newton solve of one env on one wavefront
 __device__ __forceinline__ void wave_solve(const Env& e, char* lds) {
   if (dense_solver(e.m)) wave_solve_dense(e, lds);
+  else if (bodies_solver(e.m)) solve_bodies<1>(e, lds);
   else wave_solve_blocks(e, lds);
 }
 // dynamic LDS of wave_solve
 __host__ __device__ inline size_t solve_lds_bytes(const gsr_model& m) {
-  return dense_solver(m) ? dense_lds_bytes(m.n_dofs) : wave_lds_bytes(m);
+  return dense_solver(m)    ? dense_lds_bytes(m.n_dofs)
+         : bodies_solver(m) ? bodies_lds_bytes(m.n_dofs, m.wave_h_floats)
+                            : wave_lds_bytes(m);
 }
 
 }  // namespace gsr

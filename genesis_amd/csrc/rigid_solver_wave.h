@@ -1294,63 +1294,109 @@ __device__ __forceinline__ WLS ls_point_from(const Env& e, float qg0, float qg1,
 }
 
 // The points of the exact line search (func_linesearch, constraint_solver_decomp.py:1440-1792): point(alpha, ls_it)
-// evaluates one and counts it; returns the step
+// evaluates one and counts it; returns the step. Written as a state machine around a single evaluation: inlined at each
+// of the search's seven places the evaluation filled the instruction cache and the registers.
 template <class Point>
 __device__ __forceinline__ float linesearch_points(const gsr_model& m, float gtol, Point point) {
-  int ls_it = 0;
-  WLS p0 = point(0.f, ls_it);
-  WLS p1 = point(p0.alpha - p0.d0 / p0.d1, ls_it);
-  if (p0.cost < p1.cost) p1 = p0;
-  if (fabsf(p1.d0) < gtol) return p1.alpha;
-  float direction = (p1.d0 < 0.f) ? 1.f : -1.f;
-  int p2update = 0;
-  WLS p2 = p1;
-  while (p1.d0 * direction <= -gtol && ls_it < m.ls_iterations) {
-    p2 = p1;
-    p2update = 1;
-    p1 = point(p1.alpha - p1.d0 / p1.d1, ls_it);
-    if (fabsf(p1.d0) < gtol) return p1.alpha;
-  }
-  if (ls_it >= m.ls_iterations) return p1.alpha;
-  if (!p2update) return p1.alpha;
-  WLS p2n = p1;
-  WLS p1n = point(p1.alpha - p1.d0 / p1.d1, ls_it);
-  while (ls_it < m.ls_iterations) {
-    WLS pm = point((p1.alpha + p2.alpha) * 0.5f, ls_it);
-    // candidates p1n, p2n, pm in this order (named values, not an indexed array, so they stay in registers)
-    const WLS c0 = p1n, c1 = p2n, c2 = pm;
-    int best = -1;
-    float bcost = 0.f, balpha = 0.f;
-    auto consider = [&](const WLS& c, int idx) {
-      if (fabsf(c.d0) < gtol && (best < 0 || c.cost < bcost)) {
-        bcost = c.cost;
-        best = idx;
-        balpha = c.alpha;
+  enum { kFirst, kSecond, kBracket, kNext, kMid, kMoved1, kMoved2 } st = kFirst;
+  int ls_it = 0, f1 = 0, f2 = 0;
+  bool p2update = false;
+  float direction = 0.f, alpha = 0.f, pm_alpha = 0.f;
+  WLS p0{}, p1{}, p2{}, p1n{}, p2n{}, c0{}, c1{}, c2{};
+  auto newton = [](const WLS& p) { return p.alpha - p.d0 / p.d1; };
+  // p moves to the candidates c0, c1, c2 whose slope has its sign and is closer to zero
+  auto narrow = [&](WLS& p) {
+    int flag = 0;
+    auto step = [&](const WLS& c) {
+      if (p.d0 < 0.f && c.d0 < 0.f && p.d0 < c.d0) { p = c; flag = 1; }
+      else if (p.d0 > 0.f && c.d0 > 0.f && p.d0 > c.d0) { p = c; flag = 2; }
+    };
+    step(c0);
+    step(c1);
+    step(c2);
+    return flag;
+  };
+  for (;;) {
+    const WLS p = point(alpha, ls_it);
+    bool mid = false;  // on to the next bracket interval's middle
+    if (st == kFirst) {
+      p0 = p;
+      alpha = newton(p0);
+      st = kSecond;
+      continue;
+    }
+    if (st == kSecond || st == kBracket) {
+      p1 = p;
+      if (st == kSecond) {
+        if (p0.cost < p1.cost) p1 = p0;
+        direction = p1.d0 < 0.f ? 1.f : -1.f;
+        p2 = p1;
       }
-    };
-    consider(c0, 0);
-    consider(c1, 1);
-    consider(c2, 2);
-    if (best >= 0) return balpha;
-    // p1, then p2, moves to the candidates whose slope has its sign and is closer to zero
-    auto narrow = [&](WLS& p) {
-      int flag = 0;
-      auto step = [&](const WLS& c) {
-        if (p.d0 < 0.f && c.d0 < 0.f && p.d0 < c.d0) { p = c; flag = 1; }
-        else if (p.d0 > 0.f && c.d0 > 0.f && p.d0 > c.d0) { p = c; flag = 2; }
+      if (fabsf(p1.d0) < gtol) return p1.alpha;
+      if (p1.d0 * direction <= -gtol && ls_it < m.ls_iterations) {
+        p2 = p1;
+        p2update = true;
+        st = kBracket;
+      } else {
+        if (ls_it >= m.ls_iterations || !p2update) return p1.alpha;
+        p2n = p1;
+        st = kNext;
+      }
+      alpha = newton(p1);
+      continue;
+    }
+    if (st == kNext) {
+      p1n = p;
+      mid = true;
+    }
+    if (st == kMid) {
+      // candidates p1n, p2n and the middle, in this order
+      c0 = p1n;
+      c1 = p2n;
+      c2 = p;
+      pm_alpha = p.alpha;
+      bool found = false;
+      float bcost = 0.f, balpha = 0.f;
+      auto consider = [&](const WLS& c) {
+        if (fabsf(c.d0) < gtol && (!found || c.cost < bcost)) {
+          bcost = c.cost;
+          balpha = c.alpha;
+          found = true;
+        }
       };
-      step(c0);
-      step(c1);
-      step(c2);
-      return flag;
-    };
-    const int f1 = narrow(p1);
-    p1n = p1;
-    if (f1 > 0) p1n = point(p1.alpha - p1.d0 / p1.d1, ls_it);
-    const int f2 = narrow(p2);
-    p2n = p2;
-    if (f2 > 0) p2n = point(p2.alpha - p2.d0 / p2.d1, ls_it);
-    if (f1 == 0 && f2 == 0) return pm.alpha;
+      consider(c0);
+      consider(c1);
+      consider(c2);
+      if (found) return balpha;
+      f1 = narrow(p1);
+      p1n = p1;
+      if (f1 > 0) {
+        alpha = newton(p1);
+        st = kMoved1;
+        continue;
+      }
+    }
+    if (st == kMoved1) p1n = p;
+    if (st == kMid || st == kMoved1) {
+      f2 = narrow(p2);
+      p2n = p2;
+      if (f2 > 0) {
+        alpha = newton(p2);
+        st = kMoved2;
+        continue;
+      }
+      mid = true;
+    }
+    if (st == kMoved2) {
+      p2n = p;
+      mid = true;
+    }
+    if (mid) {
+      if (st != kNext && f1 == 0 && f2 == 0) return pm_alpha;
+      if (ls_it >= m.ls_iterations) break;
+      alpha = (p1.alpha + p2.alpha) * 0.5f;
+      st = kMid;
+    }
   }
   if (p1.cost <= p2.cost && p1.cost < p0.cost) return p1.alpha;
   if (p2.cost <= p1.cost && p2.cost < p1.cost) return p2.alpha;
