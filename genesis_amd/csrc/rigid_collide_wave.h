@@ -5,11 +5,17 @@
 //   * Sweep-and-prune (collider_decomp.py:1331-1470): the reference warm-starts an insertion sort with strict `<`,
 //     which is a stable sort of the previous order; here each lane ranks its entries (rank = #smaller + #equal
 //     before it), which gives the same permutation. The sweep's active list at a min event holds the geoms whose
-//     min event came earlier and whose max event comes later, in min-event order; each lane walks that set for its
-//     own events and a wave prefix sum of the pair counts places every pair where the serial sweep puts it.
+//     min event came earlier and whose max event comes later, in min-event order: event after event the earlier
+//     geoms are tested on their own lanes, from AABBs in LDS, and a ballot places every pair where the serial sweep
+//     puts it.
 //   * Narrowphase: one broadphase pair per lane, contacts kept in the lane (LocalSink) and placed by a prefix sum,
 //     convex pairs first and plane-box pairs second, both in broadphase order, as the reference appends them.
-//   * Rows: equality, frictionloss and limit rows on lane 0 (few), the 4 rows of each contact on its own lane.
+//   * Rows: equality rows on lane 0 (few), frictionloss and limit rows a link per lane, the 4 rows of each contact on its
+//     own lane.
+// What bounds it is dependent work on few lanes. Measured (us, whole stage; every event's set walked by one lane, every
+// dof's tables by lane 0 and a general pow in each row -> events' sets across lanes, links across lanes, integer powers as
+// products): 64 arms 45 -> 25, 100 7-box piles 62 -> 45, 1,500 20-box piles 250 -> 192, 96 64-box piles 641 -> 486,
+// 4,096 of them 2063 -> 1713.
 // Where the broadphase pair buffer overflows (errno bit 1) the serial sweep stops clearing the normal cache of
 // later non-overlapping pairs; this path clears them all. Results differ only after that error.
 #pragma once
@@ -31,11 +37,12 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
 }
 
 __host__ __device__ inline size_t wave_collide_lds_bytes(int G) {
-  return sizeof(float) * 4 * (size_t)G + sizeof(int) * 6 * (size_t)G + 64;
+  return sizeof(float) * 10 * (size_t)G + sizeof(int) * 6 * (size_t)G + 64;
 }
 
+// box: copies of the AABBs (minimum, maximum per geom) in LDS, or null
 template <int G = 64>
-__device__ inline void wave_update_aabbs(const Env& e, int lane) {
+__device__ inline void wave_update_aabbs(const Env& e, int lane, float* box = nullptr) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
   for (int g = lane; g < m.n_geoms; g += G) {
@@ -49,6 +56,10 @@ __device__ inline void wave_update_aabbs(const Env& e, int lane) {
     }
     e.S3(s.aabb_min, g, lo);
     e.S3(s.aabb_max, g, hi);
+    if (box) {
+      const float v[6] = {lo.x, lo.y, lo.z, hi.x, hi.y, hi.z};
+      for (int q = 0; q < 6; q++) box[6 * g + q] = v[q];
+    }
   }
 }
 
@@ -63,6 +74,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   int* tig = sig + G2;
   int* minpos = tig + G2;
   int* maxpos = minpos + G;
+  const float* box = reinterpret_cast<const float*>(maxpos + G);
   const bool first = e.I(s.first_time, 0) != 0;
   for (int i = lane; i < G2; i += 64) {
     int t;
@@ -70,7 +82,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
     else t = e.I(s.sort_ig, i);
     int g = t & (MAXB - 1);
     sig[i] = t;
-    sv[i] = (t & MAXB) ? e.F(s.aabb_max, 3 * g) : e.F(s.aabb_min, 3 * g);
+    sv[i] = box[6 * g + ((t & MAXB) ? 3 : 0)];
   }
   __syncthreads();
   if (first && lane == 0) e.I(s.first_time, 0) = 0;
@@ -97,41 +109,58 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
     else minpos[t] = i;
   }
   __syncthreads();
+  // geoms in the order of their min events: order[k] (tv's place), the AABBs in LDS. The geoms a min event pairs with are
+  // those before it in this order whose max event comes later; they are tested on their own lanes, 64 at a time, event
+  // after event, and a ballot places the pairs in the serial sweep's order.
+  int* order = tig;
+  int n_min = 0;
+  for (int i0 = 0; i0 < G2; i0 += 64) {
+    const int i = i0 + lane;
+    const bool is_min = i < G2 && !(sig[i] & MAXB);
+    const unsigned long long b = __ballot(is_min);
+    const int t = is_min ? sig[i] : 0;
+    __syncthreads();
+    if (is_min) order[n_min + __popcll(b & ((1ull << lane) - 1ull))] = t;
+    n_min += __popcll(b);
+  }
+  __syncthreads();
   int base = 0;
   bool overflow = false;
-  for (int p0 = 0; p0 < G2; p0 += 64) {
-    const int p = p0 + lane;
-    const bool is_min = p < G2 && !(sig[p] & MAXB);
-    const int gi = is_min ? sig[p] : 0;
-    int cnt = 0;
-    if (is_min) {
-      for (int j = 0; j < p; j++) {
-        int t = sig[j];
-        if ((t & MAXB) || maxpos[t] <= p) continue;
-        int ga = t < gi ? t : gi, gb = t < gi ? gi : t;
-        if (m.pair_idx[(size_t)ga * G + gb] == -1) continue;
-        if (dev_aabb_overlap(e, ga, gb)) cnt++;
+  const int g0 = lane < G ? order[lane] : 0, m0 = lane < G ? maxpos[g0] : -1;
+  float b0[6];
+  for (int q = 0; q < 6; q++) b0[q] = box[6 * g0 + q];
+  for (int ev = 1; ev < G; ev++) {
+    const int gi = __builtin_amdgcn_readfirstlane(order[ev]), pos = __builtin_amdgcn_readfirstlane(minpos[gi]);
+    float bi[6];
+    for (int q = 0; q < 6; q++) bi[q] = box[6 * gi + q];
+    for (int k0 = 0; k0 < ev; k0 += 64) {
+      const int k = k0 + lane;
+      int g = g0, mp = m0;
+      float bx[6];
+      for (int q = 0; q < 6; q++) bx[q] = b0[q];
+      if (k0 > 0) {
+        g = k < ev ? order[k] : 0;
+        mp = k < ev ? maxpos[g] : -1;
+        for (int q = 0; q < 6; q++) bx[q] = box[6 * g + q];
       }
-    }
-    int total;
-    int k = base + wave_excl_scan(cnt, lane, total);
-    if (is_min) {
-      for (int j = 0; j < p; j++) {
-        int t = sig[j];
-        if ((t & MAXB) || maxpos[t] <= p) continue;
-        int ga = t < gi ? t : gi, gb = t < gi ? gi : t;
-        int pidx = m.pair_idx[(size_t)ga * G + gb];
-        if (pidx == -1) continue;
-        if (!dev_aabb_overlap(e, ga, gb)) {
-          e.S3(s.cache_normal, pidx, zero3());
-          continue;
-        }
-        if (k < m.max_broad) e.I(s.broad_pairs, k) = (ga << 16) | gb;
+      int pidx = -1;
+      const int ga = min(g, gi), gb = max(g, gi);
+      if (k < ev && mp > pos) pidx = m.pair_idx[(size_t)ga * G + gb];
+      bool hit = false;
+      if (pidx != -1) {
+        // box: minimum then maximum of each geom
+        const bool sep = bx[3] <= bi[0] || bx[4] <= bi[1] || bx[5] <= bi[2] || bx[0] >= bi[3] || bx[1] >= bi[4] || bx[2] >= bi[5];
+        hit = !sep;
+        if (sep) e.S3(s.cache_normal, pidx, zero3());
+      }
+      const unsigned long long b = __ballot(hit);
+      const int at = base + __popcll(b & ((1ull << lane) - 1ull));
+      if (hit) {
+        if (at < m.max_broad) e.I(s.broad_pairs, at) = (ga << 16) | gb;
         else overflow = true;
-        k++;
       }
+      base += __popcll(b);
     }
-    base += total;
   }
   overflow = __any(overflow);
   if (lane == 0) {
@@ -235,21 +264,39 @@ __device__ inline void wave_narrow_phase(const Env& e, int lane) {
   __syncthreads();
 }
 
-// frictionloss rows on lane 0, the 4 rows of each contact on its own lane, limit rows on lane 0 after them
+// frictionloss and limit rows with a link per lane (counted, then placed by a prefix sum, so the rows come in link
+// order), the 4 rows of each contact on its own lane. One lane walking every dof's tables took longer than the contacts.
 __device__ __forceinline__ void wave_rows(const Env& e) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
   const int lane = threadIdx.x;
-  int n_con = 0, n_fl = 0;
-  if (lane == 0) n_con = dev_frictionloss_rows(e, e.I(s.n_con, 0), n_fl);
-  n_con = __shfl(n_con, 0, 64);
+  const int n_eq = e.I(s.n_con, 0);
+  int n_con = n_eq;
+  for (int l0 = 0; l0 < m.n_links; l0 += 64) {
+    const int l = l0 + lane;
+    int cnt = 0, total = 0;
+    if (l < m.n_links) each_frictionloss(e, l, [&](int, int) { cnt++; });
+    if (!__any(cnt)) continue;
+    int c = n_con + wave_excl_scan(cnt, lane, total);
+    if (cnt) each_frictionloss(e, l, [&](int j, int d) { dev_frictionloss_row(e, j, d, c++); });
+    n_con += total;
+  }
+  const int n_fl = n_con - n_eq;
   if (m.enable_collision) {
     int nc = e.I(s.n_contacts, 0);
     for (int ic = lane; ic < nc; ic += 64) dev_contact_rows(e, ic, n_con + 4 * ic);
     n_con += 4 * nc;
   }
+  for (int l0 = 0; m.enable_joint_limit && l0 < m.n_links; l0 += 64) {
+    const int l = l0 + lane;
+    int cnt = 0, total = 0;
+    if (l < m.n_links) each_limit(e, l, [&](int, int, float, float) { cnt++; });
+    if (!__any(cnt)) continue;
+    int c = n_con + wave_excl_scan(cnt, lane, total);
+    if (cnt) each_limit(e, l, [&](int j, int d, float dmin, float dmax) { dev_limit_row(e, j, d, dmin, dmax, c++); });
+    n_con += total;
+  }
   if (lane == 0) {
-    if (m.enable_joint_limit) n_con = dev_limit_rows(e, n_con);
     e.I(s.n_con, 0) = n_con;
     e.I(s.n_con, 2) = n_fl;
   }
@@ -269,7 +316,7 @@ __device__ __forceinline__ void wave_collide(const Env& e, char* lds) {
     e.I(s.gjk_defer_n, 0) = 0;
   }
   if (m.enable_collision) {
-    wave_update_aabbs(e, lane);
+    wave_update_aabbs(e, lane, reinterpret_cast<float*>(lds) + 10 * m.n_geoms);
     __syncthreads();
     if (m.n_pairs > 0) {
       wave_broad_phase(e, lds, lane);

@@ -12,7 +12,18 @@ __device__ __forceinline__ float crsin(float x) { return (float)sin((double)x); 
 __device__ __forceinline__ float crcos(float x) { return (float)cos((double)x); }
 __device__ __forceinline__ float cratan2(float y, float x) { return (float)atan2((double)y, (double)x); }
 __device__ __forceinline__ float cracos(float x) { return (float)acos((double)x); }
-__device__ __forceinline__ float crpow(float x, float y) { return (float)pow((double)x, (double)y); }
+// Integer powers up to 4 (the defaults of every impedance, and the JOINT equalities' polynomial) are products: x * x is
+// the correctly rounded square, x^3 and x^4 are rounded once to double and once to float, like pow's result. The general
+// pow is some 250 instructions, of which a contact took 16.
+__device__ __forceinline__ float crpow(float x, float y) {
+  if (y == 2.f) return x * x;
+  if (y == 1.f) return x;
+  if (y == 0.f) return 1.f;
+  const double d = (double)x, d2 = d * d;
+  if (y == 3.f) return (float)(d2 * d);
+  if (y == 4.f) return (float)(d2 * d2);
+  return (float)pow(d, (double)y);
+}
 
 struct f3 {
   float x, y, z;
@@ -185,20 +196,32 @@ __device__ __forceinline__ void orthogonals(f3 a, f3& b, f3& c) {
   c = cross(a, b);
 }
 // constraint impedance and reference acceleration (geom.py:377-398); the 7 solver parameters at p[k * st]
-__device__ __forceinline__ void imp_aref(const float* p, size_t st, float neg_pen, float vel, float pos, float& imp,
-                                         float& aref) {
+struct Impedance {
+  float imp, bb, k;
+};
+__device__ __forceinline__ Impedance impedance(const float* p, size_t st, float neg_pen) {
   float timeconst = p[0], dampratio = p[st], dmin = p[2 * st], dmax = p[3 * st], width = p[4 * st], mid = p[5 * st],
         power = p[6 * st];
   float imp_x = fabsf(neg_pen) / width;
   float imp_a = (1.f / crpow(mid, power - 1.f)) * crpow(imp_x, power);
   float imp_b = 1.f - (1.f / crpow(1.f - mid, power - 1.f)) * crpow(1.f - imp_x, power);
   float imp_y = imp_x < mid ? imp_a : imp_b;
-  imp = dmin + imp_y * (dmax - dmin);
-  imp = fminf(fmaxf(imp, dmin), dmax);
-  imp = imp_x > 1.f ? dmax : imp;
-  float bb = 2.f / (dmax * timeconst);
-  float k = 1.f / (dmax * dmax * timeconst * timeconst * dampratio * dampratio);
-  aref = -bb * vel - k * imp * pos;
+  Impedance r;
+  r.imp = dmin + imp_y * (dmax - dmin);
+  r.imp = fminf(fmaxf(r.imp, dmin), dmax);
+  r.imp = imp_x > 1.f ? dmax : r.imp;
+  r.bb = 2.f / (dmax * timeconst);
+  r.k = 1.f / (dmax * dmax * timeconst * timeconst * dampratio * dampratio);
+  return r;
+}
+__device__ __forceinline__ float impedance_aref(const Impedance& r, float vel, float pos) {
+  return -r.bb * vel - r.k * r.imp * pos;
+}
+__device__ __forceinline__ void imp_aref(const float* p, size_t st, float neg_pen, float vel, float pos, float& imp,
+                                         float& aref) {
+  const Impedance r = impedance(p, st, neg_pen);
+  imp = r.imp;
+  aref = impedance_aref(r, vel, pos);
 }
 __device__ __forceinline__ void imp_aref(const float* p, float neg_pen, float vel, float pos, float& imp, float& aref) {
   imp_aref(p, 1, neg_pen, vel, pos, imp, aref);

@@ -72,7 +72,7 @@ __device__ inline float point_diff_row(const Env& e, int l1, f3 p1, int l2, f3 p
       const f3 tpos = p - e.L3(s.root_com, link);
       for (int k = 0; k < nd; k++) {
         const int d = de - 1 - k;
-        const f3 vel = qrot(e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d)), qid());
+        const f3 vel = e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d));
         const float jac = comp(sign * vel, i3);
         jac_qvel = jac_qvel + jac * e.F(s.vel, d);
         row_add(r, d, jac);
@@ -235,30 +235,39 @@ __device__ inline void dev_equality_rows(const Env& e) {
   e.I(s.n_con, 1) = n_con;
 }
 
-// frictionloss rows (add_frictionloss_constraints), appended from row n_con; returns the new row count
-__device__ inline int dev_frictionloss_rows(const Env& e, int n_con, int& n_fl) {
+// f(joint, dof) for the dofs of link l with frictionloss, in order
+template <class F>
+__device__ __forceinline__ void each_frictionloss(const Env& e, int l, F f) {
+  const gsr_model& m = e.m;
+  for (int j = m.link_joint_start[l]; j < m.link_joint_end[l]; j++)
+    for (int d = m.joint_dof_start[j]; d < m.joint_dof_end[j]; d++)
+      if (e.DP(m.dof_frictionloss, d) > m.eps) f(j, d);
+}
+// the frictionloss row of dof d, stored at row c
+__device__ inline void dev_frictionloss_row(const Env& e, int j, int d, int c) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
+  float imp, aref;
+  size_t sps;
+  const float* sp = e.joint_sp(j, sps);
+  imp_aref(sp, sps, 0.f, 1.f * e.F(s.vel, d), 0.f, imp, aref);
+  const float diag = fmaxf(e.DP(m.dof_invweight, d) * (1.f - imp) / imp, m.eps);
+  e.EF(s.efc_diag, c) = diag;
+  e.EF(s.efc_aref, c) = aref;
+  e.EF(s.efc_D, c) = 1.f / diag;
+  e.EF(s.efc_fl, c) = e.DP(m.dof_frictionloss, d);
+  e.JI(c, 0) = d;
+  e.JV(c, 0) = 1.f;
+  e.EI(s.jac_nnz, c) = 1;
+}
+// frictionloss rows (add_frictionloss_constraints), appended from row n_con; returns the new row count
+__device__ inline int dev_frictionloss_rows(const Env& e, int n_con, int& n_fl) {
   n_fl = 0;
-  for (int l = 0; l < m.n_links; l++)
-    for (int j = m.link_joint_start[l]; j < m.link_joint_end[l]; j++)
-      for (int d = m.joint_dof_start[j]; d < m.joint_dof_end[j]; d++) {
-        if (e.DP(m.dof_frictionloss, d) > m.eps) {
-          float imp, aref;
-          size_t sps;
-          imp_aref(e.joint_sp(j, sps), sps, 0.f, 1.f * e.F(s.vel, d), 0.f, imp, aref);
-          float diag = fmaxf(e.DP(m.dof_invweight, d) * (1.f - imp) / imp, m.eps);
-          int c = n_con++;
-          n_fl++;
-          e.EF(s.efc_diag, c) = diag;
-          e.EF(s.efc_aref, c) = aref;
-          e.EF(s.efc_D, c) = 1.f / diag;
-          e.EF(s.efc_fl, c) = e.DP(m.dof_frictionloss, d);
-          RowBuf r;
-          r.n = 1; r.idx[0] = d; r.val[0] = 1.f;
-          row_store(e, c, r);
-        }
-      }
+  for (int l = 0; l < e.m.n_links; l++)
+    each_frictionloss(e, l, [&](int j, int d) {
+      dev_frictionloss_row(e, j, d, n_con++);
+      n_fl++;
+    });
   return n_con;
 }
 
@@ -299,7 +308,7 @@ __device__ inline void contact_rows_disjoint(const Env& e, int c0, int la, int l
       const f3 tpos = cp - e.L3(s.root_com, link);
       for (int k = 0; k < nd; k++, slot--) {
         const int d = de - 1 - k;
-        const f3 vel = qrot(e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d)), qid());
+        const f3 vel = e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d));
         const float qv = e.F(s.vel, d);
         for (int i = 0; i < 4; i++) {
           const float jac = dot(sign * vel, n[i]);
@@ -325,6 +334,12 @@ __device__ inline void dev_contact_rows(const Env& e, int ic, int c0) {
   orthogonals(cn, d1, d2);
   float invw = e.LP(m.link_invweight, 2 * la);
   if (lb > -1) invw = invw + e.LP(m.link_invweight, 2 * lb);
+  // the impedance depends on the penetration alone: once per contact, not per row
+  const Impedance im = impedance(sp, 1, -pen);
+  float diag = invw + fr * fr * invw;
+  diag *= 2.f * fr * fr * (1.f - im.imp) / im.imp;
+  diag = fmaxf(diag, m.eps);
+  const float Dc = 1.f / diag;
   {
     int na, nb, lo_a, hi_a, lo_b, hi_b;
     bool desc_a, desc_b;
@@ -339,14 +354,9 @@ __device__ inline void dev_contact_rows(const Env& e, int ic, int c0) {
       for (int i = 0; i < 4; i++) {
         const int c = c0 + i;
         e.EI(s.jac_nnz, c) = na + nb;
-        float imp, aref;
-        imp_aref(sp, -pen, jq[i], -pen, imp, aref);
-        float diag = invw + fr * fr * invw;
-        diag *= 2.f * fr * fr * (1.f - imp) / imp;
-        diag = fmaxf(diag, m.eps);
         e.EF(s.efc_diag, c) = diag;
-        e.EF(s.efc_aref, c) = aref;
-        e.EF(s.efc_D, c) = 1.f / diag;
+        e.EF(s.efc_aref, c) = impedance_aref(im, jq[i], -pen);
+        e.EF(s.efc_D, c) = Dc;
       }
       return;
     }
@@ -366,7 +376,7 @@ __device__ inline void dev_contact_rows(const Env& e, int ic, int c0) {
         f3 tpos = cp - e.L3(s.root_com, link);
         for (int k = 0; k < nd; k++) {
           int d = de - 1 - k;
-          f3 vel = qrot(e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d)), qid());
+          f3 vel = e.L3(s.cdof_vel, d) - cross(tpos, e.L3(s.cdof_ang, d));
           float jac = dot(sign * vel, n);
           jac_qvel = jac_qvel + jac * e.F(s.vel, d);
           row_add(r, d, jac);
@@ -376,44 +386,47 @@ __device__ inline void dev_contact_rows(const Env& e, int ic, int c0) {
     }
     row_sort(r);
     row_store(e, c, r);
-    float imp, aref;
-    imp_aref(sp, -pen, jac_qvel, -pen, imp, aref);
-    float diag = invw + fr * fr * invw;
-    diag *= 2.f * fr * fr * (1.f - imp) / imp;
-    diag = fmaxf(diag, m.eps);
     e.EF(s.efc_diag, c) = diag;
-    e.EF(s.efc_aref, c) = aref;
-    e.EF(s.efc_D, c) = 1.f / diag;
+    e.EF(s.efc_aref, c) = impedance_aref(im, jac_qvel, -pen);
+    e.EF(s.efc_D, c) = Dc;
   }
 }
 
-// joint-limit rows (add_joint_limit_constraints), appended from row n_con; returns the new row count
-__device__ inline int dev_limit_rows(const Env& e, int n_con) {
+// f(joint, dof, distances to the lower and upper limit) for the joints of link l beyond a limit, in order
+template <class F>
+__device__ __forceinline__ void each_limit(const Env& e, int l, F f) {
+  const gsr_model& m = e.m;
+  for (int j = m.link_joint_start[l]; j < m.link_joint_end[l]; j++) {
+    const int jt = m.joint_type[j];
+    if (jt != JOINT_REVOLUTE && jt != JOINT_PRISMATIC) continue;
+    const int d = m.joint_dof_start[j];
+    const float qv = e.F(e.s.qpos, m.joint_q_start[j]);
+    const float dmin = qv - e.DP(m.dof_limit, 2 * d), dmax = e.DP(m.dof_limit, 2 * d + 1) - qv;
+    if (fminf(dmin, dmax) < 0.f) f(j, d, dmin, dmax);
+  }
+}
+// the limit row of joint j, stored at row c
+__device__ inline void dev_limit_row(const Env& e, int j, int d, float dmin, float dmax, int c) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  for (int l = 0; l < m.n_links; l++)
-    for (int j = m.link_joint_start[l]; j < m.link_joint_end[l]; j++) {
-      int jt = m.joint_type[j];
-      if (jt != JOINT_REVOLUTE && jt != JOINT_PRISMATIC) continue;
-      int q = m.joint_q_start[j], d = m.joint_dof_start[j];
-      float qv = e.F(s.qpos, q);
-      float dmin = qv - e.DP(m.dof_limit, 2 * d), dmax = e.DP(m.dof_limit, 2 * d + 1) - qv;
-      float pd = fminf(dmin, dmax);
-      if (pd < 0.f) {
-        float jac = (dmin < dmax) ? 1.f : -1.f;
-        float imp, aref;
-        size_t sps;
-        imp_aref(e.joint_sp(j, sps), sps, pd, jac * e.F(s.vel, d), pd, imp, aref);
-        float diag = fmaxf(e.DP(m.dof_invweight, d) * (1.f - imp) / imp, m.eps);
-        int c = n_con++;
-        e.EF(s.efc_diag, c) = diag;
-        e.EF(s.efc_aref, c) = aref;
-        e.EF(s.efc_D, c) = 1.f / diag;
-        RowBuf r;
-        r.n = 1; r.idx[0] = d; r.val[0] = jac;
-        row_store(e, c, r);
-      }
-    }
+  const float pd = fminf(dmin, dmax);
+  const float jac = (dmin < dmax) ? 1.f : -1.f;
+  float imp, aref;
+  size_t sps;
+  const float* sp = e.joint_sp(j, sps);
+  imp_aref(sp, sps, pd, jac * e.F(s.vel, d), pd, imp, aref);
+  const float diag = fmaxf(e.DP(m.dof_invweight, d) * (1.f - imp) / imp, m.eps);
+  e.EF(s.efc_diag, c) = diag;
+  e.EF(s.efc_aref, c) = aref;
+  e.EF(s.efc_D, c) = 1.f / diag;
+  e.JI(c, 0) = d;
+  e.JV(c, 0) = jac;
+  e.EI(s.jac_nnz, c) = 1;
+}
+// joint-limit rows (add_joint_limit_constraints), appended from row n_con; returns the new row count
+__device__ inline int dev_limit_rows(const Env& e, int n_con) {
+  for (int l = 0; l < e.m.n_links; l++)
+    each_limit(e, l, [&](int j, int d, float dmin, float dmax) { dev_limit_row(e, j, d, dmin, dmax, n_con++); });
   return n_con;
 }
 
