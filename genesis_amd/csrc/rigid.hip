@@ -517,8 +517,8 @@ static int phase_lds(const gsr_batch_info& b, int phase) {
   size_t lds = 0;
   for (int k = 0; k < b.n_types; k++) {
     const gsr_model& m = b.models[k];
-    if (phase == 1 && m.collide_variant == 1) lds = std::max(lds, (size_t)wave_collide_lds_bytes(m.n_geoms));
     // room for tiles of several envs: a group's tile size is not known here
+    if (phase == 1 && collide_waves(m)) lds = std::max(lds, wave_collide_lds_bytes(m.n_geoms, collide_packs(m) ? 4 : 1));
     if (phase == 0 || phase == 4) lds = std::max(lds, dyn_lds_bytes(m, kWave));
     if (phase == 3 && m.solver_variant == 1)
       lds = std::max(lds, (size_t)solve_lds_bytes(m));
@@ -526,7 +526,7 @@ static int phase_lds(const gsr_batch_info& b, int phase) {
   return (int)lds;
 }
 
-static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int dyn_tiles, size_t lds,
+static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int grid, size_t lds,
                               gsr_batch_info* info);
 
 int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table, int64_t table_bytes,
@@ -536,7 +536,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
   std::vector<BatchRange> ranges(n_groups);
   gsr_batch_info out;
   std::memset(&out, 0, sizeof(out));
-  int tiles = 0, wtiles = 0, dtiles = 0;
+  int tiles = 0, wtiles = 0, dtiles = 0, ctiles = 0;
   size_t lds = 0;
   for (int g = 0; g < n_groups; g++) {
     const gsr_group& G = groups[g];
@@ -563,10 +563,12 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
     lds = std::max(lds, dyn_lds_bytes(G.model, G.envs_per_tile));
     const int Td = dyn_tile_envs(G.model, G.n_envs, G.envs_per_tile);
     const int n_t = (G.n_envs + G.envs_per_tile - 1) / G.envs_per_tile, n_w = (G.n_envs + Tw - 1) / Tw;
-    const int n_d = (G.n_envs + Td - 1) / Td;
+    const int Tc = collide_tile_envs(G.model, G.n_envs, G.envs_per_tile);
+    const int n_d = (G.n_envs + Td - 1) / Td, n_c = (G.n_envs + Tc - 1) / Tc;
     ranges[g] = BatchRange{type, G.env_begin, G.n_envs, G.envs_per_tile, tiles, tiles + n_t, Tw, wtiles, wtiles + n_w,
-                           Td, dtiles, dtiles + n_d};
+                           Td, dtiles, dtiles + n_d, Tc, ctiles, ctiles + n_c};
     dtiles += n_d;
+    ctiles += n_c;
     tiles += n_t;
     wtiles += n_w;
   }
@@ -589,7 +591,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
       if (B.env_begin < A.env_begin + A.n_envs) return GSR_E_ARG;
     }
   }
-  BatchHeader h{n_groups, tiles, 0u, 0u, wtiles, dtiles, 0, 0};
+  BatchHeader h{n_groups, tiles, 0u, 0u, wtiles, dtiles, ctiles, 0};
   FusedTypes ty;
   std::memset(&ty, 0, sizeof(ty));
   for (int k = 0; k < out.n_types; k++) {
@@ -604,14 +606,14 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
     return GSR_E_LAUNCH;
   if (hipMemcpy(dev_table, &h, 2 * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(static_cast<char*>(dev_table) + offsetof(BatchHeader, n_wave_tiles), &h.n_wave_tiles,
-                2 * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess)
+                3 * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess)
     return GSR_E_LAUNCH;
-  return finish_launch_info(out, n_groups, tiles, wtiles, dtiles, lds, info);
+  return finish_launch_info(out, n_groups, tiles, wtiles, std::max(dtiles, ctiles), lds, info);
 }
 
 // Launch form of a batch whose types are in `out`: kernel attributes (dynamic LDS), grid and the form's flags, read
 // from `info` and written back to it.
-static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int dyn_tiles, size_t lds,
+static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int wave_tiles, int grid, size_t lds,
                               gsr_batch_info* info) {
   int dev = 0, n_cu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return GSR_E_LAUNCH;
@@ -634,7 +636,7 @@ static int finish_launch_info(gsr_batch_info& out, int n_groups, int tiles, int 
     out.waves_per_simd = 0;
     out.gjk_inline = 0;
     out.phased = 1;
-    out.grid = dyn_tiles;
+    out.grid = grid;  // the larger of the dynamics and the collision tiles
     out.lds_bytes = (int32_t)lds;
     *info = out;
     return GSR_OK;
@@ -676,7 +678,7 @@ int gsr_launch_fused_kernel(const void* dev_table, const gsr_batch_info* info, i
   const char* t = static_cast<const char*>(dev_table);
   if (info->phased) {
     const int lds = k == 2 ? 0 : phase_lds(*info, k);
-    const int tiles = k == 2 || k == 3 ? info->n_wave_tiles : k == 1 ? info->n_tiles : info->grid;
+    const int tiles = k == 2 || k == 3 ? info->n_wave_tiles : info->grid;
     launch_phase(k, dim3(tiles), lds, stream, t);
   } else if (k == 0) {
     uint32_t* queue = reinterpret_cast<uint32_t*>(const_cast<char*>(t) + 2 * sizeof(int32_t));

@@ -1,4 +1,5 @@
-// Collision detection and constraint rows of one environment on one wavefront (64 lanes).
+// Collision detection and constraint rows of environments on wavefronts, W lanes per env (64: one env a wavefront, 16:
+// four envs a wavefront; collide_lanes() says which).
 //
 // Same results as the one-lane-per-env path of rigid_collide.h / rigid_solver.h, spread over lanes:
 //   * AABBs: one geom per lane (rigid_solver_decomp.py:5668-5689).
@@ -16,8 +17,6 @@
 // dof's tables by lane 0 and a general pow in each row -> events' sets across lanes, links across lanes, integer powers as
 // products): 64 arms 45 -> 25, 100 7-box piles 62 -> 45, 1,500 20-box piles 250 -> 192, 96 64-box piles 641 -> 486,
 // 4,096 of them 2063 -> 1713.
-// Where the broadphase pair buffer overflows (errno bit 1) the serial sweep stops clearing the normal cache of
-// later non-overlapping pairs; this path clears them all. Results differ only after that error.
 #pragma once
 #include "rigid_collide.h"
 #include "rigid_solver.h"
@@ -26,19 +25,45 @@ namespace gsr {
 
 constexpr int kWaveMaxGeoms = 1024;
 
+// exclusive prefix sum over the W lanes of an env, its total on every lane
+template <int W>
 __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
   int x = v;
-  for (int o = 1; o < 64; o <<= 1) {
-    int y = __shfl_up(x, o, 64);
+  for (int o = 1; o < W; o <<= 1) {
+    int y = __shfl_up(x, o, W);
     if (lane >= o) x += y;
   }
-  total = __shfl(x, 63, 64);
+  total = __shfl(x, W - 1, W);
   return x - v;
 }
-
-__host__ __device__ inline size_t wave_collide_lds_bytes(int G) {
-  return sizeof(float) * 10 * (size_t)G + sizeof(int) * 6 * (size_t)G + 64;
+// the lanes of this lane's env for which v holds
+template <int W>
+__device__ __forceinline__ unsigned long long env_ballot(bool v) {
+  const unsigned long long b = __ballot(v);
+  if constexpr (W == 64) return b;
+  else return (b >> (threadIdx.x & ~(W - 1))) & ((1ull << W) - 1ull);
 }
+
+// LDS words of one env
+__host__ __device__ inline size_t wave_collide_words(int G) { return 16 * (size_t)G + 4; }
+__host__ __device__ inline size_t wave_collide_lds_bytes(int G, int envs = 1) {
+  return sizeof(float) * wave_collide_words(G) * (size_t)envs + 64;
+}
+// Models whose collision the wavefront form holds (its LDS, its contact buffer of a pair): all that any scene here has. The
+// others take a lane per env.
+__host__ __device__ inline bool collide_waves(const gsr_model& m) {
+  return m.collide_variant == 1 ||
+         (wave_collide_lds_bytes(m.n_geoms) <= 64 * 1024 && m.n_contacts_per_pair <= kMaxPairContacts);
+}
+// Models that may share a wavefront among four envs: with few entities a few pairs reach the narrowphase and a few contacts
+// the rows, which leaves most of 64 lanes idle.
+__host__ __device__ inline bool collide_packs(const gsr_model& m) { return m.n_entities <= 8 && m.n_geoms <= 32; }
+// Lanes per env of a launch over n envs. Up to 2,048 envs there are SIMDs to spare and 64 lanes finish sooner; above, four
+// envs a wavefront are faster where the model packs. Measured (us, collision and GJK/EPA pass; one lane per env, 64, 16
+// lanes): quadrupeds 2,048: 576, 68, 68; 4,000: 585, 123, 80; 32,768: 824, 939, 374; arms 2,000: 707, 76, 89; 5,000: 726,
+// 120, 98; 7-box piles 1,024: 465, 58, 55; 4,000: 488, 122, 105; 16,384: 569, 491, 342. Heaps do not pack: 20 boxes 300:
+// 4213, 172, 354; 4,000: 4437, 403, 448; 64 boxes 1,024: 25968, 566, 1529.
+__host__ __device__ inline int collide_lanes(const gsr_model& m, int n) { return n > 2048 && collide_packs(m) ? 16 : kWave; }
 
 // box: copies of the AABBs (minimum, maximum per geom) in LDS, or null
 template <int G = 64>
@@ -63,6 +88,7 @@ __device__ inline void wave_update_aabbs(const Env& e, int lane, float* box = nu
   }
 }
 
+template <int W>
 __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
@@ -76,7 +102,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   int* maxpos = minpos + G;
   const float* box = reinterpret_cast<const float*>(maxpos + G);
   const bool first = e.I(s.first_time, 0) != 0;
-  for (int i = lane; i < G2; i += 64) {
+  for (int i = lane; i < G2; i += W) {
     int t;
     if (first) t = (i & 1) ? ((i >> 1) | MAXB) : (i >> 1);
     else t = e.I(s.sort_ig, i);
@@ -87,7 +113,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   __syncthreads();
   if (first && lane == 0) e.I(s.first_time, 0) = 0;
   // stable rank sort
-  for (int i = lane; i < G2; i += 64) {
+  for (int i = lane; i < G2; i += W) {
     float v = sv[i];
     int r = 0;
     for (int j = 0; j < G2; j++) {
@@ -98,7 +124,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
     tig[r] = sig[i];
   }
   __syncthreads();
-  for (int i = lane; i < G2; i += 64) {
+  for (int i = lane; i < G2; i += W) {
     float v = tv[i];
     int t = tig[i];
     sv[i] = v;
@@ -110,14 +136,14 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   }
   __syncthreads();
   // geoms in the order of their min events: order[k] (tv's place), the AABBs in LDS. The geoms a min event pairs with are
-  // those before it in this order whose max event comes later; they are tested on their own lanes, 64 at a time, event
+  // those before it in this order whose max event comes later; they are tested on their own lanes, W at a time, event
   // after event, and a ballot places the pairs in the serial sweep's order.
   int* order = tig;
   int n_min = 0;
-  for (int i0 = 0; i0 < G2; i0 += 64) {
+  for (int i0 = 0; i0 < G2; i0 += W) {
     const int i = i0 + lane;
     const bool is_min = i < G2 && !(sig[i] & MAXB);
-    const unsigned long long b = __ballot(is_min);
+    const unsigned long long b = env_ballot<W>(is_min);
     const int t = is_min ? sig[i] : 0;
     __syncthreads();
     if (is_min) order[n_min + __popcll(b & ((1ull << lane) - 1ull))] = t;
@@ -130,10 +156,11 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   float b0[6];
   for (int q = 0; q < 6; q++) b0[q] = box[6 * g0 + q];
   for (int ev = 1; ev < G; ev++) {
-    const int gi = __builtin_amdgcn_readfirstlane(order[ev]), pos = __builtin_amdgcn_readfirstlane(minpos[gi]);
+    const int gi = order[ev], pos = minpos[gi];
+    const int full = max(base, m.max_broad);  // the serial sweep leaves an event at the first pair that finds no room
     float bi[6];
     for (int q = 0; q < 6; q++) bi[q] = box[6 * gi + q];
-    for (int k0 = 0; k0 < ev; k0 += 64) {
+    for (int k0 = 0; k0 < ev; k0 += W) {
       const int k = k0 + lane;
       int g = g0, mp = m0;
       float bx[6];
@@ -151,10 +178,10 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
         // box: minimum then maximum of each geom
         const bool sep = bx[3] <= bi[0] || bx[4] <= bi[1] || bx[5] <= bi[2] || bx[0] >= bi[3] || bx[1] >= bi[4] || bx[2] >= bi[5];
         hit = !sep;
-        if (sep) e.S3(s.cache_normal, pidx, zero3());
       }
-      const unsigned long long b = __ballot(hit);
+      const unsigned long long b = env_ballot<W>(hit);
       const int at = base + __popcll(b & ((1ull << lane) - 1ull));
+      if (pidx != -1 && !hit && at <= full) e.S3(s.cache_normal, pidx, zero3());
       if (hit) {
         if (at < m.max_broad) e.I(s.broad_pairs, at) = (ga << 16) | gb;
         else overflow = true;
@@ -162,7 +189,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
       base += __popcll(b);
     }
   }
-  overflow = __any(overflow);
+  overflow = env_ballot<W>(overflow) != 0ull;
   if (lane == 0) {
     e.I(s.n_broad, 0) = min(base, m.max_broad);
     if (overflow) e.I((int32_t*)s.errno_env, 0) |= (int)GSR_ERR_BROAD_OVERFLOW;
@@ -173,12 +200,12 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
 // one pass over the broadphase pairs of one kind (convex pairs, then plane-box pairs), contacts appended at `base`
 // kGjk: pairs that need GJK/EPA are redone in place, one lane at a time (they share the env's workspace), instead of
 // being deferred to the GJK/EPA pass
-template <bool kGjk>
+template <bool kGjk, int W>
 __device__ inline int wave_narrow_pass(const Env& e, int lane, int nb, bool plane_box_pass, int base,
                                        uint32_t& err, int& n_def) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  for (int p0 = 0; p0 < nb; p0 += 64) {
+  for (int p0 = 0; p0 < nb; p0 += W) {
     const int ip = p0 + lane;
     PairContacts pc;
     pc.cnt = 0;
@@ -199,7 +226,7 @@ __device__ inline int wave_narrow_pass(const Env& e, int lane, int nb, bool plan
       }
     }
     if (kGjk) {
-      unsigned long long redo = __ballot(pc.deferred);
+      unsigned long long redo = env_ballot<W>(pc.deferred);
       while (redo) {
         int j = __ffsll((long long)redo) - 1;
         redo &= redo - 1;
@@ -217,9 +244,9 @@ __device__ inline int wave_narrow_pass(const Env& e, int lane, int nb, bool plan
       pc.cnt = 0;
       pc.err = 0;
     }
-    const unsigned long long def = __ballot(pc.deferred);
+    const unsigned long long def = env_ballot<W>(pc.deferred);
     int total;
-    int k = base + wave_excl_scan(pc.cnt, lane, total);
+    int k = base + wave_excl_scan<W>(pc.cnt, lane, total);
     if (pc.deferred) {
       const int slot = n_def + __popcll(def & ((1ull << lane) - 1ull));
       e.I(s.gjk_defer, 2 * slot) = (ga << 16) | gb;
@@ -246,16 +273,16 @@ __device__ inline int wave_narrow_pass(const Env& e, int lane, int nb, bool plan
   return base;
 }
 
-template <bool kGjk>
+template <bool kGjk, int W>
 __device__ inline void wave_narrow_phase(const Env& e, int lane) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
   const int nb = e.I(s.n_broad, 0);
   uint32_t err = 0;
   int n_def = 0;
-  int n = wave_narrow_pass<kGjk>(e, lane, nb, false, 0, err, n_def);
-  n = wave_narrow_pass<kGjk>(e, lane, nb, true, n, err, n_def);
-  for (int o = 32; o > 0; o >>= 1) err |= (uint32_t)__shfl_xor((int)err, o, 64);
+  int n = wave_narrow_pass<kGjk, W>(e, lane, nb, false, 0, err, n_def);
+  n = wave_narrow_pass<kGjk, W>(e, lane, nb, true, n, err, n_def);
+  for (int o = W / 2; o > 0; o >>= 1) err |= (uint32_t)__shfl_xor((int)err, o, W);
   if (lane == 0) {
     e.I(s.n_contacts, 0) = min(n, m.max_contacts);
     e.I(s.gjk_defer_n, 0) = n_def;
@@ -266,33 +293,34 @@ __device__ inline void wave_narrow_phase(const Env& e, int lane) {
 
 // frictionloss and limit rows with a link per lane (counted, then placed by a prefix sum, so the rows come in link
 // order), the 4 rows of each contact on its own lane. One lane walking every dof's tables took longer than the contacts.
+template <int W = 64>
 __device__ __forceinline__ void wave_rows(const Env& e) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & (W - 1);
   const int n_eq = e.I(s.n_con, 0);
   int n_con = n_eq;
-  for (int l0 = 0; l0 < m.n_links; l0 += 64) {
+  for (int l0 = 0; l0 < m.n_links; l0 += W) {
     const int l = l0 + lane;
     int cnt = 0, total = 0;
     if (l < m.n_links) each_frictionloss(e, l, [&](int, int) { cnt++; });
-    if (!__any(cnt)) continue;
-    int c = n_con + wave_excl_scan(cnt, lane, total);
+    if (env_ballot<W>(cnt != 0) == 0ull) continue;
+    int c = n_con + wave_excl_scan<W>(cnt, lane, total);
     if (cnt) each_frictionloss(e, l, [&](int j, int d) { dev_frictionloss_row(e, j, d, c++); });
     n_con += total;
   }
   const int n_fl = n_con - n_eq;
   if (m.enable_collision) {
     int nc = e.I(s.n_contacts, 0);
-    for (int ic = lane; ic < nc; ic += 64) dev_contact_rows(e, ic, n_con + 4 * ic);
+    for (int ic = lane; ic < nc; ic += W) dev_contact_rows(e, ic, n_con + 4 * ic);
     n_con += 4 * nc;
   }
-  for (int l0 = 0; m.enable_joint_limit && l0 < m.n_links; l0 += 64) {
+  for (int l0 = 0; m.enable_joint_limit && l0 < m.n_links; l0 += W) {
     const int l = l0 + lane;
     int cnt = 0, total = 0;
     if (l < m.n_links) each_limit(e, l, [&](int, int, float, float) { cnt++; });
-    if (!__any(cnt)) continue;
-    int c = n_con + wave_excl_scan(cnt, lane, total);
+    if (env_ballot<W>(cnt != 0) == 0ull) continue;
+    int c = n_con + wave_excl_scan<W>(cnt, lane, total);
     if (cnt) each_limit(e, l, [&](int j, int d, float dmin, float dmax) { dev_limit_row(e, j, d, dmin, dmax, c++); });
     n_con += total;
   }
@@ -303,12 +331,13 @@ __device__ __forceinline__ void wave_rows(const Env& e) {
   __syncthreads();
 }
 
-// equality rows, collision detection and inequality rows of one env (k_collide's work) on one wavefront
-template <bool kGjk = false>
+// equality rows, collision detection and inequality rows of one env (k_collide's work) on the W lanes holding it; lds: the
+// env's words
+template <bool kGjk = false, int W = 64>
 __device__ __forceinline__ void wave_collide(const Env& e, char* lds) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & (W - 1);
   if (lane == 0) {
     dev_equality_rows(e);
     e.I(s.n_contacts, 0) = 0;
@@ -316,17 +345,17 @@ __device__ __forceinline__ void wave_collide(const Env& e, char* lds) {
     e.I(s.gjk_defer_n, 0) = 0;
   }
   if (m.enable_collision) {
-    wave_update_aabbs(e, lane, reinterpret_cast<float*>(lds) + 10 * m.n_geoms);
+    wave_update_aabbs<W>(e, lane, reinterpret_cast<float*>(lds) + 10 * m.n_geoms);
     __syncthreads();
     if (m.n_pairs > 0) {
-      wave_broad_phase(e, lds, lane);
-      wave_narrow_phase<kGjk>(e, lane);
+      wave_broad_phase<W>(e, lds, lane);
+      wave_narrow_phase<kGjk, W>(e, lane);
     }
   }
   __syncthreads();
   // with deferred pairs the contact list is not final yet: the GJK/EPA pass builds the rows after inserting them
   if (e.I(s.gjk_defer_n, 0) > 0) return;
-  wave_rows(e);
+  wave_rows<W>(e);
 }
 
 // The GJK/EPA pass of one env on one wavefront: lane 0 recomputes the deferred pairs with GJK/EPA (they share the

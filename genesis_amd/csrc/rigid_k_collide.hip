@@ -1,4 +1,5 @@
-// Collision stage of the plain step: k_collide (one lane per env) or k_collide_wave (one wavefront per env), then
+// Collision stage of the plain step: k_collide_wave (16 or 64 lanes per env; k_collide, one lane per env, only for models
+// its LDS does not hold), then
 // the GJK/EPA pass k_gjk_fixup over the pairs the narrowphase deferred.
 #include "rigid_tiles.h"
 
@@ -27,22 +28,26 @@ k_gjk_fixup(gsr_model m, gsr_state s) {
 // Register budget of two waves per SIMD: left to itself the narrowphase takes 256 VGPRs plus AGPRs (one wave per
 // SIMD); held to 256 it spills more to scratch but doubles the waves that hide each other's latency (25 % faster on
 // the 20-box pile)
+template <int W>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 8)))
 k_collide_wave(gsr_model m, gsr_state s) {
   extern __shared__ char lds[];
-  if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
-  const int b = xcd_env(blockIdx.x, s.n_envs);
-  Env e(m, s, b);
-  wave_collide(e, lds);
+  constexpr int kEnvs = kWave / W;
+  const int sub = threadIdx.x / W, b = xcd_env(blockIdx.x, (s.n_envs + kEnvs - 1) / kEnvs) * kEnvs + sub;
+  if (b >= s.n_envs) return;  // uniform across an env's lanes
+  wave_collide<false, W>(Env(m, s, b), lds + sizeof(float) * wave_collide_words(m.n_geoms) * sub);
 }
 
 }  // namespace
 
 void launch_collide(const gsr_model& m, const gsr_state& s, hipStream_t st) {
-  if (m.collide_variant == 1)
-    hipLaunchKernelGGL(k_collide_wave, dim3(s.n_envs), dim3(kWave), wave_collide_lds_bytes(m.n_geoms), st, m, s);
-  else
+  if (!collide_waves(m))
     hipLaunchKernelGGL(k_collide, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);
+  else if (collide_lanes(m, s.n_envs) == 16)
+    hipLaunchKernelGGL(k_collide_wave<16>, dim3((s.n_envs + 3) / 4), dim3(kWave), wave_collide_lds_bytes(m.n_geoms, 4), st,
+                       m, s);
+  else
+    hipLaunchKernelGGL(k_collide_wave<kWave>, dim3(s.n_envs), dim3(kWave), wave_collide_lds_bytes(m.n_geoms), st, m, s);
   hipLaunchKernelGGL(k_gjk_fixup, dim3(s.n_envs), dim3(kWave), 0, st, m, s);
 }
 

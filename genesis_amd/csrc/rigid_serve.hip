@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(kSchedThreads) k_serve_schedule(ServeDev* S, c
     if (a) {
       const int p = pool_of_tile(S, g);
       const int ept = S->pools[p].envs_per_tile;
-      R[idx] = BatchRange{p, (g - S->pool_tile0[p]) * ept, T.n[g], ept, idx, idx + 1, ept, idx, idx + 1, ept, idx, idx + 1};
+      R[idx] = BatchRange{p, (g - S->pool_tile0[p]) * ept, T.n[g], ept, idx, idx + 1, ept, idx, idx + 1, ept, idx, idx + 1, ept, idx, idx + 1};
     }
     base += chunk;
   }
@@ -198,6 +198,7 @@ __global__ void __launch_bounds__(kSchedThreads) k_serve_schedule(ServeDev* S, c
     H->n_tiles = base;
     H->n_wave_tiles = base;
     H->n_dyn_tiles = base;
+    H->n_collide_tiles = base;
   }
 }
 

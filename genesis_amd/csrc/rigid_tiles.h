@@ -88,6 +88,25 @@ __host__ __device__ inline int dyn_tile_envs(const gsr_model& m, int n, int envs
   if (m.dyn_variant != 1) return envs_per_tile;
   return tree_dynamics(m) ? kWave / tree_lanes(m, n) : 1;
 }
+// envs per tile of the phased collision, likewise
+__host__ __device__ inline int collide_tile_envs(const gsr_model& m, int n, int envs_per_tile) {
+  return collide_waves(m) ? kWave / collide_lanes(m, n) : envs_per_tile;
+}
+// envs [b0, b0 + n) of the wavefront collision: one after the other, or four at a time where the model packs
+__device__ __forceinline__ void wave_collide_tile(const gsr_model& m, const gsr_state& s, int b0, int n, char* lds) {
+  if (n > 1 && collide_packs(m)) {
+    const int sub = threadIdx.x / 16;
+    for (int j = sub; j < n; j += 4) {
+      wave_collide<false, 16>(Env(m, s, b0 + j), lds + sizeof(float) * wave_collide_words(m.n_geoms) * sub);
+      __syncthreads();
+    }
+  } else {
+    for (int j = 0; j < n; j++) {
+      wave_collide(Env(m, s, b0 + j), lds);
+      __syncthreads();
+    }
+  }
+}
 
 // an env whose narrowphase deferred pairs to the GJK/EPA pass: its contact list and rows are completed there
 __device__ __forceinline__ bool gjk_pending(const Env& e) { return e.I(e.s.gjk_defer_n, 0) > 0; }
@@ -101,15 +120,17 @@ struct BatchHeader {
   uint32_t counter, done;  // work queue: next tile, finished workgroups (the last one resets both)
   int32_t n_wave_tiles;    // tiles of the phased launch's wavefront-per-env stages (GJK/EPA pass, solve)
   int32_t n_dyn_tiles;     // tiles of the phased launch's dynamics stages (step_1, step_2)
-  int32_t pad0, pad1;
+  int32_t n_collide_tiles; // tiles of the phased launch's collision
+  int32_t pad0;
 };
-// A group's envs cut into tiles three times: envs_per_tile for the single fused kernel and the phased collision;
-// wave_envs_per_tile for the phased GJK/EPA pass and solve, whose wavefront variants take a tile's envs one after
-// the other (a lane-per-env collision wants 64 envs a tile, a wavefront solve few); and dyn_envs_per_tile for the phased
-// dynamics, as many envs as their wavefront serves at once (dyn_tile_envs)
+// A group's envs cut into tiles four times: envs_per_tile for the single fused kernel; wave_envs_per_tile for the phased
+// GJK/EPA pass and solve, whose wavefront variants take a tile's envs one after the other; and dyn_envs_per_tile and
+// collide_envs_per_tile for the phased dynamics and collision, as many envs as their wavefront serves at once
+// (dyn_tile_envs, collide_tile_envs)
 struct BatchRange {
   int32_t type, env_begin, n_envs, envs_per_tile, tile_begin, tile_end;
   int32_t wave_envs_per_tile, wave_tile_begin, wave_tile_end, dyn_envs_per_tile, dyn_tile_begin, dyn_tile_end;
+  int32_t collide_envs_per_tile, collide_tile_begin, collide_tile_end;
 };
 struct FusedTypes {
   gsr_model m[GSR_MAX_TYPES];
@@ -213,7 +234,7 @@ template <int P>
 __device__ __forceinline__ void phase_tile(const gsr_model& m, const gsr_state& s, int env0, int n_here, char* lds) {
   const int lane = threadIdx.x;
   const bool mine = lane < n_here;
-  const bool wave = P == 0 || P == 4 ? m.dyn_variant == 1 : P == 1 ? m.collide_variant == 1 : P == 3 ? m.solver_variant == 1 : true;
+  const bool wave = P == 0 || P == 4 ? m.dyn_variant == 1 : P == 1 ? collide_waves(m) : P == 3 ? m.solver_variant == 1 : true;
   if (!wave) {
     if (!mine) return;
     Env e(m, s, env0 + lane);
@@ -235,13 +256,16 @@ __device__ __forceinline__ void phase_tile(const gsr_model& m, const gsr_state& 
     wave_step1(m, s, env0, n_here, lds);
     return;
   }
+  if (P == 1) {
+    wave_collide_tile(m, s, env0, n_here, lds);
+    return;
+  }
   if (P == 4) {
     wave_step2<false>(m, s, env0, n_here, lds);
     return;
   }
   for (int j = 0; j < n_here; j++) {
     Env e(m, s, env0 + j);
-    if (P == 1) wave_collide(e, lds);
     if (P == 2 && wave_gjk_fixup(e)) wave_rows(e);
     if (P == 3) wave_solve(e, lds);
     __syncthreads();
@@ -256,18 +280,18 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 8
   ConstTypes* types = (ConstTypes*)(table + kTypesOffset);
   const BatchRange* __restrict__ R = reinterpret_cast<const BatchRange*>(table + kRangesOffset);
   constexpr bool kWaveTiles = P == 2 || P == 3, kDynTiles = P == 0 || P == 4;
-  const int n_tiles = kWaveTiles ? H->n_wave_tiles : kDynTiles ? H->n_dyn_tiles : H->n_tiles, n_groups = H->n_groups;
+  const int n_tiles = kWaveTiles ? H->n_wave_tiles : kDynTiles ? H->n_dyn_tiles : H->n_collide_tiles, n_groups = H->n_groups;
   if ((int)blockIdx.x >= n_tiles) return;
   const int tile = xcd_env(blockIdx.x, n_tiles);
   int lo = 0, hi = n_groups - 1;
   while (lo < hi) {
     int mid = (lo + hi) >> 1;
-    if (tile < (kWaveTiles ? R[mid].wave_tile_end : kDynTiles ? R[mid].dyn_tile_end : R[mid].tile_end)) hi = mid;
+    if (tile < (kWaveTiles ? R[mid].wave_tile_end : kDynTiles ? R[mid].dyn_tile_end : R[mid].collide_tile_end)) hi = mid;
     else lo = mid + 1;
   }
   const BatchRange g = R[lo];
-  const int T = kWaveTiles ? g.wave_envs_per_tile : kDynTiles ? g.dyn_envs_per_tile : g.envs_per_tile;
-  const int first = (tile - (kWaveTiles ? g.wave_tile_begin : kDynTiles ? g.dyn_tile_begin : g.tile_begin)) * T;
+  const int T = kWaveTiles ? g.wave_envs_per_tile : kDynTiles ? g.dyn_envs_per_tile : g.collide_envs_per_tile;
+  const int first = (tile - (kWaveTiles ? g.wave_tile_begin : kDynTiles ? g.dyn_tile_begin : g.collide_tile_begin)) * T;
   const int n_here = min(T, g.n_envs - first);
   const int k = __builtin_amdgcn_readfirstlane(g.type);
   const FusedTypes* ty = (const FusedTypes*)types;

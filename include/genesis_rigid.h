@@ -54,7 +54,9 @@ typedef struct gsr_model {
   int32_t iterations, ls_iterations, n_contacts_per_pair;
   int32_t enable_collision, enable_joint_limit, enable_multi_contact;
   int32_t solver_variant;  /* 0: one lane per env (rows env-minor), 1: one wavefront per env (rows env-major) */
-  int32_t collide_variant; /* 0: one lane per env, 1: one wavefront per env (pairs across lanes) */
+  int32_t collide_variant; /* the single fused kernel's collision: 0 one lane per env, 1 one wavefront per env (pairs
+                              across lanes). The plain and phased steps take 64 or 16 lanes per env by size; a lane per
+                              env only where 0 is set and the model has more than 1,018 geoms */
   int32_t dyn_variant;     /* step_1 / step_2: 0 one lane per env, 1 one wavefront per env (entities across lanes) */
   int32_t batch_dofs;      /* 1: dof_kp, dof_kv, dof_force_range, dof_stiffness, dof_damping, dof_frictionloss,
                               dof_limit, dof_armature and dof_invweight hold one value per env, env-minor like the state
@@ -235,7 +237,7 @@ typedef struct gsr_group {
 
 typedef struct gsr_batch_info {
   int32_t n_groups, n_tiles; /* groups and tiles in the batch */
-  int32_t grid;              /* workgroups per launch (phased: of the dynamics stages) */
+  int32_t grid;              /* workgroups per launch (phased: of the dynamics and collision stages) */
   int32_t lds_bytes;         /* dynamic LDS per workgroup (largest wavefront-variant group) */
   int32_t n_types;           /* distinct (model, state) pairs, in first-appearance order */
   int32_t persistent;        /* input: 1 = CUs x resident workgroups pull tiles from a queue, 0 = one per tile */

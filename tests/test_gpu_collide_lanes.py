@@ -1,0 +1,62 @@
+"""Collision with 16 lanes per env (many envs of a small model), 64 lanes, and one lane per env (the single fused kernel's
+variant 0) give the same bits, also where the broadphase buffer overflows."""
+import numpy as np
+import pytest
+import torch
+
+from genesis_amd import workloads as W
+from genesis_amd.model import CompileOptions, compile_model
+from tests.test_gpu_bodies import stacks
+
+pytestmark = pytest.mark.gpu
+
+COMPARED = ["qpos", "vel", "n_con", "n_contacts", "n_broad", "broad_pairs", "contact_geoms", "contact_pos", "contact_normal",
+            "contact_pen", "cache_normal", "sort_value", "sort_ig", "aabb_min", "aabb_max", "errno_env"]
+B = 2051  # 513 wavefronts of four envs, the last one partly filled
+
+
+@pytest.mark.parametrize("name,pairs", [("quadruped", 300), ("arm", 300), ("boxes", 300), ("boxes", 1)])
+def test_collision_lanes_agree(name, pairs):
+    from genesis_amd.batch import FusedBatch, Group
+    from genesis_amd.rigid_solver import RigidSolver
+    if name == "boxes":
+        ents, q = stacks(7, 41, 5)
+    else:
+        ents = [W.plane_entity(), W.go2_entity() if name == "quadruped" else W.panda_entity()]
+    M = compile_model(ents, CompileOptions(dt=0.005, max_collision_pairs=pairs))
+    if name != "boxes":
+        rng = np.random.default_rng(2)
+        q = np.tile(np.asarray(M.qpos0, np.float64), (41, 1))
+        if name == "quadruped":
+            q[:, 2] = rng.uniform(0.05, 0.4, 41)  # from lying to hanging in the air
+            q[:, 7:] += rng.uniform(-0.3, 0.3, (41, M.n_qs - 7))
+        else:
+            q[:, 1] = rng.uniform(1.2, 1.7, 41)  # the hand reaches the ground or stays clear of it
+            q[:, 3] = rng.uniform(-0.3, -0.1, 41)
+    q = torch.as_tensor(np.tile(q, (B // 41 + 1, 1))[:B], dtype=torch.float32)
+    many, few, lane = (RigidSolver(M, n, "cuda", solver_variant=1, collide_variant=v, dyn_variant=1)
+                       for n, v in ((B, 1), (41, 1), (41, 0)))
+    for S in (many, few, lane):
+        S.set_qpos(q[:S._B])
+    fb = FusedBatch([Group(lane, envs_per_tile=1, solver_variant=1, collide_variant=0)])
+    seen = 0
+    for _ in range(3):
+        many.substep()
+        few.substep()
+        fb.step()
+        torch.cuda.synchronize()
+        seen = max(seen, int(few.st.t["n_contacts"][0].max()))
+        for k in COMPARED:
+            a, b, c = (S.st.t[k] for S in (many, few, lane))
+            if k in ("broad_pairs", "contact_geoms", "contact_pos", "contact_normal", "contact_pen"):
+                # entries beyond an env's count are left over from earlier steps
+                n = few.st.t["n_broad" if k == "broad_pairs" else "n_contacts"][0].long()
+                per = {"broad_pairs": 1, "contact_geoms": 2, "contact_pos": 3, "contact_normal": 3, "contact_pen": 1}[k]
+                keep = torch.arange(b.shape[0], device=b.device)[:, None] < per * n[None]
+                a, b, c = (torch.where(keep, x[:, :41], torch.zeros_like(x[:, :41])) for x in (a, b, c))
+            assert torch.equal(b, c), f"{k}: 64 lanes and one lane differ"
+            assert torch.equal(a[..., :41], b), f"{k}: 16 and 64 lanes differ"
+            if a.shape[-1] == B:
+                assert torch.equal(a[..., 41:82], a[..., :41]) and torch.equal(a[..., -1], a[..., (B - 1) % 41]), k
+    assert seen > 0
+    assert bool((few.st.t["errno_env"] & 1).any()) == (pairs == 1)
