@@ -2,12 +2,12 @@
 //
 // Plain drop-in form: one substep = four stages launched in stream order over env-minor SoA state (consecutive lanes
 // or workgroups touch consecutive envs for every per-env field):
-//   step_1     smooth dynamics (kernel_step_1): k_step1 (one lane per env) or k_step1_wave (one wavefront per env)
+//   step_1     smooth dynamics (kernel_step_1): k_step1_tree, or k_step1 where an entity is one lane's
 //   collision  equality rows, AABBs, sweep-and-prune, narrowphase, inequality rows (_func_constraint_force):
 //              k_collide / k_collide_wave, then the GJK/EPA pass k_gjk_fixup (rigid_k_collide.hip)
 //   solve      Newton solve + qacc/contact-force epilogue (ConstraintSolver.resolve): k_solve / k_solve_wave
 //              (rigid_k_solve.hip)
-//   step_2     integration, NaN-guarded commit, end-of-step kinematics (kernel_step_2): k_step2 / k_step2_wave
+//   step_2     integration, NaN-guarded commit, end-of-step kinematics (kernel_step_2): k_step2_tree / k_step2
 // This unit holds step_1, step_2, the kinematics refresh, resets and readback kernels and every C-ABI entry point;
 // the batching form's kernels live in rigid_k_fused_*.hip, rigid_k_phase_*.hip and rigid_k_resume.hip.
 #include <hip/hip_runtime.h>
@@ -24,24 +24,51 @@ using namespace gsr;
 
 namespace {
 
-__global__ void __launch_bounds__(kBlock) k_kinematics(gsr_model m, gsr_state s, const int32_t* envs_idx, int n_idx) {
-  int t = env_id();
-  if (t >= n_idx) return;
-  int b = envs_idx ? envs_idx[t] : t;
-  if (b < 0 || b >= s.n_envs) return;
-  Env e(m, s, b);
-  dev_kinematics(e);
-  if (m.enable_collision) dev_update_aabbs(e);
+// Dynamics and kinematics that walk each entity on one lane (free bodies; articulated entities that the tree kernels do not
+// take): a workgroup holds `envs` envs with 512 / envs entities of each at a time, the env fastest. State is env-minor, so
+// a wavefront reads a run of envs of one array element, and an entity's long dependent walk is one lane's. E grows with the
+// env count (whole 128-byte lines) and L with the entities, down to a lane per env for a single robot.
+// Measured (us, step_1, step_2, kinematics; a wavefront per env or, in the kinematics, a lane -> this): 4,096 64-box piles
+// 1138 -> 315, 528 -> 106, 799 -> 73; 96 of them 157 -> 155, 61 -> 60, 780 -> 44; 1,500 20-box piles 116 -> 78, 54 -> 35,
+// 273 -> 46; 100 7-box piles 60 -> 63, 27 -> 26, 99 -> 21.
+struct EntitySplit {
+  int envs, lanes;  // powers of two
+};
+EntitySplit entity_split(const gsr_model& m, int n) {
+  EntitySplit x{1, 1};
+  while (m.n_entities > 2 && x.lanes < m.n_entities && x.lanes < 64) x.lanes *= 2;
+  while (x.envs < 64 && (x.envs * x.lanes < kWave || x.envs * 2 * 256 <= n)) x.envs *= 2;
+  x.lanes = std::min(x.lanes, 512 / x.envs);
+  return x;
+}
+struct EntityLane {
+  int sub, lane, t;  // env of the workgroup, entity lane, env of the launch
+  __device__ EntityLane(int envs, int n)
+      : sub(threadIdx.x % envs), lane(threadIdx.x / envs), t(xcd_env(blockIdx.x, (n + envs - 1) / envs) * envs + sub) {}
+};
+
+__global__ void __launch_bounds__(512) k_kinematics(gsr_model m, gsr_state s, const int32_t* envs_idx, int n_idx, int envs,
+                                                    int lanes) {
+  const EntityLane x(envs, n_idx);
+  const int b = x.t >= n_idx ? -1 : envs_idx ? envs_idx[x.t] : x.t;
+  const bool on = b >= 0 && b < s.n_envs;
+  Env e(m, s, on ? b : 0);
+  if (on) {
+    dev_forward_kinematics(e, x.lane, lanes);
+    dev_com_links(e, x.lane, lanes);
+  }
+  __syncthreads();
+  if (on) {
+    dev_update_geoms(e, x.lane, lanes);
+    if (m.enable_collision) dev_update_aabbs(e, x.lane, lanes);
+    dev_forward_velocity(e, x.lane, lanes);
+  }
 }
 
-__global__ void __launch_bounds__(kBlock) k_step1(gsr_model m, gsr_state s, int refresh_kinematics) {
-  int b = env_id();
-  if (b >= s.n_envs) return;
-  Env e(m, s, b);
-  if (refresh_kinematics) dev_kinematics(e);
-  dev_smooth_dynamics(e);
+__global__ void __launch_bounds__(512) k_step1(gsr_model m, gsr_state s, int envs, int lanes) {
+  const EntityLane x(envs, s.n_envs);
+  if (x.t < s.n_envs) dev_smooth_dynamics(Env(m, s, x.t), x.lane, lanes);
 }
-
 
 // G lanes per env: the lanes share an articulated env's tree ...
 template <int G>
@@ -76,7 +103,7 @@ __global__ void __launch_bounds__(kWave) k_kinematics_tree(gsr_model m, gsr_stat
   Env e(m, s, b);
   tree_refresh<G>(e, t, p);
   __syncthreads();
-  if (m.enable_collision) wave_update_aabbs<G>(e, threadIdx.x & (G - 1));
+  if (m.enable_collision) dev_update_aabbs(e, threadIdx.x & (G - 1), G);
 }
 
 template <class K16, class K64, class... Args>
@@ -88,22 +115,25 @@ void launch_tree(K16 k16, K64 k64, const gsr_model& m, int n, hipStream_t st, Ar
 }
 
 // ... and take the entities of an env of free bodies
-__global__ void __launch_bounds__(kWave) k_step1_wave(gsr_model m, gsr_state s) {
-  if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
-  dev_smooth_dynamics(Env(m, s, xcd_env(blockIdx.x, s.n_envs)), threadIdx.x, kWave);
-}
-
-__global__ void __launch_bounds__(kWave) k_step2_wave(gsr_model m, gsr_state s) {
-  if ((int)blockIdx.x >= s.n_envs) return;  // uniform across the block
-  wave_step2_entities(Env(m, s, xcd_env(blockIdx.x, s.n_envs)));
-}
-
-__global__ void __launch_bounds__(kBlock) k_step2(gsr_model m, gsr_state s) {
-  int b = env_id();
-  if (b >= s.n_envs) return;
-  Env e(m, s, b);
-  dev_integrate(e);
-  dev_kinematics(e);
+__global__ void __launch_bounds__(512) k_step2(gsr_model m, gsr_state s, int envs, int lanes) {
+  __shared__ int nan[64];  // envs with a NaN
+  const EntityLane x(envs, s.n_envs);
+  const bool on = x.t < s.n_envs;
+  Env e(m, s, on ? x.t : 0);
+  if (x.lane == 0) nan[x.sub] = 0;
+  __syncthreads();
+  if (on && !dev_integrate_next(e, x.lane, lanes)) nan[x.sub] = 1;
+  __syncthreads();
+  if (on) {
+    dev_integrate_commit(e, x.lane, lanes, nan[x.sub] == 0, x.lane == 0);
+    dev_forward_kinematics(e, x.lane, lanes);
+    dev_com_links(e, x.lane, lanes);
+  }
+  __syncthreads();
+  if (on) {
+    dev_update_geoms(e, x.lane, lanes);
+    dev_forward_velocity(e, x.lane, lanes);
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) k_reset(gsr_model m, gsr_state s, const int32_t* envs_idx, int n_idx,
@@ -248,23 +278,27 @@ int launch_status() {
 
 inline dim3 grid_for(int n) { return dim3((n + kBlock - 1) / kBlock); }
 
+template <typename K, typename... A>
+void launch_entities(K kernel, const gsr_model& m, int n, hipStream_t st, A... args) {
+  const EntitySplit x = entity_split(m, n);
+  hipLaunchKernelGGL(kernel, dim3((n + x.envs - 1) / x.envs), dim3(x.envs * x.lanes), 0, st, args..., x.envs, x.lanes);
+}
+
 // kinematics of n listed envs (all when idx is null); an articulated env takes a wavefront whatever the step's variant
 void launch_kinematics(const gsr_model& m, const gsr_state& s, const int32_t* idx, int n, hipStream_t st) {
   if (tree_dynamics(m))
     launch_tree(k_kinematics_tree<16>, k_kinematics_tree<kWave>, m, n, st, m, s, idx, n);
   else
-    hipLaunchKernelGGL(k_kinematics, grid_for(n), dim3(kBlock), 0, st, m, s, idx, n);
+    launch_entities(k_kinematics, m, n, st, m, s, idx, n);
 }
 
 void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
-  dim3 g = grid_for(s->n_envs);
   switch (k) {
     // kinematics of the current pose are refreshed at the end of every step (and by gsr_forward_kinematics after a
     // pose write), so kernel_step_1 never needs to recompute them (enable_mujoco_compatibility = False)
     case 0:
       if (dyn_lds_bytes(*m)) launch_tree(k_step1_tree<16>, k_step1_tree<kWave>, *m, s->n_envs, st, *m, *s);
-      else if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step1_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
-      else hipLaunchKernelGGL(k_step1, g, dim3(kBlock), 0, st, *m, *s, 0);
+      else launch_entities(k_step1, *m, s->n_envs, st, *m, *s);
       break;
     case 1:
       launch_collide(*m, *s, st);
@@ -274,8 +308,7 @@ void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
       break;
     default:
       if (dyn_lds_bytes(*m)) launch_tree(k_step2_tree<16>, k_step2_tree<kWave>, *m, s->n_envs, st, *m, *s);
-      else if (m->dyn_variant == 1) hipLaunchKernelGGL(k_step2_wave, dim3(s->n_envs), dim3(kWave), 0, st, *m, *s);
-      else hipLaunchKernelGGL(k_step2, g, dim3(kBlock), 0, st, *m, *s);
+      else launch_entities(k_step2, *m, s->n_envs, st, *m, *s);
       break;
   }
 }

@@ -16,10 +16,11 @@ constexpr int kCcdIters = 50;
 // The reference's portal-refinement loops are unbounded; this cap only guards pathological inputs on the GPU.
 constexpr int kMprLoopCap = 1000;
 
-__device__ inline void dev_update_aabbs(const Env& e) {
+// geoms g0, g0 + gs, ...; box: copies of the AABBs (minimum, maximum per geom) in LDS, or null
+__device__ inline void dev_update_aabbs(const Env& e, int g0 = 0, int gs = 1, float* box = nullptr) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  for (int g = 0; g < m.n_geoms; g++) {
+  for (int g = g0; g < m.n_geoms; g += gs) {
     f3 gp = e.L3(s.geoms_pos, g);
     q4 gq = e.L4(s.geoms_quat, g);
     f3 lo{INFINITY, INFINITY, INFINITY}, hi{-INFINITY, -INFINITY, -INFINITY};
@@ -30,6 +31,10 @@ __device__ inline void dev_update_aabbs(const Env& e) {
     }
     e.S3(s.aabb_min, g, lo);
     e.S3(s.aabb_max, g, hi);
+    if (box) {
+      const float v[6] = {lo.x, lo.y, lo.z, hi.x, hi.y, hi.z};
+      for (int q = 0; q < 6; q++) box[6 * g + q] = v[q];
+    }
   }
 }
 

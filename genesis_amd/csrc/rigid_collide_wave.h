@@ -65,29 +65,6 @@ __host__ __device__ inline bool collide_packs(const gsr_model& m) { return m.n_e
 // 4213, 172, 354; 4,000: 4437, 403, 448; 64 boxes 1,024: 25968, 566, 1529.
 __host__ __device__ inline int collide_lanes(const gsr_model& m, int n) { return n > 2048 && collide_packs(m) ? 16 : kWave; }
 
-// box: copies of the AABBs (minimum, maximum per geom) in LDS, or null
-template <int G = 64>
-__device__ inline void wave_update_aabbs(const Env& e, int lane, float* box = nullptr) {
-  const gsr_model& m = e.m;
-  const gsr_state& s = e.s;
-  for (int g = lane; g < m.n_geoms; g += G) {
-    f3 gp = e.L3(s.geoms_pos, g);
-    q4 gq = e.L4(s.geoms_quat, g);
-    f3 lo{INFINITY, INFINITY, INFINITY}, hi{-INFINITY, -INFINITY, -INFINITY};
-    for (int c = 0; c < 8; c++) {
-      f3 p = xform(T3(m.geom_init_aabb, 8 * g + c), gp, gq);
-      lo = vmin(lo, p);
-      hi = vmax(hi, p);
-    }
-    e.S3(s.aabb_min, g, lo);
-    e.S3(s.aabb_max, g, hi);
-    if (box) {
-      const float v[6] = {lo.x, lo.y, lo.z, hi.x, hi.y, hi.z};
-      for (int q = 0; q < 6; q++) box[6 * g + q] = v[q];
-    }
-  }
-}
-
 template <int W>
 __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   const gsr_model& m = e.m;
@@ -345,7 +322,7 @@ __device__ __forceinline__ void wave_collide(const Env& e, char* lds) {
     e.I(s.gjk_defer_n, 0) = 0;
   }
   if (m.enable_collision) {
-    wave_update_aabbs<W>(e, lane, reinterpret_cast<float*>(lds) + 10 * m.n_geoms);
+    dev_update_aabbs(e, lane, W, reinterpret_cast<float*>(lds) + 10 * m.n_geoms);
     __syncthreads();
     if (m.n_pairs > 0) {
       wave_broad_phase<W>(e, lds, lane);
