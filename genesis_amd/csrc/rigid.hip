@@ -846,15 +846,18 @@ int gsr_serve_tick(void* dev_state, void* dev_table, const gsr_batch_info* info,
   gsr_serve_host* hd = nullptr;
   if (hipHostGetDevicePointer((void**)&hd, host, 0) != hipSuccess || !hd) return GSR_E_ARG;
   const int n_tiles = info->n_tiles;
-  launch_serve(0, dev_state, dev_table, hd, n_tiles, stream);
-  launch_serve(1, dev_state, dev_table, hd, n_tiles, stream);
-  launch_serve(2, dev_state, dev_table, hd, n_tiles, stream);
+  size_t init_lds = 0;  // the kinematics of the reset envs
+  for (int k = 0; k < info->n_types; k++)
+    if (tree_dynamics(info->models[k])) init_lds = std::max(init_lds, tree_lds_bytes(info->models[k], kWave));
+  launch_serve(0, dev_state, dev_table, hd, n_tiles, (unsigned)init_lds, stream);
+  launch_serve(1, dev_state, dev_table, hd, n_tiles, (unsigned)init_lds, stream);
+  launch_serve(2, dev_state, dev_table, hd, n_tiles, (unsigned)init_lds, stream);
   const int n = gsr_fused_kernel_count(info);
   for (int k = 0; k < n; k++) {
     const int rc = gsr_launch_fused_kernel(dev_table, info, k, stream);
     if (rc) return rc;
   }
-  launch_serve(3, dev_state, dev_table, hd, n_tiles, stream);
+  launch_serve(3, dev_state, dev_table, hd, n_tiles, (unsigned)init_lds, stream);
   return launch_status();
 }
 

@@ -369,6 +369,6 @@ size_t serve_table_bytes(int n_tiles);
 int serve_init(const gsr_serve_pool* pools, int n_pools, double mem_budget, double tick_budget, void* dev_state,
                int64_t state_bytes, void* dev_table, int64_t table_bytes, hipStream_t stream);
 void launch_serve(int stage, void* dev_state, void* dev_table, gsr_serve_host* host_dev, int n_tiles,
-                  hipStream_t stream);
+                  unsigned init_lds, hipStream_t stream);
 
 }  // namespace gsr
