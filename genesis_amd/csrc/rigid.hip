@@ -551,7 +551,10 @@ static int phase_lds(const gsr_batch_info& b, int phase) {
   for (int k = 0; k < b.n_types; k++) {
     const gsr_model& m = b.models[k];
     // room for tiles of several envs: a group's tile size is not known here
-    if (phase == 1 && collide_waves(m)) lds = std::max(lds, wave_collide_lds_bytes(m.n_geoms, collide_packs(m) ? 4 : 1));
+    if (phase == 1 && collide_waves(m)) {
+      lds = std::max(lds, wave_collide_lds_bytes(m.n_geoms));
+      if (collide_packs(m)) lds = std::max(lds, wave_collide_lds_bytes(m.n_geoms, 16));
+    }
     if (phase == 0 || phase == 4) lds = std::max(lds, dyn_lds_bytes(m, kWave));
     if (phase == 3 && m.solver_variant == 1)
       lds = std::max(lds, (size_t)solve_lds_bytes(m));

@@ -407,107 +407,123 @@ __device__ inline void dev_contact_orthogonals(const Env& e, int ga, int gb, f3 
   a1 = cross(normal, a0);
 }
 
-// func_convex_convex_contact (collider_decomp.py:2328-2725); MPR path with multi-contact
+// func_convex_convex_contact (collider_decomp.py:2328-2725); MPR path with multi-contact: one detection in the pair's own
+// poses, then four with both geoms turned about two axes through the first contact
+struct Detection {
+  bool is_col;
+  float pen;
+  f3 normal, pos;
+};
+__device__ __forceinline__ bool dev_multi_contact(const gsr_model& m, int ga, int gb) {
+  const int ta = m.geom_type[ga], tb = m.geom_type[gb];
+  return m.enable_multi_contact && ta != GEOM_SPHERE && ta != GEOM_ELLIPSOID && tb != GEOM_SPHERE && tb != GEOM_ELLIPSOID;
+}
+__device__ __forceinline__ int dev_pair_index(const gsr_model& m, int ga, int gb) {
+  return m.pair_idx[(size_t)min(ga, gb) * m.n_geoms + max(ga, gb)];
+}
+// one detection; cache: the pair's normal cache. Returns false where the pair needs GJK/EPA and snk has no workspace for it.
+template <class Sink>
+__device__ inline bool dev_detect(const Env& e, int ga, int gb, const GPose& A, const GPose& Bp, bool first, f3 cache,
+                                  float tol, Sink& snk, Detection& o) {
+  const gsr_model& m = e.m;
+  const float EPS = m.eps;
+  if (m.geom_type[ga] == GEOM_PLANE) {
+    f3 pd = qrot(f3{m.geom_data[7 * ga], m.geom_data[7 * ga + 1], m.geom_data[7 * ga + 2]}, A.q);
+    o.normal = -normalized(pd);
+    f3 v1 = dev_support(m, gb, Bp, o.normal);
+    o.pen = dot(o.normal, v1 - A.p);
+    o.pos = v1 - 0.5f * o.pen * o.normal;
+    o.is_col = o.pen > 0.f;
+    return true;
+  }
+  f3 nws = cache;
+  bool guess = fabsf(nws.x) > EPS || fabsf(nws.y) > EPS || fabsf(nws.z) > EPS;
+  // the first detection that misses from the cached normal is repeated without it
+  for (int im = 0; im < 2; im++) {
+    if (im == 1) {
+      if (!(first && !o.is_col && guess)) break;
+      nws = zero3();
+      guess = false;
+    }
+    dev_mpr_contact(m, ga, gb, A, Bp, nws, o.is_col, o.normal, o.pen, o.pos);
+  }
+  if (o.pen > tol) {
+    bool prefer_gjk = !guess || (m.mc_tolerance * o.pen >= m.mpr_to_gjk * tol);
+    if (prefer_gjk) {
+      if (!snk.gjk_allowed()) return false;
+      snk.flag(GSR_ERR_DEEP_PENETRATION);
+      float gpen;
+      f3 gn, gp;
+      o.is_col = dev_gjk_contact(m, gjk_ws(e), ga, gb, A, Bp, gpen, gn, gp);
+      o.pen = gpen;
+      if (o.is_col) {
+        o.pos = gp;
+        o.normal = gn;
+      }
+    }
+  }
+  return true;
+}
+// poses of detection det (1..4), both geoms turned by opposite halves about an axis through cp0; returns the rotation
+__device__ __forceinline__ q4 dev_perturb(const gsr_model& m, int det, f3 cp0, f3 ax0, f3 ax1, GPose& A, GPose& Bp) {
+  f3 axis = (float)(2 * (det % 2) - 1) * ax0 + (float)(1 - 2 * ((det / 2) % 2)) * ax1;
+  q4 qr = rotvec_to_quat(m.mc_perturbation * axis, m.eps);
+  dev_rotate_frame(A, cp0, qr);
+  dev_rotate_frame(Bp, cp0, qinv(qr));
+  return qr;
+}
+// a contact of turned poses back in the pair's own
+__device__ __forceinline__ void dev_unperturb(const gsr_model& m, Detection& o, q4 qr, f3 cp0, f3 n0) {
+  f3 cpa = qrot((o.pos - 0.5f * o.pen * o.normal) - cp0, qinv(qr)) + cp0;
+  f3 cpb = qrot((o.pos + 0.5f * o.pen * o.normal) - cp0, qr) + cp0;
+  o.pos = 0.5f * (cpa + cpb);
+  f3 tw = cross(o.normal, n0);
+  float mp = m.mc_perturbation;
+  tw = f3{fminf(fmaxf(tw.x, -mp), mp), fminf(fmaxf(tw.y, -mp), mp), fminf(fmaxf(tw.z, -mp), mp)};
+  o.normal = o.normal + cross(tw, o.normal);
+  o.pen = dot(o.normal, cpb - cpa);
+}
+
 template <class Sink>
 __device__ inline void dev_convex_convex(const Env& e, int ga, int gb, Sink& snk) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  const float EPS = m.eps;
-  int ta = m.geom_type[ga], tb = m.geom_type[gb];
-  bool multi = m.enable_multi_contact && ta != GEOM_SPHERE && ta != GEOM_ELLIPSOID && tb != GEOM_SPHERE && tb != GEOM_ELLIPSOID;
-  float tol = dev_tolerance(m, ga, gb, m.mc_tolerance);
+  const bool multi = dev_multi_contact(m, ga, gb);
+  const float tol = dev_tolerance(m, ga, gb, m.mc_tolerance);
   const GPose A0{e.L3(s.geoms_pos, ga), e.L4(s.geoms_quat, ga)};
   const GPose B0{e.L3(s.geoms_pos, gb), e.L4(s.geoms_quat, gb)};
-  bool is_col0 = false, is_col = false;
-  float pen0 = 0.f, pen = 0.f;
-  f3 n0 = zero3(), cp0 = zero3(), normal = zero3(), cpos = zero3(), ax0 = zero3(), ax1 = zero3();
-  q4 qr{0.f, 0.f, 0.f, 0.f};
-  int n_con = 0;
-  int gmin = ga < gb ? ga : gb, gmax = ga < gb ? gb : ga;
-  int i_pair = m.pair_idx[(size_t)gmin * m.n_geoms + gmax];
-  // the pair's normal cache, read once and written back at the end (det 0 sets it, later detections read it)
+  const int i_pair = dev_pair_index(m, ga, gb);
+  // the pair's normal cache, read once and written back at the end (the first detection sets it, later ones read it)
   f3 cache = e.L3(s.cache_normal, i_pair);
+  f3 n0 = zero3(), cp0 = zero3(), ax0 = zero3(), ax1 = zero3();
+  int n_con = 0;
   for (int det = 0; det < 5; det++) {
     GPose A = A0, Bp = B0;
-    if (multi && is_col0) {
-      f3 axis = (float)(2 * (det % 2) - 1) * ax0 + (float)(1 - 2 * ((det / 2) % 2)) * ax1;
-      qr = rotvec_to_quat(m.mc_perturbation * axis, EPS);
-      dev_rotate_frame(A, cp0, qr);
-      dev_rotate_frame(Bp, cp0, qinv(qr));
-    }
-    if ((multi && is_col0) || det == 0) {
-      if (ta == GEOM_PLANE) {
-        f3 pd = qrot(f3{m.geom_data[7 * ga], m.geom_data[7 * ga + 1], m.geom_data[7 * ga + 2]}, A.q);
-        normal = -normalized(pd);
-        f3 v1 = dev_support(m, gb, Bp, normal);
-        pen = dot(normal, v1 - A.p);
-        cpos = v1 - 0.5f * pen * normal;
-        is_col = pen > 0.f;
-      } else {
-        bool updated = false;
-        f3 nws = cache;
-        bool guess = fabsf(nws.x) > EPS || fabsf(nws.y) > EPS || fabsf(nws.z) > EPS;
-        for (int im = 0; im < 2; im++) {
-          if (im == 1 && det == 0 && !is_col && guess) {
-            nws = zero3();
-            guess = false;
-            updated = false;
-          }
-          if (!updated) {
-            dev_mpr_contact(m, ga, gb, A, Bp, nws, is_col, normal, pen, cpos);
-            updated = true;
-          }
-        }
-        if (pen > tol) {
-          bool prefer_gjk = !guess || (m.mc_tolerance * pen >= m.mpr_to_gjk * tol);
-          if (prefer_gjk) {
-            if (!snk.gjk_allowed()) {
-              snk.defer(ga, gb);
-              return;
-            }
-            snk.flag(GSR_ERR_DEEP_PENETRATION);
-            float gpen;
-            f3 gn, gp;
-            is_col = dev_gjk_contact(m, gjk_ws(e), ga, gb, A, Bp, gpen, gn, gp);
-            pen = gpen;
-            if (is_col) {
-              cpos = gp;
-              normal = gn;
-            }
-          }
-        }
-      }
+    q4 qr{0.f, 0.f, 0.f, 0.f};
+    if (det > 0) qr = dev_perturb(m, det, cp0, ax0, ax1, A, Bp);
+    Detection o;
+    if (!dev_detect(e, ga, gb, A, Bp, det == 0, cache, tol, snk, o)) {
+      snk.defer(ga, gb);
+      return;
     }
     if (det == 0) {
-      is_col0 = is_col; n0 = normal; pen0 = pen; cp0 = cpos;
-      if (is_col0) {
-        snk.add(ga, gb, n0, cp0, pen0);
-        if (multi) {
-          dev_contact_orthogonals(e, ga, gb, normal, ax0, ax1);
-          n_con = 1;
-        }
-        cache = normal;
-      } else {
-        cache = zero3();
-      }
-    } else if (multi && is_col0 && is_col) {
-      f3 cpa = qrot((cpos - 0.5f * pen * normal) - cp0, qinv(qr)) + cp0;
-      f3 cpb = qrot((cpos + 0.5f * pen * normal) - cp0, qr) + cp0;
-      cpos = 0.5f * (cpa + cpb);
-      f3 tw = cross(normal, n0);
-      float mp = m.mc_perturbation;
-      tw = f3{fminf(fmaxf(tw.x, -mp), mp), fminf(fmaxf(tw.y, -mp), mp), fminf(fmaxf(tw.z, -mp), mp)};
-      normal = normal + cross(tw, normal);
-      pen = dot(normal, cpb - cpa);
+      cache = o.is_col ? o.normal : zero3();
+      if (o.is_col) snk.add(ga, gb, o.normal, o.pos, o.pen);
+      if (!o.is_col || !multi) break;
+      n0 = o.normal;
+      cp0 = o.pos;
+      dev_contact_orthogonals(e, ga, gb, n0, ax0, ax1);
+      n_con = 1;
+    } else if (o.is_col) {
+      dev_unperturb(m, o, qr, cp0, n0);
       bool repeated = false;
       for (int ic = 0; ic < n_con; ic++) {
         if (!repeated) {
-          if (norm(cpos - snk.recent_pos(ic)) < tol) repeated = true;
+          if (norm(o.pos - snk.recent_pos(ic)) < tol) repeated = true;
         }
       }
-      if (!repeated && pen > -tol) {
-        pen = fmaxf(pen, 0.f);
-        snk.add(ga, gb, normal, cpos, pen);
+      if (!repeated && o.pen > -tol) {
+        snk.add(ga, gb, o.normal, o.pos, fmaxf(o.pen, 0.f));
         n_con++;
       }
     }

@@ -44,10 +44,12 @@ __device__ __forceinline__ unsigned long long env_ballot(bool v) {
   else return (b >> (threadIdx.x & ~(W - 1))) & ((1ull << W) - 1ull);
 }
 
-// LDS words of one env
-__host__ __device__ inline size_t wave_collide_words(int G) { return 16 * (size_t)G + 4; }
-__host__ __device__ inline size_t wave_collide_lds_bytes(int G, int envs = 1) {
-  return sizeof(float) * wave_collide_words(G) * (size_t)envs + 64;
+// LDS words of one env: the sweep's arrays (16 a geom), then in their place the narrowphase's (32 a lane)
+__host__ __device__ inline size_t wave_collide_words(int G, int W) {
+  return (16 * (size_t)G > 32 * (size_t)W ? 16 * (size_t)G : 32 * (size_t)W) + 4;
+}
+__host__ __device__ inline size_t wave_collide_lds_bytes(int G, int W = 64) {
+  return sizeof(float) * wave_collide_words(G, W) * (size_t)(64 / W) + 64;
 }
 // Models whose collision the wavefront form holds (its LDS, its contact buffer of a pair): all that any scene here has. The
 // others take a lane per env.
@@ -62,7 +64,8 @@ __host__ __device__ inline bool collide_packs(const gsr_model& m) { return m.n_e
 // envs a wavefront are faster where the model packs. Measured (us, collision and GJK/EPA pass; one lane per env, 64, 16
 // lanes): quadrupeds 2,048: 576, 68, 68; 4,000: 585, 123, 80; 32,768: 824, 939, 374; arms 2,000: 707, 76, 89; 5,000: 726,
 // 120, 98; 7-box piles 1,024: 465, 58, 55; 4,000: 488, 122, 105; 16,384: 569, 491, 342. Heaps do not pack: 20 boxes 300:
-// 4213, 172, 354; 4,000: 4437, 403, 448; 64 boxes 1,024: 25968, 566, 1529.
+// 4213, 172, 354; 4,000: 4437, 403, 448; 64 boxes 1,024: 25968, 566, 1529 (heaps with a pair per lane throughout; wave_convex
+// has taken 15 to 40 % off their 64-lane figures since).
 __host__ __device__ inline int collide_lanes(const gsr_model& m, int n) { return n > 2048 && collide_packs(m) ? 16 : kWave; }
 
 template <int W>
@@ -174,94 +177,243 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
   __syncthreads();
 }
 
-// one pass over the broadphase pairs of one kind (convex pairs, then plane-box pairs), contacts appended at `base`
+// a contact of the env's list, or the overflow bit
+__device__ __forceinline__ void put_contact(const Env& e, int k, int ga, int gb, f3 n, f3 p, float pen, uint32_t& err) {
+  const gsr_model& m = e.m;
+  const gsr_state& s = e.s;
+  if (k >= m.max_contacts) {
+    err |= GSR_ERR_CONTACT_OVERFLOW;
+    return;
+  }
+  e.I(s.contact_geoms, 2 * k) = ga;
+  e.I(s.contact_geoms, 2 * k + 1) = gb;
+  e.S3(s.contact_normal, k, n);
+  e.S3(s.contact_pos, k, p);
+  e.F(s.contact_pen, k) = pen;
+  e.F(s.contact_friction, k) = fmaxf(fmaxf(m.geom_friction[ga] * e.F(s.friction_ratio, ga),
+                                           m.geom_friction[gb] * e.F(s.friction_ratio, gb)), 1e-2f);
+}
+// records of the pairs that need GJK/EPA, with the index their contacts go to
+template <int W>
+__device__ __forceinline__ void defer_pairs(const Env& e, int lane, bool deferred, int pr, int k, int& n_def) {
+  const unsigned long long def = env_ballot<W>(deferred);
+  if (deferred) {
+    const int slot = n_def + __popcll(def & ((1ull << lane) - 1ull));
+    e.I(e.s.gjk_defer, 2 * slot) = pr;
+    e.I(e.s.gjk_defer, 2 * slot + 1) = min(k, e.m.max_contacts);
+  }
+  n_def += __popcll(def);
+}
+// geoms of a pair in type order
+__device__ __forceinline__ void pair_geoms(const gsr_model& m, int pr, int& ga, int& gb) {
+  ga = pr >> 16;
+  gb = pr & 0xffff;
+  if (m.geom_type[ga] > m.geom_type[gb]) { int t = ga; ga = gb; gb = t; }
+}
+
+// Up to W pairs of one kind (q[lane], lane < cnt), a pair per lane, contacts appended at `base`.
 // kGjk: pairs that need GJK/EPA are redone in place, one lane at a time (they share the env's workspace), instead of
 // being deferred to the GJK/EPA pass
 template <bool kGjk, int W>
-__device__ inline int wave_narrow_pass(const Env& e, int lane, int nb, bool plane_box_pass, int base,
-                                       uint32_t& err, int& n_def) {
+__device__ inline int wave_pairs(const Env& e, int lane, const int* q, int cnt, bool plane_box, int base,
+                                 uint32_t& err) {
+  PairContacts pc;
+  pc.cnt = 0;
+  pc.err = 0;
+  pc.deferred = false;
+  int ga = 0, gb = 0;
+  if (lane < cnt) {
+    pair_geoms(e.m, q[lane], ga, gb);
+    LocalSink<false> snk{pc};
+    if (plane_box) dev_plane_box(e, ga, gb, snk);
+    else if constexpr (kGjk) dev_convex_convex(e, ga, gb, snk);
+  }
+  if constexpr (kGjk) {
+    unsigned long long redo = env_ballot<W>(pc.deferred);
+    while (redo) {
+      int j = __ffsll((long long)redo) - 1;
+      redo &= redo - 1;
+      if (lane == j) {
+        pc.cnt = 0;
+        pc.err = 0;
+        pc.deferred = false;
+        LocalSink<true> snk{pc};
+        dev_convex_convex(e, ga, gb, snk);
+      }
+    }
+  }
+  int total;
+  const int k = base + wave_excl_scan<W>(pc.cnt, lane, total);
+  for (int c = 0; c < pc.cnt; c++) put_contact(e, k + c, ga, gb, pc.n[c], pc.p[c], pc.pen[c], err);
+  err |= pc.err;
+  return base + total;
+}
+
+// Up to W convex pairs (q[lane], lane < cnt): the first detection with a pair per lane, then the turned detections of the
+// pairs that touch with a detection per lane, four lanes beside each other for a pair. They depend on the first alone,
+// except that a contact near an earlier one of its pair is dropped, which the four lanes settle among themselves. lds: 30 W
+// words; the turned contacts wait there, since in registers they made the fused kernel spill. What bounds it is the chain of support points of one detection: a pair's five in turn on its lane, with the
+// lanes of other pairs idle, were most of a heap's collision. Measured (us, collision and GJK/EPA pass, a pair per lane ->
+// this): 20-box piles 300: 172 -> 106, 1,500: 193 -> 145, 4,000: 403 -> 325; 1,024 64-box piles 566 -> 388.
+template <int W>
+__device__ inline int wave_convex(const Env& e, int lane, const int* q, int cnt, float* lds, int base, uint32_t& err,
+                                  int& n_def) {
   const gsr_model& m = e.m;
   const gsr_state& s = e.s;
-  for (int p0 = 0; p0 < nb; p0 += W) {
+  // of each touching pair: first contact, its normal and the two axes (12 words), then 7 words of each turned contact in
+  // their place; the pair's geoms in the last word
+  constexpr int kPair = 29;
+  int* count = reinterpret_cast<int*>(lds + kPair * W);  // which turned contacts stay (4 bits, -1: deferred), first index << 4
+  PairContacts none;
+  LocalSink<false> snk{none};
+  int ga = 0, gb = 0;
+  Detection o;
+  o.is_col = false;
+  bool deferred = false, turn = false;
+  f3 ax0 = zero3(), ax1 = zero3();
+  if (lane < cnt) {
+    pair_geoms(m, q[lane], ga, gb);
+    const GPose A{e.L3(s.geoms_pos, ga), e.L4(s.geoms_quat, ga)}, Bp{e.L3(s.geoms_pos, gb), e.L4(s.geoms_quat, gb)};
+    deferred = !dev_detect(e, ga, gb, A, Bp, true, e.L3(s.cache_normal, dev_pair_index(m, ga, gb)),
+                           dev_tolerance(m, ga, gb, m.mc_tolerance), snk, o);
+    turn = !deferred && o.is_col && dev_multi_contact(m, ga, gb);
+    if (turn) dev_contact_orthogonals(e, ga, gb, o.normal, ax0, ax1);
+  }
+  const unsigned long long turned = env_ballot<W>(turn);
+  const int n_turn = __popcll(turned), rank = __popcll(turned & ((1ull << lane) - 1ull));
+  __syncthreads();
+  if (turn) {
+    const float v[12] = {o.pos.x, o.pos.y, o.pos.z, o.normal.x, o.normal.y, o.normal.z, ax0.x, ax0.y, ax0.z, ax1.x, ax1.y, ax1.z};
+    for (int j = 0; j < 12; j++) lds[kPair * rank + j] = v[j];
+    lds[kPair * rank + 28] = __int_as_float(q[lane]);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int t0 = 0; t0 < 4 * n_turn; t0 += W) {
+    const int t = t0 + lane, k = t >> 2, quad = t & 3;
+    Detection d;
+    d.is_col = false;
+    d.pen = 0.f;
+    d.pos = d.normal = zero3();
+    bool def = false;
+    float tol = 0.f;
+    f3 p0 = zero3();
+    float* v = lds + kPair * min(k, W - 1);
+    if (k < n_turn) {
+      p0 = f3{v[0], v[1], v[2]};
+      const f3 n0{v[3], v[4], v[5]}, a0{v[6], v[7], v[8]}, a1{v[9], v[10], v[11]};
+      int ta, tb;
+      pair_geoms(m, __float_as_int(v[28]), ta, tb);
+      tol = dev_tolerance(m, ta, tb, m.mc_tolerance);
+      GPose A{e.L3(s.geoms_pos, ta), e.L4(s.geoms_quat, ta)}, Bp{e.L3(s.geoms_pos, tb), e.L4(s.geoms_quat, tb)};
+      const q4 qr = dev_perturb(m, quad + 1, p0, a0, a1, A, Bp);
+      def = !dev_detect(e, ta, tb, A, Bp, false, n0, tol, snk, d);
+      if (!def && d.is_col) dev_unperturb(m, d, qr, p0, n0);
+    }
+    // which of the pair's four are contacts, in order, each against those before it
+    const bool cand = !def && d.is_col && d.pen > -tol;
+    f3 at[4];
+    unsigned keep = 0, bad = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      at[j] = f3{__shfl(d.pos.x, j, 4), __shfl(d.pos.y, j, 4), __shfl(d.pos.z, j, 4)};
+      bad |= __shfl((int)def, j, 4);
+      bool c = __shfl((int)cand, j, 4) != 0 && !(norm(at[j] - p0) < tol);
+#pragma unroll
+      for (int i = 0; i < j; i++) c = c && !((keep >> i & 1u) && norm(at[j] - at[i]) < tol);
+      keep |= (unsigned)c << j;
+    }
+    __syncthreads();
+    if (k < n_turn) {
+      if (quad == 0) count[k] = bad ? -1 : (int)keep;
+      const float w[7] = {d.normal.x, d.normal.y, d.normal.z, d.pos.x, d.pos.y, d.pos.z, fmaxf(d.pen, 0.f)};
+      for (int j = 0; j < 7; j++) v[7 * quad + j] = w[j];
+    }
+  }
+  __syncthreads();
+  int n = 0;
+  if (lane < cnt && !deferred) {
+    n = o.is_col ? 1 : 0;
+    if (turn) {
+      const int c = count[rank];
+      deferred = c < 0;
+      n = deferred ? 0 : n + __popc((unsigned)c);
+    }
+    if (!deferred) e.S3(s.cache_normal, dev_pair_index(m, ga, gb), o.is_col ? o.normal : zero3());
+  }
+  int total;
+  const int k = base + wave_excl_scan<W>(n, lane, total);
+  defer_pairs<W>(e, lane, deferred, (ga << 16) | gb, k, n_def);
+  __syncthreads();
+  if (turn) count[rank] = (k << 4) | (n > 0 ? count[rank] : 0);
+  if (n > 0) put_contact(e, k, ga, gb, o.normal, o.pos, o.pen, err);
+  __syncthreads();
+  for (int t = lane; t < 4 * n_turn; t += W) {
+    const int c = count[t >> 2], quad = t & 3;
+    if (!(c >> quad & 1)) continue;
+    const float* v = lds + kPair * (t >> 2);
+    const float* w = v + 7 * quad;
+    int ta, tb;
+    pair_geoms(m, __float_as_int(v[28]), ta, tb);
+    put_contact(e, (c >> 4) + 1 + __popc((unsigned)c & ((1u << quad) - 1u)), ta, tb, f3{w[0], w[1], w[2]}, f3{w[3], w[4], w[5]},
+                w[6], err);
+  }
+  __syncthreads();
+  return base + total;
+}
+
+// The broadphase pairs of one kind (convex pairs, or plane-box pairs), W at a time: they are gathered in a queue first,
+// since the two kinds come mixed
+template <bool kGjk, int W>
+__device__ inline int wave_narrow_pass(const Env& e, int lane, float* lds, int nb, bool plane_box_pass, int base,
+                                       uint32_t& err, int& n_def) {
+  const gsr_model& m = e.m;
+  int* q = reinterpret_cast<int*>(lds) + 30 * W;
+  int n = 0;
+  for (int p0 = 0; p0 < nb || n > 0; p0 += W) {
     const int ip = p0 + lane;
-    PairContacts pc;
-    pc.cnt = 0;
-    pc.err = 0;
-    pc.deferred = false;
-    int ga = 0, gb = 0;
-    bool pb = false;
+    int pr = 0;
+    bool mine = false;
     if (ip < nb) {
-      int pr = e.I(s.broad_pairs, ip);
-      ga = pr >> 16;
-      gb = pr & 0xffff;
-      if (m.geom_type[ga] > m.geom_type[gb]) { int t = ga; ga = gb; gb = t; }
-      pb = m.geom_type[ga] == GEOM_PLANE && m.geom_type[gb] == GEOM_BOX;
-      if (pb == plane_box_pass) {
-        LocalSink<false> snk{pc};
-        if (pb) dev_plane_box(e, ga, gb, snk);
-        else dev_convex_convex(e, ga, gb, snk);
-      }
+      pr = e.I(e.s.broad_pairs, ip);
+      int ga, gb;
+      pair_geoms(m, pr, ga, gb);
+      mine = (m.geom_type[ga] == GEOM_PLANE && m.geom_type[gb] == GEOM_BOX) == plane_box_pass;
     }
-    if (kGjk) {
-      unsigned long long redo = env_ballot<W>(pc.deferred);
-      while (redo) {
-        int j = __ffsll((long long)redo) - 1;
-        redo &= redo - 1;
-        if (lane == j) {
-          pc.cnt = 0;
-          pc.err = 0;
-          pc.deferred = false;
-          LocalSink<true> snk{pc};
-          dev_convex_convex(e, ga, gb, snk);
-        }
-      }
+    const unsigned long long b = env_ballot<W>(mine);
+    if (mine) q[n + __popcll(b & ((1ull << lane) - 1ull))] = pr;
+    n += __popcll(b);
+    __syncthreads();
+    if (n < W && p0 + W < nb) continue;
+    if (n == 0) break;
+    const int cnt = min(n, W);
+    if constexpr (kGjk) {
+      base = wave_pairs<true, W>(e, lane, q, cnt, plane_box_pass, base, err);
+    } else {
+      if (plane_box_pass) base = wave_pairs<false, W>(e, lane, q, cnt, true, base, err);
+      else base = wave_convex<W>(e, lane, q, cnt, lds, base, err, n_def);
     }
-    // a pair that needs GJK/EPA contributes no contact here; it is recorded with the index its contacts go to
-    if (pc.deferred) {
-      pc.cnt = 0;
-      pc.err = 0;
-    }
-    const unsigned long long def = env_ballot<W>(pc.deferred);
-    int total;
-    int k = base + wave_excl_scan<W>(pc.cnt, lane, total);
-    if (pc.deferred) {
-      const int slot = n_def + __popcll(def & ((1ull << lane) - 1ull));
-      e.I(s.gjk_defer, 2 * slot) = (ga << 16) | gb;
-      e.I(s.gjk_defer, 2 * slot + 1) = min(k, m.max_contacts);
-    }
-    n_def += __popcll(def);
-    float fr = fmaxf(fmaxf(m.geom_friction[ga] * e.F(s.friction_ratio, ga),
-                           m.geom_friction[gb] * e.F(s.friction_ratio, gb)), 1e-2f);
-    for (int c = 0; c < pc.cnt; c++, k++) {
-      if (k < m.max_contacts) {
-        e.I(s.contact_geoms, 2 * k) = ga;
-        e.I(s.contact_geoms, 2 * k + 1) = gb;
-        e.S3(s.contact_normal, k, pc.n[c]);
-        e.S3(s.contact_pos, k, pc.p[c]);
-        e.F(s.contact_pen, k) = pc.pen[c];
-        e.F(s.contact_friction, k) = fr;
-      } else {
-        pc.err |= GSR_ERR_CONTACT_OVERFLOW;
-      }
-    }
-    err |= pc.err;
-    base += total;
+    n -= cnt;
+    const int left = lane < n ? q[W + lane] : 0;
+    __syncthreads();
+    if (lane < n) q[lane] = left;
+    __syncthreads();
   }
   return base;
 }
 
 template <bool kGjk, int W>
-__device__ inline void wave_narrow_phase(const Env& e, int lane) {
-  const gsr_model& m = e.m;
+__device__ inline void wave_narrow_phase(const Env& e, char* lds, int lane) {
   const gsr_state& s = e.s;
+  float* w = reinterpret_cast<float*>(lds);
   const int nb = e.I(s.n_broad, 0);
   uint32_t err = 0;
   int n_def = 0;
-  int n = wave_narrow_pass<kGjk, W>(e, lane, nb, false, 0, err, n_def);
-  n = wave_narrow_pass<kGjk, W>(e, lane, nb, true, n, err, n_def);
+  int n = wave_narrow_pass<kGjk, W>(e, lane, w, nb, false, 0, err, n_def);
+  n = wave_narrow_pass<kGjk, W>(e, lane, w, nb, true, n, err, n_def);
   for (int o = W / 2; o > 0; o >>= 1) err |= (uint32_t)__shfl_xor((int)err, o, W);
   if (lane == 0) {
-    e.I(s.n_contacts, 0) = min(n, m.max_contacts);
+    e.I(s.n_contacts, 0) = min(n, e.m.max_contacts);
     e.I(s.gjk_defer_n, 0) = n_def;
     if (err) e.I((int32_t*)s.errno_env, 0) |= (int)err;
   }
@@ -326,7 +478,7 @@ __device__ __forceinline__ void wave_collide(const Env& e, char* lds) {
     __syncthreads();
     if (m.n_pairs > 0) {
       wave_broad_phase<W>(e, lds, lane);
-      wave_narrow_phase<kGjk, W>(e, lane);
+      wave_narrow_phase<kGjk, W>(e, lds, lane);
     }
   }
   __syncthreads();

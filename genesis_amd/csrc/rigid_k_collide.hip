@@ -35,7 +35,7 @@ k_collide_wave(gsr_model m, gsr_state s) {
   constexpr int kEnvs = kWave / W;
   const int sub = threadIdx.x / W, b = xcd_env(blockIdx.x, (s.n_envs + kEnvs - 1) / kEnvs) * kEnvs + sub;
   if (b >= s.n_envs) return;  // uniform across an env's lanes
-  wave_collide<false, W>(Env(m, s, b), lds + sizeof(float) * wave_collide_words(m.n_geoms) * sub);
+  wave_collide<false, W>(Env(m, s, b), lds + sizeof(float) * wave_collide_words(m.n_geoms, W) * sub);
 }
 
 }  // namespace
@@ -44,7 +44,7 @@ void launch_collide(const gsr_model& m, const gsr_state& s, hipStream_t st) {
   if (!collide_waves(m))
     hipLaunchKernelGGL(k_collide, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);
   else if (collide_lanes(m, s.n_envs) == 16)
-    hipLaunchKernelGGL(k_collide_wave<16>, dim3((s.n_envs + 3) / 4), dim3(kWave), wave_collide_lds_bytes(m.n_geoms, 4), st,
+    hipLaunchKernelGGL(k_collide_wave<16>, dim3((s.n_envs + 3) / 4), dim3(kWave), wave_collide_lds_bytes(m.n_geoms, 16), st,
                        m, s);
   else
     hipLaunchKernelGGL(k_collide_wave<kWave>, dim3(s.n_envs), dim3(kWave), wave_collide_lds_bytes(m.n_geoms), st, m, s);

@@ -97,7 +97,7 @@ __device__ __forceinline__ void wave_collide_tile(const gsr_model& m, const gsr_
   if (n > 1 && collide_packs(m)) {
     const int sub = threadIdx.x / 16;
     for (int j = sub; j < n; j += 4) {
-      wave_collide<false, 16>(Env(m, s, b0 + j), lds + sizeof(float) * wave_collide_words(m.n_geoms) * sub);
+      wave_collide<false, 16>(Env(m, s, b0 + j), lds + sizeof(float) * wave_collide_words(m.n_geoms, 16) * sub);
       __syncthreads();
     }
   } else {
