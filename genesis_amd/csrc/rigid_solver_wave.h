@@ -209,8 +209,8 @@ __device__ inline void wave_min_degree(const WaveCtx& w, unsigned long long (&ad
 // Row walks of multi-entity models (J^T f, J^T D J) give each lane the dofs it writes: one entity per lane, or one
 // dof per lane when rows have at most kStage entries and the dofs fit two passes of the wavefront. A dof lane reads
 // each of its entity's rows like an entity lane but does one entry's work per row instead of the row's whole pair
-// set: measured on 20-box piles (120 dofs) the solve takes 15 % less time, on 64-box piles (384 dofs, six passes)
-// 15 % more, hence the bound.
+// set: measured on 20-box piles (120 dofs), which this solver took before free bodies had their own, the solve takes 15 %
+// less time, on 64-box piles (384 dofs, six passes) 15 % more, hence the bound.
 __device__ __forceinline__ bool wave_dof_lanes(const WaveCtx& w) {
   return w.e.m.row_width <= kStage && w.D <= 2 * kWave;
 }
