@@ -252,7 +252,7 @@ __device__ inline int wave_pairs(const Env& e, int lane, const int* q, int cnt, 
 // Up to W convex pairs (q[lane], lane < cnt): the first detection with a pair per lane, then the turned detections of the
 // pairs that touch with a detection per lane, four lanes beside each other for a pair. They depend on the first alone,
 // except that a contact near an earlier one of its pair is dropped, which the four lanes settle among themselves. lds: 30 W
-// words; the turned contacts wait there, since in registers they made the fused kernel spill. What bounds it is the chain of support points of one detection: a pair's five in turn on its lane, with the
+// words; the turned contacts wait there too. What bounds it is the chain of support points of one detection: a pair's five in turn on its lane, with the
 // lanes of other pairs idle, were most of a heap's collision. Measured (us, collision and GJK/EPA pass, a pair per lane ->
 // this): 20-box piles 300: 172 -> 106, 1,500: 193 -> 145, 4,000: 403 -> 325; 1,024 64-box piles 566 -> 388.
 template <int W>
