@@ -135,10 +135,11 @@ __device__ __forceinline__ void bodies_sum(const BodyCtx<kWaves>& w, int items, 
 // ---- rows -----------------------------------------------------------------------------------------------------------
 // Bodies of row c (the second << 8). A row that does not store all six entries of its bodies (frictionloss, JOINT
 // equalities) is rewritten with zeros in the places that lack, so that every row holds body a's entries first and, if it
-// has two bodies, b's after them.
+// has two bodies, b's after them. A row without an entry (an equality between two fixed links) is counted to body 0, with
+// six zeros.
 __device__ inline int body_row(const Env& e, int c) {
   const int nnz = e.EI(e.s.jac_nnz, c);
-  const int a = e.JI(c, 0) / 6, b = e.JI(c, nnz - 1) / 6;
+  const int a = nnz > 0 ? e.JI(c, 0) / 6 : 0, b = nnz > 0 ? e.JI(c, nnz - 1) / 6 : 0;
   if (nnz != (a == b ? 6 : 12)) {
     float v[12];
 #pragma unroll

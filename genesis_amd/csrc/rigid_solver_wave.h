@@ -155,11 +155,12 @@ struct WaveCtx {
   }
 };
 
-// entities touched by constraint row c (first and last stored dof; rows touch at most two entities), model numbering
+// entities touched by constraint row c (first and last stored dof; rows touch at most two entities), model numbering. A
+// row without an entry (an equality between two fixed links) is counted to entity 0, where it adds nothing.
 __device__ __forceinline__ void row_entities(const WaveCtx& w, int c, int& ea, int& eb) {
-  int nnz = w.e.EI(w.e.s.jac_nnz, c);
-  ea = w.L.nent[w.e.JI(c, 0)];
-  eb = w.L.nent[w.e.JI(c, nnz - 1)];
+  const int nnz = w.e.EI(w.e.s.jac_nnz, c);
+  ea = nnz > 0 ? w.L.nent[w.e.JI(c, 0)] : 0;
+  eb = nnz > 0 ? w.L.nent[w.e.JI(c, nnz - 1)] : 0;
 }
 
 // Minimum-degree elimination order of the entity graph (entities as nodes, an edge per pair of entities sharing a

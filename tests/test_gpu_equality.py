@@ -173,3 +173,29 @@ def test_per_env_equality_solver_parameters_match_per_env_oracles(variant):
                 assert (err <= TOL + TOL * np.abs(o_)).all(), f"step {step} env {b} {name}"
     z = S.st.t["qpos"][2].cpu().numpy()  # the welded box's height per env
     assert z[2] < z[0] - 1e-3  # time constant 0.2 against the build's 0.02: a softer weld sags further
+
+
+@pytest.mark.parametrize("scene", ["boxes", "arm", "arm_boxes"])
+def test_weld_between_fixed_links(scene):
+    """A weld of two fixed links has no dof: its rows hold no entry and change no motion, whichever wavefront solver
+    reads them (free bodies, a single articulated entity, entity blocks). They are the env's first rows, the first of the
+    row arrays in env 0."""
+    _need_gpu()
+    from genesis_amd.rigid_solver import RigidSolver
+    from oracle.oracle import Oracle
+    B = 4
+    plane, post = W.plane_entity(), W.box_entity((0.1, 0.1, 0.1), (2.0, 0.0, 0.5), fixed=True)
+    post.links[0].name = "post"
+    plane.equalities = [EqualitySpec(EQ_WELD, "plane_baselink", "post")]
+    ents = [plane, post]
+    if "arm" in scene:
+        ents.append(W.panda_entity())
+    if "boxes" in scene:  # two on the ground, so that contact rows follow, and one above
+        ents += [W.box_entity((0.1, 0.1, 0.1), (0.6, 0.3 * i, 0.0499 + 0.0998 * (i % 2))) for i in range(3)]
+    M = compile_model(ents, CompileOptions(dt=0.01, enable_self_collision=False))
+    S = RigidSolver(M, B, "cuda", solver_variant=1)
+    O = Oracle(M, B, 32)
+    _step_against_oracle(S, O, 10, scene)
+    nnz = S.st.t["jac_nnz"].reshape(B, M.max_rows)
+    assert int(S.st.t["n_con"][1].min()) == 6 + ("arm" in scene)  # the arm's fingers are coupled by one row
+    assert int(nnz[:, 6:].max()) > 0
