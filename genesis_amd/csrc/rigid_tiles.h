@@ -45,7 +45,10 @@ __device__ __forceinline__ void wave_step1(const gsr_model& m, const gsr_state& 
       __syncthreads();
     }
   } else {
-    for (int j = 0; j < n; j++) tree_step1<kWave>(Env(m, s, b0 + j), t, tree_words(m, lds, 0));
+    for (int j = 0; j < n; j++) {
+      tree_step1<kWave>(Env(m, s, b0 + j), t, tree_words(m, lds, 0));
+      __syncthreads();  // the next env takes the same LDS words
+    }
   }
 }
 
@@ -88,8 +91,10 @@ __device__ __forceinline__ void wave_step2(const gsr_model& m, const gsr_state& 
       __syncthreads();
     }
   } else {
-    for (int j = 0; j < n; j++)
+    for (int j = 0; j < n; j++) {
       if (!skip(b0 + j)) tree_step2<kWave>(Env(m, s, b0 + j), t, tree_words(m, lds, 0));
+      __syncthreads();
+    }
   }
 }
 // dynamic LDS of wave_step1 and wave_step2 over tiles of n envs

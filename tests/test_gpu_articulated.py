@@ -107,3 +107,22 @@ def test_tree_dynamics_equal_the_lane_per_env_ones(name, B):
         out.append({k: S.st.t[k].clone() for k in COMPARED})
     for k in COMPARED:
         assert torch.equal(out[0][k], out[1][k]), k
+
+
+def test_trees_one_after_the_other_equal_the_plain_step():
+    """Four envs of a tree whose four copies do not fit the LDS of a workgroup (40 dofs) take their turns on a wavefront of
+    the fused kernel, in the same LDS words; the plain step gives each a wavefront of its own."""
+    from genesis_amd.batch import FusedBatch, Group
+    from genesis_amd.rigid_solver import RigidSolver
+    M = compile_model([chain_entity(40)], CompileOptions(dt=0.005, enable_collision=False))
+    B = 9
+    plain, fused = (RigidSolver(M, B, "cuda", solver_variant=1, dyn_variant=1) for _ in range(2))
+    for S in (plain, fused):
+        start(S, M, B, 7)
+    fb = FusedBatch([Group(fused, envs_per_tile=4)])
+    for _ in range(3):
+        plain.substep()
+        fb.step()
+    torch.cuda.synchronize()
+    for k in COMPARED:
+        assert torch.equal(plain.st.t[k], fused.st.t[k]), k
