@@ -259,8 +259,9 @@ int check(const gsr_model* m, const gsr_state* s) {
   if (m->n_geoms >= (1 << 15)) return GSR_E_SHAPE;
   if (m->solver_variant == 1) {
     if (m->n_entities > kMaxPatternEntities) return GSR_E_SHAPE;
-    if (m->wave_h_floats < 0 || solve_lds_bytes(*m) > 160 * 1024)
-      return GSR_E_SHAPE;
+    // the entity-block solver's LDS bounds the Hessian's budget whichever wavefront solver runs: the single-entity solver
+    // takes at most 50 KB, and the free-body solver only models that fit it
+    if (m->wave_h_floats < 0 || wave_lds_bytes(*m) > kMaxSolveLds) return GSR_E_SHAPE;
   }
   if (m->collide_variant == 1) {
     if (m->n_geoms > kWaveMaxGeoms || m->n_contacts_per_pair > kMaxPairContacts) return GSR_E_SHAPE;

@@ -33,17 +33,19 @@ constexpr int kMaxBodies = 128;  // two 64-bit words per pattern row, two bodies
 constexpr int kBlk = 36;         // floats of a 6 x 6 block
 constexpr int kDiaLds = 24, kDiaMem = 21;  // floats from one diagonal block's lower triangle to the next
 
-// every entity has six dofs or none (sum of squares = 6 x sum), and a row has room for all entries of its bodies
-__host__ __device__ inline bool bodies_solver(const gsr_model& m) {
-  return m.n_dofs > 0 && m.max_entity_dofs == 6 && m.mass_blk_size == 6 * m.n_dofs && m.n_dofs <= 6 * kMaxBodies &&
-         m.row_width == (m.n_dofs == 6 ? 6 : 12) && m.max_rows < (1 << 20);
-}
 // rows whose force and weight have a place in LDS: three a dof (a settled heap has 2.5 to 2.8)
 __host__ __device__ inline int bodies_lds_rows(int D) { return (3 * D + 63) & ~63; }
 __host__ __device__ inline size_t bodies_lds_bytes(int D, int H) {
   const int nb = D / 6;
   return sizeof(float) * (size_t)(6 * D + ((H + 3) & ~3) + bodies_lds_rows(D)) + 16 * (size_t)nb + 8 * 32 +
          sizeof(int) * (size_t)(12 * nb + 16 + 2 * (H / kBlk)) + 32;
+}
+// every entity has six dofs or none (sum of squares = 6 x sum), a row has room for all entries of its bodies, and the
+// Hessian's budget leaves room for the rest (the entity-block solver needs less beside it)
+__host__ __device__ inline bool bodies_solver(const gsr_model& m) {
+  return m.n_dofs > 0 && m.max_entity_dofs == 6 && m.mass_blk_size == 6 * m.n_dofs && m.n_dofs <= 6 * kMaxBodies &&
+         m.row_width == (m.n_dofs == 6 ? 6 : 12) && m.max_rows < (1 << 20) &&
+         bodies_lds_bytes(m.n_dofs, m.wave_h_floats) <= kMaxSolveLds;
 }
 
 // Wavefronts per env of the plain step's solve: two up to 128 dofs, four above. Measured (us a pass of three steps at

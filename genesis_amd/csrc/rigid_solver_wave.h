@@ -90,6 +90,7 @@ struct WaveLds {
   lds_i* moff;                // [E] offset of each entity's mass block (copy of ent_mass_offset, model numbering)
 };
 
+constexpr size_t kMaxSolveLds = 160 * 1024;  // LDS of a CU
 constexpr int kWavePreSlots = 256;   // off-diagonal pattern blocks addressable in LDS mode
 
 // H = floats of LDS for the Hessian of one env (gsr_model.wave_h_floats): a pattern that needs more keeps H in global

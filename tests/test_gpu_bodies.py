@@ -68,3 +68,24 @@ def test_free_body_solver(n, friction):
                 assert (np.abs(got[b] - o[b]) <= bound).all(), f"step {step} env {b} {name}"
             assert torch.equal(S.st.t[name], solvers[1].st.t[name]), f"step {step} {name}: fused and plain differ"
     assert rows >= 12 * n, rows
+
+
+def test_budgets_beyond_the_body_solver():
+    """A Hessian budget that leaves no room for the free-body solver's arrays goes to the entity-block solver, which gives
+    the same bits: the largest budget of ten boxes, against the default one."""
+    from genesis_amd.rigid_solver import RigidSolver
+    n, B = 10, 3
+    ents, q = stacks(n, B, n)
+    M = compile_model(ents, CompileOptions(dt=0.005, max_collision_pairs=400))
+    D, E = M.n_dofs, M.n_entities
+    rest = 4 * 6 * D + 16 * E + 4 * 3 * D + 4 * (9 * E + 6) + 4 * (6 * E + 257) + 64
+    a, b = (RigidSolver(M, B, "cuda", solver_variant=1, wave_h_floats=h) for h in (None, (160 * 1024 - rest) // 4))
+    for S in (a, b):
+        S.set_qpos(torch.as_tensor(q, dtype=torch.float32))
+    for _ in range(5):
+        a.substep()
+        b.substep()
+    torch.cuda.synchronize()
+    assert int(a.st.t["n_con"][0].max()) > 0 and int(a.st.t["solver_iters"].max()) > 0
+    for k in ("qpos", "vel", "efc_force", "n_con"):
+        assert torch.equal(a.st.t[k], b.st.t[k]), k

@@ -173,3 +173,27 @@ def test_noalloc_scratch_size_matches_state_layout(lib):
             want = sum(-(-sz[k] * n * 4 // 256) * 256 for k in NOALLOC_SCRATCH)
             assert lib.gsr_noalloc_scratch_bytes(ctypes.byref(d), n) == want
         assert lib.gsr_noalloc_scratch_bytes(ctypes.byref(d), 0) == -1
+
+
+@pytest.mark.parametrize("scene", ["boxes", "arm", "arm_boxes"])
+def test_hessian_budget_limit_is_that_of_the_entity_block_solver(lib, scene):
+    """The largest Hessian budget a model may ask for is what the entity-block solver's other arrays leave of 160 KB,
+    whichever wavefront solver runs it: one float more is refused, for free bodies, a single entity and a mix. (A kinematics
+    call over no env checks the model and launches nothing.)"""
+    from genesis_amd.rigid_solver import DeviceModel, DeviceState
+    ents = [W.plane_entity()]
+    if "arm" in scene:
+        ents.append(W.panda_entity())
+    if "boxes" in scene:
+        ents += W.pile_entities(20, np.random.default_rng(1))[1:]
+    M = compile_model(ents, CompileOptions())
+    D, E = M.n_dofs, M.n_entities
+    # floats over dofs and budget, two 64-bit words and 9 + 6 ints an entity, 3 ints a dof, 6 and 257 ints, 64 bytes
+    rest = 4 * 6 * D + 16 * E + 4 * 3 * D + 4 * (9 * E + 6) + 4 * (6 * E + 257) + 64
+    limit = (160 * 1024 - rest) // 4
+    none = np.zeros(1, np.int32)
+    for budget, want in ((limit, 0), (limit + 1, -2), (-1, -2)):
+        dm = DeviceModel(M, "cpu", solver_variant=1, wave_h_floats=budget)
+        st = DeviceState(dm, 1)
+        rc = lib.gsr_forward_kinematics(ctypes.byref(dm.desc), ctypes.byref(st.desc), none.ctypes.data, 0, None)
+        assert rc == want, (budget, rc)
