@@ -298,7 +298,7 @@ void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
     // kinematics of the current pose are refreshed at the end of every step (and by gsr_forward_kinematics after a
     // pose write), so kernel_step_1 never needs to recompute them (enable_mujoco_compatibility = False)
     case 0:
-      if (dyn_lds_bytes(*m)) launch_tree(k_step1_tree<16>, k_step1_tree<kWave>, *m, s->n_envs, st, *m, *s);
+      if (dyn_form(*m, s->n_envs)) launch_tree(k_step1_tree<16>, k_step1_tree<kWave>, *m, s->n_envs, st, *m, *s);
       else launch_entities(k_step1, *m, s->n_envs, st, *m, *s);
       break;
     case 1:
@@ -308,7 +308,7 @@ void launch_one(const gsr_model* m, const gsr_state* s, int k, hipStream_t st) {
       launch_solve(*m, *s, st);
       break;
     default:
-      if (dyn_lds_bytes(*m)) launch_tree(k_step2_tree<16>, k_step2_tree<kWave>, *m, s->n_envs, st, *m, *s);
+      if (dyn_form(*m, s->n_envs)) launch_tree(k_step2_tree<16>, k_step2_tree<kWave>, *m, s->n_envs, st, *m, *s);
       else launch_entities(k_step2, *m, s->n_envs, st, *m, *s);
       break;
   }
@@ -528,6 +528,28 @@ int gsr_launch_kernel(const gsr_model* model, const gsr_state* state, int32_t ke
   if (kernel < 0 || kernel > 3) return GSR_E_ARG;
   launch_one(model, state, kernel, stream);
   return launch_status();
+}
+
+const char* gsr_kernel_name(const gsr_model* model, int32_t n_envs, int32_t kernel) {
+  if (!model || n_envs <= 0 || kernel < 0 || kernel > 3) return "";
+  const int dyn = dyn_form(*model, n_envs);
+  switch (kernel) {
+    case 0: return dyn == 16 ? "k_step1_tree<16>" : dyn ? "k_step1_tree<64>" : "k_step1";
+    case 1: {
+      const int lanes = collide_form(*model, n_envs);
+      return lanes == 1 ? "k_collide" : lanes == 16 ? "k_collide_wave<16>" : "k_collide_wave<64>";
+    }
+    case 2:
+      switch (solve_form(*model)) {
+        case kSolveLane: return "k_solve";
+        case kSolveDense: return "k_solve_dense";
+        case kSolveBodies2: return "k_solve_bodies<2>";
+        case kSolveBodies4: return "k_solve_bodies<4>";
+        case kSolveBlocks: return "k_solve_wave";
+      }
+      return "";
+    default: return dyn == 16 ? "k_step2_tree<16>" : dyn ? "k_step2_tree<64>" : "k_step2";
+  }
 }
 
 int gsr_run_stage(const gsr_model* model, const gsr_state* state, int32_t stage, hipStream_t stream) {

@@ -41,14 +41,15 @@ k_collide_wave(gsr_model m, gsr_state s) {
 }  // namespace
 
 void launch_collide(const gsr_model& m, const gsr_state& s, hipStream_t st) {
-  if (!collide_waves(m))
-    hipLaunchKernelGGL(k_collide, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);
-  else if (collide_lanes(m, s.n_envs) == 16)
-    hipLaunchKernelGGL(k_collide_wave<16>, dim3((s.n_envs + 3) / 4), dim3(kWave), wave_collide_lds_bytes(m.n_geoms, 16), st,
-                       m, s);
-  else
-    hipLaunchKernelGGL(k_collide_wave<kWave>, dim3(s.n_envs), dim3(kWave), wave_collide_lds_bytes(m.n_geoms), st, m, s);
-  hipLaunchKernelGGL(k_gjk_fixup, dim3(s.n_envs), dim3(kWave), 0, st, m, s);
+  const int n = s.n_envs;
+  switch (collide_form(m, n)) {
+    case 1: hipLaunchKernelGGL(k_collide, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s); break;
+    case 16:
+      hipLaunchKernelGGL(k_collide_wave<16>, dim3((n + 3) / 4), dim3(kWave), wave_collide_lds_bytes(m.n_geoms, 16), st, m, s);
+      break;
+    default: hipLaunchKernelGGL(k_collide_wave<kWave>, dim3(n), dim3(kWave), wave_collide_lds_bytes(m.n_geoms), st, m, s);
+  }
+  hipLaunchKernelGGL(k_gjk_fixup, dim3(n), dim3(kWave), 0, st, m, s);
 }
 
 }  // namespace gsr

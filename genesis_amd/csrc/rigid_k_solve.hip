@@ -1,5 +1,5 @@
-// Newton solve of the plain step: k_solve (one lane per env) or k_solve_wave (one wavefront per env, LDS vectors
-// and Hessian).
+// Newton solve of the plain step: k_solve (one lane per env), or on wavefronts k_solve_dense (every dof in one entity),
+// k_solve_bodies<2 | 4> (free bodies, two or four wavefronts per env) or k_solve_wave (entity blocks).
 #include "rigid_tiles.h"
 
 namespace gsr {
@@ -41,23 +41,17 @@ __global__ void __launch_bounds__(kWave * kWaves) __attribute__((amdgpu_waves_pe
   solve_bodies<kWaves>(e, lds);
 }
 
-template <int kWaves>
-void launch_bodies(const gsr_model& m, const gsr_state& s, hipStream_t st) {
-  hipLaunchKernelGGL(k_solve_bodies<kWaves>, dim3(s.n_envs), dim3(kWave * kWaves), solve_lds_bytes(m), st, m, s);
-}
-
 }  // namespace
 
 void launch_solve(const gsr_model& m, const gsr_state& s, hipStream_t st) {
-  if (m.solver_variant == 1 && dense_solver(m))
-    hipLaunchKernelGGL(k_solve_dense, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
-  else if (m.solver_variant == 1 && bodies_solver(m)) {
-    if (bodies_waves(m.n_dofs) == 2) launch_bodies<2>(m, s, st);
-    else launch_bodies<4>(m, s, st);
-  } else if (m.solver_variant == 1)
-    hipLaunchKernelGGL(k_solve_wave, dim3(s.n_envs), dim3(kWave), solve_lds_bytes(m), st, m, s);
-  else
-    hipLaunchKernelGGL(k_solve, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s);
+  const size_t lds = solve_lds_bytes(m);
+  switch (solve_form(m)) {
+    case kSolveLane: hipLaunchKernelGGL(k_solve, dim3((s.n_envs + kBlock - 1) / kBlock), dim3(kBlock), 0, st, m, s); break;
+    case kSolveDense: hipLaunchKernelGGL(k_solve_dense, dim3(s.n_envs), dim3(kWave), lds, st, m, s); break;
+    case kSolveBodies2: hipLaunchKernelGGL(k_solve_bodies<2>, dim3(s.n_envs), dim3(2 * kWave), lds, st, m, s); break;
+    case kSolveBodies4: hipLaunchKernelGGL(k_solve_bodies<4>, dim3(s.n_envs), dim3(4 * kWave), lds, st, m, s); break;
+    case kSolveBlocks: hipLaunchKernelGGL(k_solve_wave, dim3(s.n_envs), dim3(kWave), lds, st, m, s); break;
+  }
 }
 
 }  // namespace gsr

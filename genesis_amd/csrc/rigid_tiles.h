@@ -352,8 +352,22 @@ k_fused(const char* __restrict__ table, uint32_t* queue, int persistent) {
 }
 
 // ---- launchers (host code; each defined in the translation unit that holds its kernel) -----------------------
-// plain step (rigid_k_collide.hip, rigid_k_solve.hip): the collision stage (collision kernel + GJK/EPA pass) and
-// the Newton solve of the model's variants
+// plain step: which kernel a stage launches for a model over n envs (gsr_kernel_name names them by the same choice)
+inline int dyn_form(const gsr_model& m, int n) {  // lanes per env of the tree kernels, 0: (env, entity) lanes
+  return dyn_lds_bytes(m) ? tree_lanes(m, n) : 0;
+}
+inline int collide_form(const gsr_model& m, int n) {  // lanes per env
+  return collide_waves(m) ? collide_lanes(m, n) : 1;
+}
+enum SolveForm { kSolveLane, kSolveDense, kSolveBodies2, kSolveBodies4, kSolveBlocks };
+inline SolveForm solve_form(const gsr_model& m) {
+  if (m.solver_variant != 1) return kSolveLane;
+  if (dense_solver(m)) return kSolveDense;
+  if (bodies_solver(m)) return bodies_waves(m.n_dofs) == 2 ? kSolveBodies2 : kSolveBodies4;
+  return kSolveBlocks;
+}
+// its launchers (rigid_k_collide.hip, rigid_k_solve.hip): the collision stage (collision kernel + GJK/EPA pass) and
+// the Newton solve
 void launch_collide(const gsr_model& m, const gsr_state& s, hipStream_t st);
 void launch_solve(const gsr_model& m, const gsr_state& s, hipStream_t st);
 // batching form: k_fused<W, G> (rigid_k_fused_wW_gG.hip), k_phase<P> (rigid_k_phase_P.hip), k_gjk_resume

@@ -210,6 +210,9 @@ int gsr_get_equalities(const gsr_model* model, const gsr_state* state, int32_t* 
  * 3 = integration + end-of-step kinematics); gsr_step launches exactly these four in order. No counterpart in the
  * reference: used to time each kernel on the caller's stream. */
 int gsr_launch_kernel(const gsr_model* model, const gsr_state* state, int32_t kernel, hipStream_t stream);
+/* Name of the device kernel gsr_launch_kernel runs for this model over n_envs envs (kernel 1 is followed by the GJK/EPA
+ * pass k_gjk_fixup); "" for arguments out of range. */
+const char* gsr_kernel_name(const gsr_model* model, int32_t n_envs, int32_t kernel);
 
 /* Stage runner for parity tests: 1 = kinematics, 2 = + smooth dynamics, 3 = + collision detection, 0 = full step. */
 int gsr_run_stage(const gsr_model* model, const gsr_state* state, int32_t stage, hipStream_t stream);

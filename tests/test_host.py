@@ -197,3 +197,24 @@ def test_hessian_budget_limit_is_that_of_the_entity_block_solver(lib, scene):
         st = DeviceState(dm, 1)
         rc = lib.gsr_forward_kinematics(ctypes.byref(dm.desc), ctypes.byref(st.desc), none.ctypes.data, 0, None)
         assert rc == want, (budget, rc)
+
+
+@pytest.mark.parametrize("scene,n,variants,names", [
+    ("arm", 64, (), ("k_step1_tree<64>", "k_collide_wave<64>", "k_solve_dense", "k_step2_tree<64>")),
+    ("quadruped", 4000, (), ("k_step1_tree<16>", "k_collide_wave<16>", "k_solve_dense", "k_step2_tree<16>")),
+    ("quadruped", 1500, (), ("k_step1_tree<16>", "k_collide_wave<64>", "k_solve_dense", "k_step2_tree<16>")),
+    ("quadruped", 64, (0, 1, 0), ("k_step1", "k_collide_wave<64>", "k_solve", "k_step2")),
+    ("boxes20", 1500, (), ("k_step1", "k_collide_wave<64>", "k_solve_bodies<2>", "k_step2")),
+    ("boxes64", 96, (), ("k_step1", "k_collide_wave<64>", "k_solve_bodies<4>", "k_step2")),
+    ("arm_boxes", 1, (), ("k_step1_tree<64>", "k_collide_wave<64>", "k_solve_wave", "k_step2_tree<64>")),
+])
+def test_kernel_names_follow_the_launches(lib, scene, n, variants, names):
+    """kernel_name(k) names the kernel launch_kernel(k) runs: the wavefront forms by model and env count, as the launchers
+    choose them."""
+    from genesis_amd.rigid_solver import DeviceModel
+    ents = {"arm": [W.plane_entity(), W.panda_entity()], "quadruped": [W.plane_entity(), W.go2_entity()],
+            "boxes20": W.pile_entities(20, np.random.default_rng(1)), "boxes64": W.pile_entities(64, np.random.default_rng(1)),
+            "arm_boxes": [W.plane_entity(), W.panda_entity(), W.box_entity((0.1, 0.1, 0.1), (1.0, 0.0, 0.1))]}[scene]
+    dm = DeviceModel(compile_model(ents, CompileOptions(max_collision_pairs=100)), "cpu", *variants, n_envs=n)
+    assert tuple(lib.gsr_kernel_name(dm.desc, n, k).decode() for k in range(4)) == names
+    assert [lib.gsr_kernel_name(dm.desc, n, k) for k in (-1, 4)] == [b"", b""]
