@@ -622,7 +622,7 @@ int gsr_batch_upload(const gsr_group* groups, int32_t n_groups, void* dev_table,
     lds = std::max(lds, dyn_lds_bytes(G.model, G.envs_per_tile));
     const int Td = dyn_tile_envs(G.model, G.n_envs, G.envs_per_tile);
     const int n_t = (G.n_envs + G.envs_per_tile - 1) / G.envs_per_tile, n_w = (G.n_envs + Tw - 1) / Tw;
-    const int Tc = collide_tile_envs(G.model, G.n_envs, G.envs_per_tile);
+    const int Tc = collide_tile_envs(G.model, G.n_envs, G.state.n_envs, G.envs_per_tile);
     const int n_d = (G.n_envs + Td - 1) / Td, n_c = (G.n_envs + Tc - 1) / Tc;
     ranges[g] = BatchRange{type, G.env_begin, G.n_envs, G.envs_per_tile, tiles, tiles + n_t, Tw, wtiles, wtiles + n_w,
                            Td, dtiles, dtiles + n_d, Tc, ctiles, ctiles + n_c};

@@ -67,6 +67,16 @@ __host__ __device__ inline bool collide_packs(const gsr_model& m) { return m.n_e
 // 4213, 172, 354; 4,000: 4437, 403, 448; 64 boxes 1,024: 25968, 566, 1529 (heaps with a pair per lane throughout; wave_convex
 // has taken 15 to 40 % off their 64-lane figures since).
 __host__ __device__ inline int collide_lanes(const gsr_model& m, int n) { return n > 2048 && collide_packs(m) ? 16 : kWave; }
+// Models of variant 0 with few entities over so many envs that a lane per env fills the chip too: its work per env is the
+// least, and what the wavefront forms gain by spreading one env is lost. Where the line lies follows the geoms, since one lane
+// walks them all. Measured (us, lane per env, 16 lanes where the model packs, else 64), below and at the line: one sphere
+// 8,192: 32, 41; 16,384: 34, 71; one box 8,192: 54, 50; 16,384: 62, 85; two boxes 16,384: 205, 206; 32,768: 277, 411; three
+// 16,384: 348, 281; 32,768: 500, 610; seven 32,768: 386, 397; a quadruped on a plane (28 geoms) 32,768: 276, 174; 65,536:
+// 311, 344; an arm of 35 geoms 16,384: 380, 243; 32,768: 430, 479; of 121 geoms 16,384: 1265, 941; 32,768: 1419, 1942.
+__host__ __device__ inline bool collide_by_lane(const gsr_model& m, int n) {
+  const int line = m.n_geoms <= 2 ? 16384 : m.n_geoms <= 6 ? 32768 : m.n_geoms <= 32 ? 65536 : 32768;
+  return m.collide_variant == 0 && m.n_entities <= 8 && n >= line;
+}
 
 template <int W>
 __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {

@@ -1,6 +1,6 @@
-// Collision stage of the plain step: k_collide_wave (16 or 64 lanes per env; k_collide, one lane per env, only for models
-// its LDS does not hold), then
-// the GJK/EPA pass k_gjk_fixup over the pairs the narrowphase deferred.
+// Collision stage of the plain step: k_collide_wave (16 or 64 lanes per env) or k_collide (one lane per env: small models
+// over very many envs, and models the wavefront form's LDS does not hold), then the GJK/EPA pass k_gjk_fixup over the pairs
+// the narrowphase deferred.
 #include "rigid_tiles.h"
 
 namespace gsr {

@@ -108,9 +108,10 @@ __host__ __device__ inline int dyn_tile_envs(const gsr_model& m, int n, int envs
   if (m.dyn_variant != 1) return envs_per_tile;
   return tree_dynamics(m) ? kWave / tree_lanes(m, n) : n > 1024 ? 4 : 1;
 }
-// envs per tile of the phased collision, likewise
-__host__ __device__ inline int collide_tile_envs(const gsr_model& m, int n, int envs_per_tile) {
-  return collide_waves(m) ? kWave / collide_lanes(m, n) : envs_per_tile;
+// envs per tile of the phased collision of a group of n envs, likewise (n_all: envs of the group's state)
+__host__ __device__ inline int collide_tile_envs(const gsr_model& m, int n, int n_all, int envs_per_tile) {
+  if (!collide_waves(m)) return envs_per_tile;
+  return collide_by_lane(m, n_all) ? kWave : kWave / collide_lanes(m, n);
 }
 // envs [b0, b0 + n) of the wavefront collision: one after the other, or four at a time where the model packs
 __device__ __forceinline__ void wave_collide_tile(const gsr_model& m, const gsr_state& s, int b0, int n, char* lds) {
@@ -254,7 +255,11 @@ template <int P>
 __device__ __forceinline__ void phase_tile(const gsr_model& m, const gsr_state& s, int env0, int n_here, char* lds) {
   const int lane = threadIdx.x;
   const bool mine = lane < n_here;
-  const bool wave = P == 0 || P == 4 ? m.dyn_variant == 1 : P == 1 ? collide_waves(m) : P == 3 ? m.solver_variant == 1 : true;
+  // a lane per env only in tiles that a lane serves well: the serving loop's tiles hold as many envs as its pools say
+  const bool wave = P == 0 || P == 4 ? m.dyn_variant == 1
+                    : P == 1         ? collide_waves(m) && !(n_here > 4 && collide_by_lane(m, s.n_envs))
+                    : P == 3         ? m.solver_variant == 1
+                                     : true;
   if (!wave) {
     if (!mine) return;
     Env e(m, s, env0 + lane);
@@ -357,7 +362,7 @@ inline int dyn_form(const gsr_model& m, int n) {  // lanes per env of the tree k
   return dyn_lds_bytes(m) ? tree_lanes(m, n) : 0;
 }
 inline int collide_form(const gsr_model& m, int n) {  // lanes per env
-  return collide_waves(m) ? collide_lanes(m, n) : 1;
+  return collide_waves(m) && !collide_by_lane(m, n) ? collide_lanes(m, n) : 1;
 }
 enum SolveForm { kSolveLane, kSolveDense, kSolveBodies2, kSolveBodies4, kSolveBlocks };
 inline SolveForm solve_form(const gsr_model& m) {

@@ -55,8 +55,8 @@ typedef struct gsr_model {
   int32_t enable_collision, enable_joint_limit, enable_multi_contact;
   int32_t solver_variant;  /* 0: one lane per env (rows env-minor), 1: one wavefront per env (rows env-major) */
   int32_t collide_variant; /* the single fused kernel's collision: 0 one lane per env, 1 one wavefront per env (pairs
-                              across lanes). The plain and phased steps take 64 or 16 lanes per env by size; a lane per
-                              env only where 0 is set and the model has more than 1,022 geoms */
+                              across lanes). The plain and phased steps take 64 or 16 lanes per env by size with either;
+                              with 0 a lane per env over very many envs of a small model and above 1,022 geoms */
   int32_t dyn_variant;     /* step_1 / step_2: 0 one lane per env, 1 one wavefront per env (entities across lanes) */
   int32_t batch_dofs;      /* 1: dof_kp, dof_kv, dof_force_range, dof_stiffness, dof_damping, dof_frictionloss,
                               dof_limit, dof_armature and dof_invweight hold one value per env, env-minor like the state

@@ -1,5 +1,5 @@
 """Collision with 16 lanes per env (many envs of a small model), 64 lanes, and one lane per env (the single fused kernel's
-variant 0) give the same bits, also where the broadphase buffer overflows."""
+variant 0, and very many envs of a small model) give the same bits, also where the broadphase buffer overflows."""
 import numpy as np
 import pytest
 import torch
@@ -91,3 +91,36 @@ def test_many_pairs_agree(deep):
     assert int(((pairs >> 16) > 0).sum()) > 64  # geom 0 is the plane
     # without a cached normal the first step of either heap leaves some pairs to GJK/EPA
     assert bool((wave.st.t["errno_env"] & 0x100).any())
+
+
+@pytest.mark.parametrize("n,B", [(1, 16384), (5, 32768)])
+def test_lane_per_env_over_very_many_envs(n, B):
+    """At the line where variant 0 goes over to a lane per env (2 and 6 geoms), the plain and the phased step give the bits of
+    16 lanes; one env fewer still takes those."""
+    from genesis_amd.batch import FusedBatch, Group
+    from genesis_amd.rigid_solver import RigidSolver
+    ents, q = stacks(n, 41, 5)
+    M = compile_model(ents, CompileOptions(dt=0.005, max_collision_pairs=20))
+    q = torch.as_tensor(np.tile(q, (B // 41 + 1, 1))[:B], dtype=torch.float32)
+    lane, many, phased = (RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=v, dyn_variant=1) for v in (0, 1, 0))
+    fewer = RigidSolver(M, B - 1, "cuda", solver_variant=1, collide_variant=0, dyn_variant=1)
+    assert [S.kernel_name(1) for S in (lane, many, fewer)] == ["k_collide", "k_collide_wave<16>", "k_collide_wave<16>"]
+    for S in (lane, many, phased):
+        S.set_qpos(q)
+    # two groups: whole tiles of 64 lanes, then one of three envs, which its wavefront takes as the 16-lane form does
+    fb = FusedBatch([Group(phased, 0, B - 67, 1, 1, 0), Group(phased, B - 67, 67, 1, 1, 0)], phased=True)
+    for _ in range(2):
+        lane.substep()
+        many.substep()
+        fb.step()
+    torch.cuda.synchronize()
+    assert int(many.st.t["n_contacts"].min()) >= 4
+    for k in COMPARED:
+        a, b, c = (S.st.t[k] for S in (lane, many, phased))
+        if k in ("broad_pairs", "contact_geoms", "contact_pos", "contact_normal", "contact_pen"):
+            cnt = many.st.t["n_broad" if k == "broad_pairs" else "n_contacts"][0].long()
+            per = {"broad_pairs": 1, "contact_geoms": 2, "contact_pos": 3, "contact_normal": 3, "contact_pen": 1}[k]
+            keep = torch.arange(b.shape[0], device=b.device)[:, None] < per * cnt[None]
+            a, b, c = (torch.where(keep, x, torch.zeros_like(x)) for x in (a, b, c))
+        assert torch.equal(a, b), f"{k}: one and 16 lanes differ"
+        assert torch.equal(c, b), f"{k}: phased and plain differ"
