@@ -145,17 +145,34 @@ class FusedBatch:
             pass
 
 
+def _phased_choice(solver: RigidSolver, v: int, c: int, t: int, w: Optional[int]):
+    """What the phased launches read of a choice: the solver variant and the solve's tiles, the collision kernel that the
+    variant and the sizes lead to, and the group's own tiles only where a lane per env serves a stage (their number
+    follows the sizes elsewhere)."""
+    d = type(solver.dm.desc)()
+    ctypes.memmove(ctypes.byref(d), ctypes.byref(solver.dm.desc), ctypes.sizeof(d))
+    d.solver_variant, d.collide_variant = v, c
+    collide = _lib.load().gsr_kernel_name(d, solver._B, 1)
+    own = d.dyn_variant == 0 or solver.model.n_geoms > 1022
+    return v, collide, t if w is None else w, t if own else None
+
+
 def candidates(solver: RigidSolver, phased: bool = False) -> List[Tuple[int, int, int, Optional[int]]]:
     """(solver_variant, collide_variant, envs_per_tile, wave_envs_per_tile) choices worth timing for one scene type.
-    Under the phased launch the solve (and the GJK/EPA pass) has tiles of its own, so a lane-per-env collision with
-    64 envs a tile can sit beside a wavefront solve with one to four."""
+    Under the phased launch the solve (and the GJK/EPA pass) has tiles of its own, and of choices that come to the same
+    launches one is kept."""
     M = solver.model
     out = [(0, 0, 64, None), (0, 0, 32, None), (0, 1, 8, None)]
     if M.n_entities <= WAVE_MAX_ENTITIES:
         out += [(1, 1, t, None) for t in (1, 2, 4, 8)] + [(1, 0, 4, None)]
         if phased:
             out += [(1, 0, 64, w) for w in (1, 2, 4)] + [(1, 1, 4, 1), (1, 1, 8, 2)]
-    return out
+    if not phased:
+        return out
+    kept = {}
+    for x in out:
+        kept.setdefault(_phased_choice(solver, *x), x)
+    return list(kept.values())
 
 
 def _snapshot(solver: RigidSolver):

@@ -218,3 +218,28 @@ def test_kernel_names_follow_the_launches(lib, scene, n, variants, names):
     dm = DeviceModel(compile_model(ents, CompileOptions(max_collision_pairs=100)), "cpu", *variants, n_envs=n)
     assert tuple(lib.gsr_kernel_name(dm.desc, n, k).decode() for k in range(4)) == names
     assert [lib.gsr_kernel_name(dm.desc, n, k) for k in (-1, 4)] == [b"", b""]
+
+
+@pytest.mark.parametrize("scene,n,solve_tiles,both_collisions", [
+    ("arm", 5001, [1, 2, 4, 8], False), ("quadruped", 32768, [1, 2, 4, 8], False), ("box", 16384, [1, 2, 4, 8], True),
+])
+def test_phased_candidates_are_different_launches(lib, scene, n, solve_tiles, both_collisions):
+    """The phased launches take the lanes of the collision and the dynamics by size, so most (collision variant, tile) choices
+    come to the same launches: each is timed once. One box over 16,384 envs may also collide a lane per env."""
+    from types import SimpleNamespace
+
+    from genesis_amd.batch import candidates
+    from genesis_amd.rigid_solver import DeviceModel
+    ents = {"arm": [W.plane_entity(), W.panda_entity()], "quadruped": [W.plane_entity(), W.go2_entity()],
+            "box": W.pile_entities(1, np.random.default_rng(1))}[scene]
+    M = compile_model(ents, CompileOptions())
+    dm = DeviceModel(M, "cpu", 1, 0, 1, n_envs=n)
+    solver = SimpleNamespace(model=M, dm=dm, _B=n)
+    wave = [x for x in candidates(solver, phased=True) if x[0] == 1]
+    kinds = {}
+    for v, c, t, w in wave:
+        dm.desc.collide_variant = c
+        kinds.setdefault(lib.gsr_kernel_name(dm.desc, n, 1), []).append(w or t)
+    assert all(sorted(set(k)) == sorted(k) for k in kinds.values()), kinds
+    assert any(k == solve_tiles for k in kinds.values()) and len(kinds) == (2 if both_collisions else 1), kinds
+    assert len([x for x in candidates(solver) if x[0] == 1]) == 5  # the single fused kernel reads all of them
