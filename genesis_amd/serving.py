@@ -149,7 +149,11 @@ class Server:
         self.host = hp.contents
         self.info = _lib.GsrBatchInfo()
         self.info.persistent = int(bool(launch.get("persistent", False)))
-        self.info.waves_per_simd = int(launch.get("waves_per_simd", 4))
+        # 256 VGPRs: a tick rarely has more tiles than the SIMDs hold at two waves, and at 128 the fused kernel spills most of
+        # its registers. Measured (ms, whole bursts of 12 requests of arms, quadrupeds and piles, 128 -> 256 VGPRs): requests
+        # of up to 30 envs 6.53 -> 6.40, 96: 13.30 -> 12.05, 400: 10.64 -> 9.79, 1,000: 13.71 -> 13.08, 2,500: 28.8 -> 27.4,
+        # 5,000: 67.2 -> 67.8
+        self.info.waves_per_simd = int(launch.get("waves_per_simd", 2))
         self.info.gjk_inline = int(bool(launch.get("gjk_inline", False)))
         self.info.phased = int(bool(launch.get("phased", False)))
         torch.cuda.synchronize(self.device)

@@ -146,3 +146,19 @@ def test_bench_sized_pools_large_request_alone_and_in_mix():
     st = srv.run(mix, record=True)
     assert st["completed"] == len(mix) and st["failed"] == 0
     _same(lone.result, mix[2].result, "4,096-env pile request alone vs in the mix")
+
+
+def test_register_budgets_of_the_tick_agree():
+    """A server takes the 256-VGPR fused kernel unless told otherwise; the 128-VGPR one gives the same results."""
+    from genesis_amd.serving import Request
+    reqs = [Request(0, "arm", 5, 6, 0.0, seed=7), Request(1, "quadruped", 6, 5, 0.0, seed=8),
+            Request(2, "pile20", 3, 4, 0.0, seed=9)]
+    got = []
+    for launch, waves in ((None, 2), (dict(waves_per_simd=4), 4)):
+        srv = _server(launch=launch)
+        assert srv.info.waves_per_simd == waves
+        run = [_copy(r) for r in reqs]
+        srv.run(run, record=True)
+        got.append([r.result for r in run])
+    for r, a, b in zip(reqs, *got):
+        _same(a, b, r.scene)
