@@ -125,7 +125,7 @@ __device__ inline void wave_broad_phase(const Env& e, char* lds, int lane) {
     else minpos[t] = i;
   }
   __syncthreads();
-  // geoms in the order of their min events: order[k] (tv's place), the AABBs in LDS. The geoms a min event pairs with are
+  // geoms in the order of their min events: order[k] (in tig's place, whose contents sig has now), the AABBs in LDS. The geoms a min event pairs with are
   // those before it in this order whose max event comes later; they are tested on their own lanes, W at a time, event
   // after event, and a ballot places the pairs in the serial sweep's order.
   int* order = tig;

@@ -17,8 +17,7 @@
 //
 // Measured (MI355X, us per launch, one lane per env -> 64 lanes -> 16 lanes per env), step_1: 64 arms 172 -> 23, 5,001
 // arms 204 -> 81 -> 31, 4,000 quadrupeds 475 -> 114 -> 58, 32,768 quadrupeds 571 -> 846 -> 232; step_2: 64 arms 92 -> 36,
-// 5,001 arms 122 -> 72 -> 44, 32,768 quadrupeds 190 -> 259 -> 145; kinematics of 20,000 listed quadrupeds
-// 198 -> 261 -> 113.
+// 5,001 arms 122 -> 72 -> 44, 32,768 quadrupeds 190 -> 259 -> 145; kinematics of 20,000 quadrupeds 198 -> 261 -> 113.
 #pragma once
 #include "rigid_kin.h"
 #include "rigid_solver.h"
@@ -39,14 +38,17 @@ __host__ __device__ inline int tree_env_words(const gsr_model& m) {
 __host__ __device__ inline size_t tree_lds_bytes(const gsr_model& m, int G) {
   return sizeof(float) * (size_t)(tree_table_words(m.n_links, m.n_dofs, m.mass_blk_size) + kWave / G * tree_env_words(m));
 }
-// Models this path serves: one with an articulated entity (free bodies and fixed links alone, at most 6 dofs each, are
-// better off with one lane per entity: nothing in them is serial but the entity itself) whose values fit
-// kTreeMaxLds.
+// Models this path serves: one with an entity of more than six dofs whose values fit kTreeMaxLds. Free bodies and fixed links
+// alone are better off with one lane per entity: nothing in them is serial but the entity itself. Arms of up to six joints
+// are told apart from those by nothing here and take a lane too, which walks their chain through global memory (one arm of
+// six joints, 1 to 2,048 envs: step_1 72 to 79 us, step_2 64 to 68).
 __host__ __device__ inline bool tree_dynamics(const gsr_model& m) {
   return m.max_entity_dofs > 6 && tree_lds_bytes(m, kWave) <= kTreeMaxLds;
 }
 // Lanes per env of a launch over n envs: 16 once there are more envs than SIMDs (1,024), unless four envs take more LDS
-// than kTreeMaxLds.
+// than kTreeMaxLds. Measured around the line (us, 64 lanes, 16 lanes): quadrupeds step_1 1,024: 38, 45; 2,048: 42, 48; 3,072:
+// 72, 48; step_2 1,024: 34, 28; 2,048: 32, 31; 3,072: 38, 30; arms step_1 1,024: 24, 27; 2,048: 26, 26; 3,072: 43, 28; step_2
+// 1,024: 48, 36; 2,048: 44, 40; 3,072: 52, 41.
 __host__ __device__ inline int tree_lanes(const gsr_model& m, int n) {
   return n > 1024 && tree_lds_bytes(m, 16) <= kTreeMaxLds ? 16 : kWave;
 }

@@ -1,4 +1,5 @@
-// Newton solver of models made of free bodies (every dof belongs to a body of six), kWaves wavefronts per env.
+// Newton solver of models whose entities have six dofs or none, kWaves wavefronts per env: free bodies, and arms of six
+// joints, which are "bodies" below as well.
 //
 // Same algorithm as the other solvers (func_init_solver / func_solve / func_linesearch / rank-1 Cholesky updates of
 // constraint_solver_decomp.py). A heap couples its bodies through contacts, so the Hessian is a sparse matrix of 6 x 6
@@ -9,7 +10,7 @@
 //     short steps, run on the first without barriers;
 //   * dof d belongs to body d / 6 and a row holds its bodies' six entries side by side, so no index is looked up: J^T f
 //     and J^T D J read a row's entries at (row, first or second half + d mod 6); rows that hold fewer entries
-//     (frictionloss, JOINT equalities) are first filled up with zeros;
+//     (frictionloss, JOINT equalities, a part of an arm's chain) are first filled up with zeros;
 //   * forces, weights, Jaref and the line search's terms of the first kBodyRows rows a thread stay in registers; the
 //     forces (then the active rows' weights) lie in LDS for the lanes that walk a body's rows;
 //   * blocks lie whole in LDS, so a row is read with three wide loads and a block with nine; a rank-1 update keeps a
@@ -136,7 +137,7 @@ __device__ __forceinline__ void bodies_sum(const BodyCtx<kWaves>& w, int items, 
 
 // ---- rows -----------------------------------------------------------------------------------------------------------
 // Bodies of row c (the second << 8). A row that does not store all six entries of its bodies (frictionloss, JOINT
-// equalities) is rewritten with zeros in the places that lack, so that every row holds body a's entries first and, if it
+// equalities, a part of an arm's chain) is rewritten with zeros in the places that lack, so that every row holds body a's entries first and, if it
 // has two bodies, b's after them. A row without an entry (an equality between two fixed links) is counted to body 0, with
 // six zeros.
 __device__ inline int body_row(const Env& e, int c) {
