@@ -223,8 +223,5 @@ __device__ __forceinline__ void imp_aref(const float* p, size_t st, float neg_pe
   imp = r.imp;
   aref = impedance_aref(r, vel, pos);
 }
-__device__ __forceinline__ void imp_aref(const float* p, float neg_pen, float vel, float pos, float& imp, float& aref) {
-  imp_aref(p, 1, neg_pen, vel, pos, imp, aref);
-}
 
 }  // namespace gsr

@@ -97,9 +97,6 @@ __device__ __forceinline__ T wave_reduce(T v, Op op) {
   v = op(v, dpp<kDppXor2>(v));
   return op(v, dpp<kDppXor1>(v));
 }
-__device__ __forceinline__ float wave_sum(float v) {
-  return wave_reduce(v, [](float a, float b) { return a + b; });
-}
 // Sums over rows or dofs whose rounding steers discrete decisions (the line search's bracketing, the Newton stop
 // test) are accumulated in double: the reference adds them one by one in FP32, an order a wavefront cannot follow,
 // and a tree of FP32 partial sums has a different rounding error; the double sum is closer to both.
