@@ -10,8 +10,45 @@ from tests.test_gpu_bodies import stacks
 
 pytestmark = pytest.mark.gpu
 
-COMPARED = ["qpos", "vel", "n_con", "n_contacts", "n_broad", "broad_pairs", "contact_geoms", "contact_pos", "contact_normal",
-            "contact_pen", "cache_normal", "sort_value", "sort_ig", "aabb_min", "aabb_max", "errno_env"]
+# fields compared whole; the first `count` entries of lists (entries beyond are left over from earlier steps), by their width
+WHOLE = ["qpos", "vel", "n_con", "n_contacts", "n_broad", "cache_normal", "sort_value", "sort_ig", "first_time", "aabb_min",
+         "aabb_max", "errno_env"]
+LISTS = {"broad_pairs": ("n_broad", 1), "contact_geoms": ("n_contacts", 2), "contact_pos": ("n_contacts", 3),
+         "contact_normal": ("n_contacts", 3), "contact_pen": ("n_contacts", 1), "contact_friction": ("n_contacts", 1)}
+ROWS = ["jac_nnz", "efc_diag", "efc_aref", "efc_D"]
+
+
+def collided(S, n=None, first=0):
+    """What the collision stage of n envs of S wrote (solver variant 1: rows env-major), blank beyond each env's counts."""
+    t, M, dev = S.st.t, S.model, S.device
+    envs = slice(first, first + (S._B if n is None else n))
+    out = {k: t[k][:, envs].clone() for k in WHOLE}
+    for k, (count, width) in LISTS.items():
+        x = t[k][:, envs]
+        keep = torch.arange(len(x), device=dev)[:, None] < width * t[count][0, envs].long()[None]
+        out[k] = torch.where(keep, x, torch.zeros_like(x))
+    R, W = M.max_rows, M.row_width
+    con = t["n_con"][:, envs].long()
+    row = torch.arange(R, device=dev)[None]
+    live = row < con[0][:, None]
+    for k in ROWS:
+        x = t[k].reshape(S._B, R)[envs]
+        out[k] = torch.where(live, x, torch.zeros_like(x))
+    fl = (row >= con[1][:, None]) & (row < (con[1] + con[2])[:, None])
+    x = t["efc_fl"].reshape(S._B, R)[envs]
+    out["efc_fl"] = torch.where(fl, x, torch.zeros_like(x))
+    entry = torch.arange(W, device=dev)[None, None] < out["jac_nnz"].long()[:, :, None]
+    for k in ("jac_val", "jac_idx"):
+        x = t[k].reshape(S._B, R, W)[envs]
+        out[k] = torch.where(entry, x, torch.zeros_like(x))
+    return out
+
+
+def assert_same(a, b, what):
+    for k in a:
+        assert torch.equal(a[k], b[k]), f"{what}: {k}"
+
+
 B = 2051  # 513 wavefronts of four envs, the last one partly filled
 
 
@@ -46,18 +83,11 @@ def test_collision_lanes_agree(name, pairs):
         fb.step()
         torch.cuda.synchronize()
         seen = max(seen, int(few.st.t["n_contacts"][0].max()))
-        for k in COMPARED:
-            a, b, c = (S.st.t[k] for S in (many, few, lane))
-            if k in ("broad_pairs", "contact_geoms", "contact_pos", "contact_normal", "contact_pen"):
-                # entries beyond an env's count are left over from earlier steps
-                n = few.st.t["n_broad" if k == "broad_pairs" else "n_contacts"][0].long()
-                per = {"broad_pairs": 1, "contact_geoms": 2, "contact_pos": 3, "contact_normal": 3, "contact_pen": 1}[k]
-                keep = torch.arange(b.shape[0], device=b.device)[:, None] < per * n[None]
-                a, b, c = (torch.where(keep, x[:, :41], torch.zeros_like(x[:, :41])) for x in (a, b, c))
-            assert torch.equal(b, c), f"{k}: 64 lanes and one lane differ"
-            assert torch.equal(a[..., :41], b), f"{k}: 16 and 64 lanes differ"
-            if a.shape[-1] == B:
-                assert torch.equal(a[..., 41:82], a[..., :41]) and torch.equal(a[..., -1], a[..., (B - 1) % 41]), k
+        a, b = collided(many, 41), collided(few)
+        assert_same(b, collided(lane), "64 lanes and one lane")
+        assert_same(a, b, "16 and 64 lanes")
+        assert_same(collided(many, 41, 41), a, "two runs of 41 envs")
+        assert_same(collided(many, 1, B - 1), collided(many, 1, (B - 1) % 41), "the last env")
     assert seen > 0
     assert bool((few.st.t["errno_env"] & 1).any()) == (pairs == 1)
 
@@ -79,14 +109,7 @@ def test_many_pairs_agree(deep):
     wave.substep()
     fb.step()
     torch.cuda.synchronize()
-    for k in COMPARED:
-        a, b = wave.st.t[k], lane.st.t[k]
-        if k in ("broad_pairs", "contact_geoms", "contact_pos", "contact_normal", "contact_pen"):
-            n = wave.st.t["n_broad" if k == "broad_pairs" else "n_contacts"][0].long()
-            per = {"broad_pairs": 1, "contact_geoms": 2, "contact_pos": 3, "contact_normal": 3, "contact_pen": 1}[k]
-            keep = torch.arange(b.shape[0], device=b.device)[:, None] < per * n[None]
-            a, b = (torch.where(keep, x, torch.zeros_like(x)) for x in (a, b))
-        assert torch.equal(a, b), k
+    assert_same(collided(wave), collided(lane), "64 lanes and one lane")
     pairs = wave.st.t["broad_pairs"][:int(wave.st.t["n_broad"][0, 0]), 0]
     assert int(((pairs >> 16) > 0).sum()) > 64  # geom 0 is the plane
     # without a cached normal the first step of either heap leaves some pairs to GJK/EPA
@@ -115,12 +138,35 @@ def test_lane_per_env_over_very_many_envs(n, B):
         fb.step()
     torch.cuda.synchronize()
     assert int(many.st.t["n_contacts"].min()) >= 4
-    for k in COMPARED:
-        a, b, c = (S.st.t[k] for S in (lane, many, phased))
-        if k in ("broad_pairs", "contact_geoms", "contact_pos", "contact_normal", "contact_pen"):
-            cnt = many.st.t["n_broad" if k == "broad_pairs" else "n_contacts"][0].long()
-            per = {"broad_pairs": 1, "contact_geoms": 2, "contact_pos": 3, "contact_normal": 3, "contact_pen": 1}[k]
-            keep = torch.arange(b.shape[0], device=b.device)[:, None] < per * cnt[None]
-            a, b, c = (torch.where(keep, x, torch.zeros_like(x)) for x in (a, b, c))
-        assert torch.equal(a, b), f"{k}: one and 16 lanes differ"
-        assert torch.equal(c, b), f"{k}: phased and plain differ"
+    b = collided(many)
+    assert_same(collided(lane), b, "one and 16 lanes")
+    assert_same(collided(phased), b, "phased and plain")
+
+
+@pytest.mark.parametrize("G,variant,kernel", [(1022, 0, "k_collide_wave<64>"), (1024, 1, "k_collide_wave<64>"),
+                                              (1023, 0, "k_collide")])
+def test_about_a_thousand_geoms(G, variant, kernel):
+    """The largest models of the wavefront collision (64 KB of LDS, a little more where variant 1 asks for it) and the first
+    beyond: two boxes on a bed of spheres, against a lane per env in the single fused kernel; the phased launch too."""
+    from genesis_amd.batch import FusedBatch, Group
+    from genesis_amd.model import GEOM_SPHERE, JOINT_FIXED, EntitySpec, GeomSpec, JointSpec, LinkSpec
+    from genesis_amd.rigid_solver import RigidSolver
+    one = np.array([1.0, 0, 0, 0])
+    bed = [GeomSpec(GEOM_SPHERE, pos=np.array([0.1 * (i % 32), 0.1 * (i // 32), 0.05]), data=(0.05,)) for i in range(G - 3)]
+    ents = [W.plane_entity(), EntitySpec([LinkSpec("bed", -1, np.zeros(3), one, [JointSpec("fix", JOINT_FIXED)], bed)], name="bed"),
+            W.box_entity((0.25, 0.25, 0.1), (0.55, 0.55, 0.1495)), W.box_entity((0.2, 0.2, 0.2), (2.32, 1.37, 0.1995))]
+    M = compile_model(ents, CompileOptions(dt=0.005, max_collision_pairs=40))
+    assert M.n_geoms == G
+    B = 3
+    plain, lane, phased = (RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=v, dyn_variant=1) for v in (variant, 0, variant))
+    assert plain.kernel_name(1) == kernel
+    fb = FusedBatch([Group(lane, envs_per_tile=2)])
+    fp = FusedBatch([Group(phased, envs_per_tile=2)], phased=True)
+    for _ in range(3):
+        plain.substep()
+        fb.step()
+        fp.step()
+    torch.cuda.synchronize()
+    assert int(plain.st.t["n_contacts"].min()) >= 8  # four spheres under each box
+    assert_same(collided(plain), collided(lane), "plain and one lane")
+    assert_same(collided(phased), collided(lane), "phased and one lane")

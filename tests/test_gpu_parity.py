@@ -264,10 +264,13 @@ def test_step_parity_resynced(case, B, steps, variant, pre):
 @pytest.mark.parametrize("case", ["arm", "quadruped", "pile8", "pile64"])
 def test_wave_collide_equals_lane_collide(case):
     """The wavefront collision kernel (pairs across lanes, prefix-sum placement) writes bitwise what the one-lane-per-env
-    kernel writes: sort buffers, broadphase pairs in order, contacts in order, normal cache and constraint rows, over
-    two consecutive steps (so the warm-started sort and the cached normals are exercised too)."""
+    form writes (the single fused kernel's variant 0, 32 lanes of one tile): sort buffers, broadphase pairs in order,
+    contacts in order, normal cache and constraint rows, over two consecutive steps (so the warm-started sort and the
+    cached normals are exercised too)."""
     _need_gpu()
+    from genesis_amd.batch import FusedBatch, Group
     from genesis_amd.rigid_solver import RigidSolver
+    from tests.test_gpu_collide_lanes import assert_same, collided
     ents, opt = CASES[case]()
     M = compile_model(ents, opt)
     B = 32
@@ -275,24 +278,17 @@ def test_wave_collide_equals_lane_collide(case):
     q = torch.as_tensor(_random_qpos(M, B, rng, base_z=(0.05, 0.35)), dtype=torch.float32)
     lane = RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=0)
     wave = RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=1)
+    assert wave.kernel_name(1) == "k_collide_wave<64>"
     for S in (lane, wave):
         S.set_qpos(q)
-    fields = ["sort_value", "sort_ig", "first_time", "n_broad", "broad_pairs", "n_contacts", "contact_geoms",
-              "contact_pos", "contact_normal", "contact_pen", "contact_friction", "cache_normal", "n_con", "jac_val",
-              "jac_idx", "jac_nnz", "efc_diag", "efc_aref", "efc_D", "efc_fl", "aabb_min", "aabb_max", "errno_env"]
+    fb = FusedBatch([Group(lane, envs_per_tile=32, solver_variant=1, collide_variant=0)])
     for step in range(2):
-        for S in (lane, wave):
-            S.launch_kernel(0)
-            S.launch_kernel(1)
+        fb.step()
+        wave.substep()
         torch.cuda.synchronize()
-        for f in fields:
-            a, b = lane.st.t[f], wave.st.t[f]
-            assert torch.equal(a, b), f"{case} step {step}: {f} differs"
+        assert_same(collided(lane), collided(wave), f"{case} step {step}")
         if case != "arm":
             assert int(wave.st.t["n_contacts"].sum()) > 0
-        for S in (lane, wave):
-            S.launch_kernel(2)
-            S.launch_kernel(3)
 
 
 @pytest.mark.parametrize("case,B,steps", [("arm", 8, 1000), ("quadruped", 8, 1000), ("pile20", 8, 500)])
@@ -346,8 +342,10 @@ def test_mesh_arm_contacts_match_oracle(collide_variant):
     """The Panda arm's collision meshes (convex hulls, support-field lookups in MPR and GJK/EPA) against the plane:
     random joint angles within the limits put links into the floor; from the same state the HIP collision stage
     gives the oracle's contacts in the same order, positions, normals and depths within 1e-4, over resynced steps
-    of the full step (variant 1 solver, both collision variants)."""
+    of the full step (variant 1 solver). Variant 0 is the single fused kernel with a lane per env, whose whole step leaves
+    the contacts too."""
     _need_gpu()
+    from genesis_amd.batch import FusedBatch, Group
     from genesis_amd.model import GEOM_MESH
     from genesis_amd.rigid_solver import RigidSolver
     ents, opt = CASES["arm"]()
@@ -358,13 +356,18 @@ def test_mesh_arm_contacts_match_oracle(collide_variant):
     S = RigidSolver(M, B, "cuda", solver_variant=1, collide_variant=collide_variant)
     S.set_qpos(torch.as_tensor(_random_qpos(M, B, rng), dtype=torch.float32))
     O = _oracle(M, B)
+    fb = FusedBatch([Group(S, envs_per_tile=32, solver_variant=1, collide_variant=0)]) if collide_variant == 0 else None
+    step_once = fb.step if fb else S.substep
     n_mesh = 0
     worst = 0.0
     for step in range(8):
         torch.cuda.synchronize()
         keep = {k: v.clone() for k, v in S.st.t.items()}
         gpu_to_oracle(S, O)
-        S.run_stage(3)
+        if fb:
+            fb.step()
+        else:
+            S.run_stage(3)
         O.run(stage=3)
         torch.cuda.synchronize()
         t = S.st.t
@@ -386,7 +389,7 @@ def test_mesh_arm_contacts_match_oracle(collide_variant):
         for k, v in keep.items():
             t[k].copy_(v)
         gpu_to_oracle(S, O)
-        S.substep()
+        step_once()
         O.run(1)
         torch.cuda.synchronize()
         for name in ("qpos", "vel"):
