@@ -60,8 +60,10 @@ WAVE_MAX_ENTITIES = 128
 
 
 # Up to this many envs, one wavefront per env still fills the chip (8 waves per CU at 2,048 envs) and cuts the
-# per-env latency that a few envs' step is made of; beyond it, the dynamics and collision stages of a small
-# articulation run one lane per env.
+# per-env latency that a few envs' step is made of; beyond it, variant 0 is the default of small models' collision and of
+# free bodies' dynamics. In the single fused kernel that is a lane per env; the plain and phased collision take 64 or 16
+# lanes per env by size with either variant, and with 0 a lane per env over very many envs (collide_by_lane in
+# rigid_collide_wave.h), and the plain dynamics of free bodies take (env, entity) lanes with either.
 WAVE_MAX_SMALL_ENVS = 2048
 
 
@@ -72,8 +74,8 @@ def default_solver_variant(M: RigidModel, n_envs: int = None) -> int:
 
 
 def default_stage_variant(M: RigidModel, n_envs: int = None) -> int:
-    """Variant of the dynamics and collision stages: 1 = one wavefront per env (large systems, or few envs), 0 = one
-    lane per env (many envs of a small articulation)."""
+    """Variant of the free bodies' dynamics and of the collision: 1 = one wavefront per env (large systems, or few envs), 0 =
+    one lane per env where the launch has that form (many envs of a small model)."""
     return 1 if (M.n_dofs >= 48 or (n_envs is not None and n_envs <= WAVE_MAX_SMALL_ENVS)) else 0
 
 
@@ -86,8 +88,8 @@ def default_dyn_variant(M: RigidModel, n_envs: int = None) -> int:
 
 
 def default_collide_variant(M: RigidModel, n_envs: int = None) -> int:
-    """As default_stage_variant, except that mesh geoms take the wavefront collision (support-field lookups diverge
-    across a lane-per-env wavefront: the Panda's meshes collide 10x slower one lane per env at 5,492 envs)."""
+    """As default_stage_variant, except that mesh geoms always take wavefronts (support-field lookups diverge across a
+    lane-per-env wavefront: the Panda's meshes collide 10x slower one lane per env at 5,492 envs)."""
     from .model import GEOM_MESH
     return 1 if (np.asarray(M.geom_type) == GEOM_MESH).any() else default_stage_variant(M, n_envs)
 

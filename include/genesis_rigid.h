@@ -57,7 +57,9 @@ typedef struct gsr_model {
   int32_t collide_variant; /* the single fused kernel's collision: 0 one lane per env, 1 one wavefront per env (pairs
                               across lanes). The plain and phased steps take 64 or 16 lanes per env by size with either;
                               with 0 a lane per env over very many envs of a small model and above 1,022 geoms */
-  int32_t dyn_variant;     /* step_1 / step_2: 0 one lane per env, 1 one wavefront per env (entities across lanes) */
+  int32_t dyn_variant;     /* step_1 / step_2: 1 spreads an articulated env's tree over 64 or 16 lanes (in the fused and phased
+                              launches also a free-body env's entities over a wavefront), 0 a lane per env there; an
+                              entity per lane in the plain step where the tree is not spread */
   int32_t batch_dofs;      /* 1: dof_kp, dof_kv, dof_force_range, dof_stiffness, dof_damping, dof_frictionloss,
                               dof_limit, dof_armature and dof_invweight hold one value per env, env-minor like the state
                               (component c of dof d of env b at [(d * k + c) * n_envs + b]); 0: one value per dof
