@@ -366,9 +366,7 @@ class RigidSolver:
 
     def kernel_name(self, k: int) -> str:
         """Device kernel that launch_kernel(k) runs for this model's variant switches and env count."""
-        if not 0 <= k <= 3:
-            raise IndexError(f"kernel {k} of 0..3")
-        return self._lib.gsr_kernel_name(self.dm.desc, self._B, k).decode()
+        return self._lib.gsr_kernel_name(self.dm.desc, self._B, range(4)[k]).decode()
 
     def run_stage(self, stage: int):
         _lib.check(self._lib.gsr_run_stage(self.dm.desc, self.st.desc, stage, self._stream()), "gsr_run_stage")
